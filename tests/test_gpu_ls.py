@@ -502,6 +502,46 @@ def test_frozen_bermudan_with_displaced_rates_vs_fp64_oracle(torch_cuda):
     _check_frozen(torch, w, pr, z, price.item(), greeks, "displaced")
 
 
+@pytest.mark.parametrize("P,N,F,k", [(70, 2, 2, 1), (500, 3, 5, 2), (300, 4, 6, 1), (777, 5, 3, 2),
+                                     (300, 9, 8, 4), (400, 45, 2, 8), (400, 46, 4, 8),
+                                     (130, 60, 7, 1)])
+def test_bermudan_windows_and_blocks_vs_fp64_oracle(torch_cuda, P, N, F, k):
+    """Path quantities and the frozen-strategy adjoint on curves about and below
+    the step loops' window of rates, both block sizes, path counts that leave
+    lanes idle.  The strategy exercises on a constant continuation value, so
+    that no regression is involved; tolerances as the tests above."""
+    torch = torch_cuda
+    rng = np.random.RandomState(100 * N + F)
+    f0 = 0.05 + 0.005 * rng.uniform(size=N)
+    vols = np.full(N, 0.2)
+    A = 0.2 * np.sqrt(0.5 / F) * rng.uniform(0.6, 1.0, size=(N, N, F))
+    f0, A = (x.astype(np.float32).astype(np.float64) for x in (f0, A))
+    ex = np.unique(np.linspace(0, N - 1, min(N, 9)).astype(np.int32))
+    w = configs.LMMWorkload("windows", P, N, F, 0.5, f0, vols, 0.5 * np.arange(1, N + 2), A, 0.045,
+                            "bermudan", np.zeros(N * F, np.uint32), exercise_steps=ex,
+                            basis_shift=np.full((ex.size, 2), 0.05),
+                            basis_scale=np.full((ex.size, 2), 100.0))
+    pr = pipeline.BermudanPricer(w)
+    z = rng.normal(size=(N, F, P)).astype(np.float32)
+    pr.z.copy_(torch.from_numpy(z.reshape(-1)))
+    pr.paths_kernel()
+    E = pr.E
+    m, z = _oracle_model(w), z.astype(np.float64)
+    bvo, evo, numo = O.bermudan_paths(m, z, ex)
+    bv, ev, num = (t.cpu().numpy() for t in (pr.bv, pr.ev, pr.num))
+    assert np.allclose(bv.reshape(E, 2, P), bvo, rtol=2e-5)
+    assert np.max(np.abs(ev.reshape(E, P) - evo)) < 1e-5 * np.max(evo)
+    # a product of up to N factors 1 + tau f: each adds a rounding and at most a
+    # fifth (tau f / (1 + tau f), rates to 50%) of its rate's relative error,
+    # which is below two roundings for each of the steps it has moved
+    assert np.allclose(num.reshape(E, P), numo, rtol=N * (1 + 0.2 * 2 * N) * 2.0 ** -24, atol=0)
+    pr.coeffs.zero_()
+    pr.coeffs.view(E, 6)[:, 0] = 0.6 * float(np.median(evo[evo > 0]))
+    price, greeks = pr.greeks(checkpoint_every=k)
+    torch.cuda.synchronize()
+    _check_frozen(torch, w, pr, z, price.item(), greeks, f"P={P} N={N} F={F} k={k}")
+
+
 # ---------------------------------------------------------------- batched portfolio
 
 def test_batched_portfolio_equals_per_product_calls(torch_cuda):

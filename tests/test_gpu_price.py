@@ -205,3 +205,44 @@ def test_repeat_calls_are_deterministic(torch_cuda):
     p2, g2 = pr.price_and_greeks()
     assert a == p1 == p2.item()
     assert torch_cuda.equal(g1, g2)
+
+
+@pytest.mark.parametrize("P,N,F,k", [
+    (70, 1, 1, 1), (65, 2, 8, 1), (130, 3, 2, 2), (64, 4, 8, 2), (257, 5, 6, 3), (1000, 7, 7, 1),
+    (300, 8, 5, 8), (65600, 9, 2, 4), (66000, 13, 3, 1), (65537, 45, 1, 8), (300, 46, 5, 8),
+    (200, 90, 3, 30), (100, 90, 8, 1)])
+def test_windows_blocks_and_intervals_vs_fp64_adjoint(torch_cuda, P, N, F, k):
+    """Curves about and below the step loops' window of rates, every factor
+    class, both block sizes (few paths and long curves run single-wavefront
+    blocks), path counts that leave lanes idle, checkpoint intervals from
+    every step to none.  Strikes far in the money, so no path of FP32 rounding
+    falls on the other side: what is left is the rounding of the states,
+    below 4 units of 2^-24 a step on every path, so at most 90 x 4 x 6e-8 =
+    2e-5 of the largest Greek (and of the price)."""
+    rng = np.random.RandomState(100 * N + F)
+    f0 = 0.04 + 0.01 * rng.uniform(size=N)
+    taus = np.full(N, 0.5)
+    vols = rng.uniform(0.1, 0.2, N)
+    A = (vols[None, :, None] * np.sqrt(0.5 / F) * rng.uniform(0.5, 1.0, size=(N, N, F)))
+    f0, vols, A = (x.astype(np.float32).astype(np.float64) for x in (f0, vols, A))
+    w = configs.LMMWorkload("windows", P, N, F, 0.5, f0, vols, 0.5 * np.arange(1, N + 2), A, 0.0,
+                            "caplets", np.zeros(N * F, np.uint32), checkpoint_every=k,
+                            displacements=np.full(N, 0.0078125))
+    pr = pipeline.LMMPricer(w)
+    z = rng.normal(size=(N, F, P)).astype(np.float32)
+    pr.z.copy_(torch_cuda.from_numpy(z.reshape(-1)))
+    pp, d, v = O.caplet_adjoint_paths(
+        O.caplet_model(f0, taus, w.disp(), A, vols, w.strike, P), z.astype(np.float64))
+    pr.price_kernel(checkpoints=False)
+    alone = pr.price_out.item()
+    pr.price_kernel(checkpoints=True)
+    pr.greeks_kernel()
+    g = pr.greeks_out.cpu().numpy()
+    g64 = np.concatenate([d, v]) / P
+    print(f"P={P} N={N} F={F} k={k}: price rel {alone / pp.mean() - 1:.2e}, deltas "
+          f"{np.max(np.abs(g - g64)[:N]) / np.max(np.abs(d / P)):.2e}, vegas "
+          f"{np.max(np.abs(g - g64)[N:]) / np.max(np.abs(v / P)):.2e}", flush=True)
+    assert alone == pr.price_out.item()
+    assert abs(alone / pp.mean() - 1) < 2e-5
+    assert np.all(np.abs(g - g64)[:N] <= 2e-5 * np.max(np.abs(d / P)))
+    assert np.all(np.abs(g - g64)[N:] <= 2e-5 * np.max(np.abs(v / P)))

@@ -25,23 +25,32 @@ namespace {
 
 using namespace lmm;
 
-template <int F>
-__global__ void __launch_bounds__(256)
+template <int F, int BD, int U>
+__global__ void __launch_bounds__(BD)
     k_berm_fwd(KOO_MODEL_PARAMS, const BermArgs b, const double* __restrict__ coeffs,
                float* __restrict__ ckpt, float* __restrict__ lamt, int* __restrict__ tau_out,
                float* __restrict__ vout, double* __restrict__ part) {
   KOO_MODEL_LOCAL;
-  berm_fwd_block<F>(m, b, CoefGlobal{coeffs}, ckpt, lamt, tau_out, vout, part, blockIdx.x);
+  berm_fwd_block<F, BD, U>(m, b, CoefGlobal{coeffs}, ckpt, lamt, tau_out, vout, part, blockIdx.x);
 }
 
-template <int F>
-__global__ void __launch_bounds__(256)
+template <int F, int BD, int U>
+__global__ void __launch_bounds__(BD)
     k_berm_bwd(KOO_MODEL_PARAMS, const float* __restrict__ vols, const float* __restrict__ ckpt,
                const float* __restrict__ lamt, const int* __restrict__ tau_in,
                const float* __restrict__ vin, float* __restrict__ scratch,
                double* __restrict__ part) {
   KOO_MODEL_LOCAL;
-  berm_bwd_block<F>(m, vols, ckpt, lamt, tau_in, vin, scratch, part, blockIdx.x);
+  berm_bwd_block<F, BD, U>(m, vols, ckpt, lamt, tau_in, vin, scratch, part, blockIdx.x);
+}
+
+// The step table (lmm_step.h) behind the checkpoints, which the forward and
+// the backward read with scalar loads.  One lane per entry of the square.
+template <int F>
+__global__ void __launch_bounds__(256) k_berm_step_table(KOO_MODEL_PARAMS, float* __restrict__ ckpt) {
+  KOO_MODEL_LOCAL;
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < m.N * m.N) put_step_entry<F>(m, q, ckpt + berm_ckpt_floats<F>(m));
 }
 
 // ---------------------------------------------------------------------------
@@ -75,6 +84,22 @@ __device__ __forceinline__ Model item_model(const BermItem& it) {
                it.P, it.N, it.k};
 }
 
+// Every product's step table; grid (blocks of 256 entries, products).
+__global__ void __launch_bounds__(256) k_berm_step_table_batch(const BermItem* __restrict__ items) {
+  const BermItem& it = items[blockIdx.y];
+  const Model m = item_model(it);
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= it.N * it.N) return;
+  switch (it.F) {
+#define KOO_CASE(F)                                                      \
+  case F:                                                                \
+    put_step_entry<F>(m, q, gmem(it.ckpt) + berm_ckpt_floats<F>(m));     \
+    break;
+    KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
+#undef KOO_CASE
+  }
+}
+
 __global__ void __launch_bounds__(256)
     k_berm_fwd_batch(const BermItem* __restrict__ items, int n, int block_offset) {
   const int block = blockIdx.x + block_offset;
@@ -84,8 +109,14 @@ __global__ void __launch_bounds__(256)
   switch (it.F) {
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
-    berm_fwd_block<F>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.ckpt), gmem(it.lamt),       \
-                      gmem(it.tau), gmem(it.vout), gmem(it.part_fwd), blk);                    \
+    if (it.N >= kShortCurve)                                                                   \
+      berm_fwd_block<F, 256, kWindow<F>>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.ckpt),  \
+                                         gmem(it.lamt), gmem(it.tau), gmem(it.vout),           \
+                                         gmem(it.part_fwd), blk);                              \
+    else                                                                                       \
+      berm_fwd_block<F, 256, 1>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.ckpt),           \
+                                gmem(it.lamt), gmem(it.tau), gmem(it.vout), gmem(it.part_fwd), \
+                                blk);                                                          \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
 #undef KOO_CASE
@@ -101,8 +132,13 @@ __global__ void __launch_bounds__(256)
   switch (it.F) {
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
-    berm_bwd_block<F>(m, gmem(it.vols), gmem(it.ckpt), gmem(it.lamt), gmem(it.tau),            \
-                      gmem(it.vout), gmem(it.scratch), gmem(it.part_bwd), blk);               \
+    if (it.N >= kShortCurve)                                                                   \
+      berm_bwd_block<F, 256, kWindow<F>>(m, gmem(it.vols), gmem(it.ckpt), gmem(it.lamt),       \
+                                         gmem(it.tau), gmem(it.vout), gmem(it.scratch),        \
+                                         gmem(it.part_bwd), blk);                              \
+    else                                                                                       \
+      berm_bwd_block<F, 256, 1>(m, gmem(it.vols), gmem(it.ckpt), gmem(it.lamt), gmem(it.tau),  \
+                                gmem(it.vout), gmem(it.scratch), gmem(it.part_bwd), blk);      \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
 #undef KOO_CASE
@@ -145,10 +181,8 @@ extern "C" int bermudan_adjoint_workspace(int paths, int rates, int factors, int
                                   (rates + 1 + 2 * factors) * P;
   // payoff adjoints (rates x P floats), exercise step (P ints), value (P floats)
   if (path_bytes) *path_bytes = sizeof(float) * (static_cast<size_t>(rates) + 2) * P;
-  const size_t bf = (P + fwd_threads(rates) - 1) / fwd_threads(rates);
-  const size_t bb = (P + bwd_threads(rates) - 1) / bwd_threads(rates);
-  const size_t need = bf > bb * 2 * rates ? bf : bb * 2 * rates;
-  if (partial_bytes) *partial_bytes = sizeof(double) * need;
+  const int t = block_lanes(rates);
+  if (partial_bytes) *partial_bytes = sizeof(double) * ((P + t - 1) / t) * 2 * rates;
   return KOO_OK;
 }
 
@@ -172,21 +206,31 @@ extern "C" int bermudan_frozen_fwd(int paths, int rates, int factors, int checkp
   float* lamt = path_buffers;
   int* tau = reinterpret_cast<int*>(path_buffers + static_cast<size_t>(rates) * P);
   float* vout = path_buffers + static_cast<size_t>(rates + 1) * P;
-  const int threads = fwd_threads(rates);
+  const int threads = block_lanes(rates);
   const int blocks = (paths + threads - 1) / threads;
-  const size_t lds = fwd_lds(rates, threads);
+  const size_t lds = rows_lds(rates, threads, false);
   hipStream_t st = as_stream(stream);
   switch (factors) {
+#define KOO_FWD(F, BD, U)                                                                      \
+  hipLaunchKernelGGL((k_berm_fwd<F, BD, U>), dim3(blocks), dim3(BD), lds, st, variates,           \
+                     initial_rates, taus, displacements, pseudo_roots, strike, paths, rates,   \
+                     checkpoint_every, b, coefficients, checkpoints, lamt, tau, vout, partials)
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
-    hipLaunchKernelGGL(k_berm_fwd<F>, dim3(blocks), dim3(threads), lds, st, variates,          \
-                       initial_rates, taus, displacements, pseudo_roots, strike, paths, rates, \
-                       checkpoint_every, b, coefficients, checkpoints, lamt, tau, vout,        \
-                       partials);                                                              \
+    hipLaunchKernelGGL(k_berm_step_table<F>, dim3((rates * rates + 255) / 256), dim3(256), 0,  \
+                       st, variates, initial_rates, taus, displacements, pseudo_roots, strike, \
+                       paths, rates, checkpoint_every, checkpoints);                           \
+    if (threads == 64)                                                                         \
+      KOO_FWD(F, 64, kWindow<F>);                                                               \
+    else if (rates >= kShortCurve)                                                             \
+      KOO_FWD(F, 256, kWindow<F>);                                                              \
+    else                                                                                       \
+      KOO_FWD(F, 256, 1);                                                                       \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5) KOO_CASE(6) KOO_CASE(7)
     KOO_CASE(8)
 #undef KOO_CASE
+#undef KOO_FWD
   }
   hipLaunchKernelGGL(k_finalize_cols, dim3(1), dim3(256), 0, st, partials, blocks, 1,
                      1.0 / static_cast<double>(paths), price_out);
@@ -208,21 +252,29 @@ extern "C" int bermudan_frozen_bwd(int paths, int rates, int factors, int checkp
   const float* lamt = path_buffers;
   const int* tau = reinterpret_cast<const int*>(path_buffers + static_cast<size_t>(rates) * P);
   const float* vin = path_buffers + static_cast<size_t>(rates + 1) * P;
-  const int threads = bwd_threads(rates);
+  const int threads = block_lanes(rates);
   const int blocks = (paths + threads - 1) / threads;
-  const size_t lds = bwd_lds(rates, threads, false);
+  const size_t lds = rows_lds(rates, threads, false);
   hipStream_t st = as_stream(stream);
   switch (factors) {
+#define KOO_BWD(F, BD, U)                                                                      \
+  hipLaunchKernelGGL((k_berm_bwd<F, BD, U>), dim3(blocks), dim3(BD), lds, st, variates,           \
+                     initial_rates, taus, displacements, pseudo_roots, strike, paths, rates,   \
+                     checkpoint_every, vols, checkpoints, lamt, tau, vin, segment_scratch,     \
+                     partials)
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
-    hipLaunchKernelGGL(k_berm_bwd<F>, dim3(blocks), dim3(threads), lds, st, variates,          \
-                       initial_rates, taus, displacements, pseudo_roots, strike, paths, rates, \
-                       checkpoint_every, vols, checkpoints, lamt, tau, vin, segment_scratch,   \
-                       partials);                                                              \
+    if (threads == 64)                                                                         \
+      KOO_BWD(F, 64, kWindow<F>);                                                               \
+    else if (rates >= kShortCurve)                                                             \
+      KOO_BWD(F, 256, kWindow<F>);                                                              \
+    else                                                                                       \
+      KOO_BWD(F, 256, 1);                                                                       \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5) KOO_CASE(6) KOO_CASE(7)
     KOO_CASE(8)
 #undef KOO_CASE
+#undef KOO_BWD
   }
   hipLaunchKernelGGL(k_finalize_cols, dim3(2 * rates), dim3(256), 0, st, partials, blocks,
                      2 * rates, 1.0 / static_cast<double>(paths), greeks_out);
@@ -329,16 +381,19 @@ static int portfolio_launch(const char* who, bool fwd, const koo_portfolio_plan*
   const BermItem* items = static_cast<const BermItem*>(descriptors_device);
   const int N = plan->max_rates;
   hipStream_t st = as_stream(stream);
+  if (fwd)
+    hipLaunchKernelGGL(k_berm_step_table_batch, dim3((N * N + 255) / 256, plan->products),
+                       dim3(256), 0, st, items);
   for (int c = 0; c < plan->classes; ++c) {
     const int nc = plan->class_max_rates[c], b0 = plan->class_first_block[c];
     const int nb = plan->class_blocks[c];
     if (nc < 1 || nc > N || nb < 1 || b0 < 0 || b0 + nb > plan->blocks)
       return set_error(KOO_ERR_INVALID, "%s: bad plan class %d", who, c);
     if (fwd)
-      hipLaunchKernelGGL(k_berm_fwd_batch, dim3(nb), dim3(256), fwd_lds(nc, 256), st, items,
+      hipLaunchKernelGGL(k_berm_fwd_batch, dim3(nb), dim3(256), rows_lds(nc, 256, false), st, items,
                          plan->products, b0);
     else
-      hipLaunchKernelGGL(k_berm_bwd_batch, dim3(nb), dim3(256), bwd_lds(nc, 256, false), st, items,
+      hipLaunchKernelGGL(k_berm_bwd_batch, dim3(nb), dim3(256), rows_lds(nc, 256, false), st, items,
                          plan->products, b0);
   }
   hipLaunchKernelGGL(k_berm_finalize_batch, dim3(fwd ? 1 : 2 * N, plan->products), dim3(256), 0,

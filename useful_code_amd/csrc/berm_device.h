@@ -12,8 +12,6 @@ namespace {
 using namespace lmm;
 
 constexpr int kMaxBermDates = 40;
-constexpr int kStatePrefetch = 8;
-
 struct BermArgs {
   int E, itm_only, last;
   signed char e_of_step[kMaxRates];  // exercise index of each step, -1 if none
@@ -45,68 +43,77 @@ struct CoefTable {
   __device__ float operator()(int ei, int j) const { return t[6 * ei + j]; }
 };
 
-// One block of the forward: paths [block * blockDim, ...) of product m.
-// Agent: the block's price partial stored agent-coherent (persistent kernel).
-template <int F, bool Agent = false, class Coef>
+// One block of the forward: paths [block * BD, ...) of product m.  Ctab: the
+// step table behind the checkpoints (scalar loads), or the block's own copy in
+// LDS behind its states (the persistent kernel, whose backward runs in the
+// same launch).  Agent: the block's price partial stored agent-coherent (the
+// persistent kernel).
+template <int F, int BD, int U, bool Agent = false, class Coef>
 __device__ __forceinline__ void berm_fwd_block(const Model& m, const BermArgs& b, const Coef& cf,
                                                float* __restrict__ ckpt, float* __restrict__ lamt,
                                                int* __restrict__ tau_out,
                                                float* __restrict__ vout,
                                                double* __restrict__ part, int block) {
   extern __shared__ float lds[];
-  __shared__ double red[4];
-  const int bd = blockDim.x;
-  const int p = block * bd + threadIdx.x;
-  const bool valid = p < m.P;
-  const int pc = valid ? p : m.P - 1;
-  float* L = lds + threadIdx.x;
-  float* ctab = lds + static_cast<size_t>(m.N) * bd;
-  const size_t P = static_cast<size_t>(m.P);
-  fill_step_table<F>(m, ctab);
-  for (int r = 0; r < m.N; ++r) L[r * bd] = logf(m.f0[r] + m.disp[r]);
-  __syncthreads();
-  // Block 0 of a single-product or batched forward also copies the step
-  // table behind the checkpoints, where the backward reads it (the
-  // persistent kernel's backward keeps its own LDS copy: it runs in the same
-  // launch as this forward).
-  if (!Agent && ckpt && block == 0) {
-    float* tab = ckpt + berm_ckpt_floats<F>(m);
-    for (int i = threadIdx.x; i < step_table_floats(m.N); i += bd) tab[i] = ctab[i];
-  }
+  const BlockPaths bp(m.P, block, BD);
+  const int N = m.N;
+  const bool valid = static_cast<int>(threadIdx.x) < bp.n;
+  const size_t p = bp.p0 + threadIdx.x;
+  const LaneRows<BD> X{lds + threadIdx.x};
+  float* ltab = lds + static_cast<size_t>(N) * BD;
+  if (Agent) fill_step_table<F>(m, ltab);
+  for (int r = 0; r < N; ++r) X.set(r, 0.0f);
+  if (Agent) __syncthreads();
+  const auto ctab = [&]() {
+    if constexpr (Agent) return static_cast<const float*>(ltab);
+    else return cmem(ckpt + berm_ckpt_floats<F>(m));
+  }();
   float invB = 1.0f, V = 0.0f;
   int tau = -1;
   bool done = !valid;
-  const int rows = m.k == 1 ? m.N + 1 + 2 * F : m.N + 1;
-  for (int s = 0; s <= b.last; ++s) {
-    if (__all(done)) break;  // the wavefront's paths have all exercised
-    const bool save = ckpt && valid && (s % m.k) == 0;
-    float* c = save ? ckpt + static_cast<size_t>(s / m.k) * rows * P + p : nullptr;
-    if (save) {
-      for (int r = s; r < m.N; ++r) c[static_cast<size_t>(r) * P] = L[r * bd];
-      c[static_cast<size_t>(m.N) * P] = invB;
-    }
-    float z[F], e[F], ep[F];
-    load_z<F>(m, s, pc, z);
-    pc_step<F>(m, s, ctab + s * m.N, z, e, ep, [&](int r) { return L[r * bd]; },
-               [&](int r, float v) { L[r * bd] = v; });
-    if (save && m.k == 1) {
+  const int rows = m.k == 1 ? N + 1 + 2 * F : N + 1;
+  auto slot = [&](int s) { return ckpt + static_cast<size_t>(s / m.k) * rows * bp.P; };
+  for (int r = 0; r < N; ++r) bp.row(slot(0), r).store(0.0f);
+  auto load = [&](int r) { return X.get(r); };
+  float zn[F];
+  load_z<F>(m, bp, 0, zn);
+  Ahead<F, U> ahead;
+  pc_fetch<F, U>(ahead, m, 0, ctab, load);
+  // last step: none from when all of the wavefront's paths have exercised (a
+  // scalar in the loop's one exit, so what the loop carries stays uniform)
+  const auto last_step = [&](int last) {
+    return __builtin_amdgcn_readfirstlane(__builtin_amdgcn_ballot_w64(!done) != 0 ? last : -1);
+  };
+  for (int s = 0, last = last_step(b.last); s <= last; ++s, last = last_step(last)) {
+    float z[F], y[F], d[F];
 #pragma unroll
-      for (int f = 0; f < F; ++f) {
-        c[static_cast<size_t>(m.N + 1 + f) * P] = e[f];
-        c[static_cast<size_t>(m.N + 1 + F + f) * P] = ep[f];
-      }
+    for (int f = 0; f < F; ++f) z[f] = zn[f];
+    load_z<F>(m, bp, min(s + 1, N - 1), zn);
+    float xs;
+    if (s + 1 < N && (s + 1) % m.k == 0) {
+      const float* next = slot(s + 1);
+      xs = pc_step<F, U>(m, s, ctab, ahead, z, y, d, load, [&](int r, float x) {
+        X.set(r, x);
+        bp.row(next, r).store(x);
+      });
+    } else {
+      xs = pc_step<F, U>(m, s, ctab, ahead, z, y, d, load, [&](int r, float x) { X.set(r, x); });
     }
-    const float fs = fast_exp(L[s * bd]) - m.disp[s];
+    if (s + 1 < N) pc_fetch<F, U>(ahead, m, s + 1, ctab, load);
+    if (s % m.k == 0) {
+      const float* c = slot(s) + static_cast<size_t>(N) * bp.P;
+      bp.row(c).store(invB);
+      if (m.k == 1) store_sums<F>(bp, c + bp.P, y, d);
+    }
+    const float fs = fmaf(start_level(m, s), fast_exp2(xs), -m.disp[s]);
     const int ei = b.e_of_step[s];
-    if (ei >= 0 && !done) {
+    if (ei >= 0) {  // uniform: done lanes walk along
       float disc = 1.0f, ann = 0.0f, flt = 0.0f;
-      for (int r = s; r < m.N; ++r) {
-        const float fr = fast_exp(L[r * bd]) - m.disp[r];
-        const float tr = m.taus[r];
+      walk_curve<U, false>(m, s, X, [&](int, float, float fr, float tr) {
         disc *= fast_rcp(1.0f + tr * fr);
         ann += tr * disc;
         flt += tr * fr * disc;
-      }
+      });
       const float sr = flt / ann;
       const float ev = (sr - m.strike) * ann;
       const float x0 = (sr - b.sh[ei][0]) * b.sc[ei][0];
@@ -115,21 +122,23 @@ __device__ __forceinline__ void berm_fwd_block(const Model& m, const BermArgs& b
                          cf(ei, 4) * x0 * x1 + cf(ei, 5) * x1 * x1;
       const float evp = ev > 0.0f ? ev : 0.0f;
       const bool allowed = !b.itm_only || evp > 0.0f;
-      if (allowed && cont - evp < 0.0f) {
-        done = true;
-        tau = s;
-        V = evp * invB;
-        // payoff adjoint on the end-of-step log-rates r >= s
+      const bool now = !done && allowed && cont - evp < 0.0f;
+      if (__any(now)) {
+        done = done || now;
+        tau = now ? s : tau;
+        V = now ? evp * invB : V;
+        // payoff adjoint on the end-of-step states r >= s (the other lanes'
+        // stores are out of their buffer's range)
+        const int byte = now ? static_cast<int>(4 * threadIdx.x) : -4;
         float Pr = disc, Q = 0.0f;  // P_{r+1}, sum_{m>r} tau_{m-1} P_m
-        for (int r = m.N - 1; r >= s; --r) {
-          const float x = fast_exp(L[r * bd]);
-          const float fr = x - m.disp[r];
-          const float tr = m.taus[r];
+        walk_curve<U, true>(m, s, X, [&](int r, float x, float fr, float tr) {
           const float g = tr * fast_rcp(1.0f + tr * fr);
           Q += tr * Pr;
-          lamt[static_cast<size_t>(r) * P + p] = ev > 0.0f ? g * (disc + m.strike * Q) * invB * x : 0.0f;
+          PathRow row = bp.row(lamt, r);
+          row.byte = byte;
+          row.store(ev > 0.0f ? g * (disc + m.strike * Q) * invB * x * kLn2 : 0.0f);
           Pr *= 1.0f + tr * fr;
-        }
+        });
       }
     }
     invB *= fast_rcp(1.0f + m.taus[s] * fs);
@@ -138,16 +147,16 @@ __device__ __forceinline__ void berm_fwd_block(const Model& m, const BermArgs& b
     tau_out[p] = tau;
     vout[p] = V;
   }
-  block_sum_to<Agent>(valid ? static_cast<double>(V) : 0.0, red, part + block);
+  // (the states are done with: their rows hold the wavefronts' sums)
+  block_sum_to<Agent>(valid ? static_cast<double>(V) : 0.0, reinterpret_cast<double*>(lds),
+                      part + block);
 }
 
-// One block of the backward (paths [block * blockDim, ...)).  Agent: the
-// block's partials stored agent-coherent (persistent kernel).  LDS: the
-// adjoints of rates 1..N-1 [N-1][lanes] (rate 0's in a register), the step
-// table [N][N+1] in the persistent kernel only (the others read the
-// forward's copy behind the checkpoints through the scalar cache), and one
-// vega partial sum per wavefront and rate [wave][N].
-template <int F, bool Agent = false>
+// One block of the backward (paths [block * BD, ...)).  Agent: the block's
+// partials stored agent-coherent (persistent kernel).  LDS: the state adjoints
+// [N][lanes], and the step table in the persistent kernel only (the others
+// read the forward's behind the checkpoints through the scalar cache).
+template <int F, int BD, int U, bool Agent = false>
 __device__ __forceinline__ void berm_bwd_block(const Model& m, const float* __restrict__ vols,
                                                const float* __restrict__ ckpt,
                                                const float* __restrict__ lamt,
@@ -156,125 +165,89 @@ __device__ __forceinline__ void berm_bwd_block(const Model& m, const float* __re
                                                float* __restrict__ scratch,
                                                double* __restrict__ part, int block) {
   extern __shared__ float lds[];
-  __shared__ double red[4];
-  const int bd = blockDim.x;
-  const int nw = bd >> 6;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int p = block * bd + threadIdx.x;
-  const bool valid = p < m.P;
-  const int pc = valid ? p : m.P - 1;
+  const BlockPaths bp(m.P, block, BD);
   const int N = m.N;
-  const size_t P = static_cast<size_t>(m.P);
-  float lam0 = 0.0f;
-  const LamReg0 lam{lds + threadIdx.x, bd, lam0};
-  float* ltab = lds + static_cast<size_t>(N - 1) * bd;
-  float* vslots = ltab + (Agent ? step_table_floats(N) : 0);
-  float* myslots = vslots + static_cast<size_t>(wave) * N;
+  const bool valid = static_cast<int>(threadIdx.x) < bp.n;
+  const size_t p = bp.p0 + threadIdx.x;
+  const LaneRows<BD> lam{lds + threadIdx.x};
+  float* ltab = lds + static_cast<size_t>(N) * BD;
   if (Agent) fill_step_table<F>(m, ltab);
-  for (int r = 1; r < N; ++r) lam.set(r, 0.0f);
-  for (int i = threadIdx.x; i < nw * N; i += bd) vslots[i] = 0.0f;
-  __syncthreads();
+  for (int r = 0; r < N; ++r) lam.set(r, 0.0f);
+  if (Agent) __syncthreads();
   const auto ctab = [&]() {
     if constexpr (Agent) return static_cast<const float*>(ltab);
     else return cmem(ckpt + berm_ckpt_floats<F>(m));
   }();
+  VegaSums<kVegaTiles<BD>> vegas;
+  vegas.clear();
 
   const int tau = valid ? tau_in[p] : -1;
   const float V = valid ? vin[p] : 0.0f;
   // The wavefront's last exercise step, made a scalar (the butterfly leaves
   // it in every lane) so the loops below and their addresses are uniform.
   const int s_top = __builtin_amdgcn_readfirstlane(wave_max_int(tau));
-  const size_t slot = static_cast<size_t>(N + 1 + 2 * F) * P;
+  const size_t slot = static_cast<size_t>(N + 1 + 2 * F) * bp.P;
   const bool every = m.k == 1;
+  Ahead<F, U> ahead;
   for (int seg = s_top < 0 ? -1 : s_top / m.k; seg >= 0; --seg) {
     const int s0 = seg * m.k;
     const int s1 = min(s_top + 1, s0 + m.k);
-    const float* ck = ckpt + static_cast<size_t>(seg) * (every ? slot : (N + 1) * P) + pc;
+    const float* ck = ckpt + static_cast<size_t>(seg) * (every ? slot : (N + 1) * bp.P);
     for (int s = s0; s < (every ? s0 : s1); ++s) {
       const int j = s - s0;
-      const float* src = (j == 0) ? ck : scratch + j * slot + pc;
-      float* dst = scratch + (j + 1) * slot + p;
-      float* sums = scratch + j * slot + static_cast<size_t>(N + 1) * P + p;
-      const bool keep = valid && (s + 1 < s1);
-      float z[F], e[F], ep[F];
-      float l_fix = 0.0f;
-      load_z<F>(m, s, pc, z);
-      pc_step<F, kStatePrefetch>(m, s, ctab + s * N, z, e, ep,
-                                 [&](int r) { return src[static_cast<size_t>(r) * P]; },
-                                 [&](int r, float v) {
-                                   if (r == s) l_fix = v;
-                                   else if (keep) dst[static_cast<size_t>(r) * P] = v;
-                                 });
-      if (valid) {
-#pragma unroll
-        for (int f = 0; f < F; ++f) {
-          sums[static_cast<size_t>(f) * P] = e[f];
-          sums[static_cast<size_t>(F + f) * P] = ep[f];
-        }
-      }
+      const float* src = j == 0 ? ck : scratch + j * slot;
+      float* cur = scratch + j * slot;
+      float* dst = cur + slot;
+      const bool keep = s + 1 < s1;
+      float z[F], y[F], d[F];
+      load_z<F>(m, bp, s, z);
+      auto load = [&](int r) { return bp.row(src, r).load(); };
+      if (j == 0) pc_fetch<F, U>(ahead, m, s, ctab, load);
+      const float xs = pc_step<F, U>(m, s, ctab, ahead, z, y, d, load, [&](int r, float x) {
+        bp.row(dst, r, keep).store(x);
+      });
+      if (keep)
+        pc_fetch<F, U>(ahead, m, s + 1, ctab, [&](int r) { return bp.row(dst, r).load(); });
+      store_sums<F>(bp, cur + static_cast<size_t>(N + 1) * bp.P, y, d);
       if (keep) {
-        const float fsx = fast_exp(l_fix) - m.disp[s];
-        dst[static_cast<size_t>(N) * P] =
-            src[static_cast<size_t>(N) * P] * fast_rcp(1.0f + m.taus[s] * fsx);
+        const float fs = fmaf(start_level(m, s), fast_exp2(xs), -m.disp[s]);
+        bp.row(dst, N).store(bp.row(src, N).load() * fast_rcp(1.0f + m.taus[s] * fs));
       }
     }
     for (int s = s1 - 1; s >= s0; --s) {
       const int j = s - s0;
-      const float* src = (j == 0) ? ck : scratch + j * slot + pc;
-      const float* sums = (every ? ck : scratch + j * slot + pc) + static_cast<size_t>(N + 1) * P;
+      const float* src = j == 0 ? ck : scratch + j * slot;
+      const float* sums = every ? ck : scratch + j * slot;
       if (s == tau)  // seed lambda with the payoff adjoint recorded at exercise
-        for (int r = s; r < N; ++r) lam.set(r, lamt[static_cast<size_t>(r) * P + p]);
-      float z[F], e[F], ep[F];
-      load_z<F>(m, s, pc, z);
-#pragma unroll
-      for (int f = 0; f < F; ++f) {
-        e[f] = sums[static_cast<size_t>(f) * P];
-        ep[f] = sums[static_cast<size_t>(F + f) * P];
-      }
-      reverse_step<F, kStatePrefetch>(
-          m, s, ctab + s * N, [&](int r) { return src[static_cast<size_t>(r) * P]; },
-          lam, z, e, ep,
-          [&](float& lp, float xs, float fs, float inv3) {
-            (void)fs;
-            if (s < tau) lp -= m.taus[s] * inv3 * V * xs;  // fixing inside B_tau
+        for (int r = s; r < N; ++r) lam.set(r, bp.row(lamt, r).load());
+      auto load = [&](int r) { return bp.row(src, r).load(); };
+      reverse_fetch<F, U>(ahead, m, s, ctab, load, lam);
+      float y[F], d[F];
+      load_sums<F>(bp, sums + static_cast<size_t>(N + 1) * bp.P, y, d);
+      // Lanes past the last path read zeros and have no exercise step: their
+      // adjoints stay zero.
+      reverse_step<F, U>(
+          m, s, ctab, ahead, load, lam, y, d,
+          [&](float& lp, float x) {
+            // the fixing inside B_tau
+            const float xs = start_level(m, s) * fast_exp2(x);
+            const float ti = m.taus[s] * fast_rcp(1.0f + m.taus[s] * (xs - m.disp[s]));
+            if (s < tau) lp -= ti * V * xs * kLn2;
           },
-          [&](int r, float w) {
-            w = valid ? w : 0.0f;
-            w += dpp_f32_quad_xor1(w);
-            w += dpp_f32_quad_xor2(w);
-            w += dpp_f32_row_half_mirror(w);
-            w += dpp_f32_row_mirror(w);
-            // every lane of a row holds the row's sum: the rows' last lanes
-            // add them to the wavefront's slot (one LDS atomic, four lanes)
-            if ((lane & 15) == 15) atomicAdd(myslots + r, w);
-          });
+          vegas);
     }
   }
-  __syncthreads();
-  for (int r = 0; r < N; ++r) {
-    const float dl = lam.get(r) / (m.f0[r] + m.disp[r]);
-    block_sum_to<Agent>(valid ? static_cast<double>(dl) : 0.0, red,
-                        part + static_cast<size_t>(block) * 2 * N + r);
-  }
-  for (int r = threadIdx.x; r < N; r += bd) {
-    double t = 0.0;
-    for (int w = 0; w < nw; ++w) t += vslots[static_cast<size_t>(w) * N + r];
-    double* o = part + static_cast<size_t>(block) * 2 * N + N + r;
-    if (Agent)
-      store_agent(o, t / vols[r]);
-    else
-      *o = t / vols[r];
-  }
+  adjoint_sums<BD, Agent>(m, vols, lds, vegas, part + static_cast<size_t>(block) * 2 * N);
 }
 
-int fwd_threads(int N) { return N <= 50 ? 256 : (N <= 75 ? 128 : 64); }
-int bwd_threads(int N) { return N <= 45 ? 256 : (N <= 71 ? 128 : 64); }
-size_t fwd_lds(int N, int t) { return sizeof(float) * (static_cast<size_t>(N) * t + step_table_floats(N)); }
-// lds_table: the persistent kernel's backward, which keeps the step table in
-// LDS.
-size_t bwd_lds(int N, int t, bool lds_table) {
-  return sizeof(float) * (static_cast<size_t>(N - 1) * t + (lds_table ? step_table_floats(N) : 0) +
-                          (t / 64) * N);
+// Blocks of 256 lanes, as the batched and persistent kernels run (the same
+// sums bit for bit); of one wavefront for long curves, whose rows fill the LDS
+// in smaller pieces.
+int block_lanes(int N) { return N <= 45 ? 256 : 64; }
+// lds_table: the persistent kernel, which keeps the step table in LDS.
+size_t rows_lds(int N, int lanes, bool lds_table) {
+  return sizeof(float) *
+         (static_cast<size_t>(N) * lanes + (lds_table ? step_table_floats(N) : 0));
 }
 
 // Host checks and the strategy argument.

@@ -36,12 +36,12 @@ using namespace lmm;
 // ---------------------------------------------------------------------------
 // Bermudan payer swaption path quantities.
 // ---------------------------------------------------------------------------
-template <int F>
-__global__ void __launch_bounds__(256)
+template <int F, int BD, int U>
+__global__ void __launch_bounds__(BD)
     k_berm_paths(KOO_MODEL_PARAMS, const ExMap ex, float* __restrict__ bv, float* __restrict__ evo,
                  float* __restrict__ numo) {
   KOO_MODEL_LOCAL;
-  berm_paths_block<F>(m, ex, bv, evo, numo, blockIdx.x);
+  berm_paths_block<F, BD, U>(m, ex, bv, evo, numo, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -540,7 +540,11 @@ __global__ void __launch_bounds__(256)
   switch (it.F) {
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
-    berm_paths_block<F>(m, it.ex, gmem(it.bv), gmem(it.ev), gmem(it.num), blk);                \
+    if (it.N >= kShortCurve)                                                                   \
+      berm_paths_block<F, 256, kWindow<F>>(m, it.ex, gmem(it.bv), gmem(it.ev), gmem(it.num),   \
+                                           blk);                                               \
+    else                                                                                       \
+      berm_paths_block<F, 256, 1>(m, it.ex, gmem(it.bv), gmem(it.ev), gmem(it.num), blk);      \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
 #undef KOO_CASE
@@ -766,15 +770,25 @@ extern "C" int bermudan_paths_gpu(int paths, int rates, int factors, const float
   const size_t lds = sizeof(float) * (static_cast<size_t>(rates) * threads + step_table_floats(rates));
   hipStream_t st = as_stream(stream);
   switch (factors) {
+#define KOO_PATHS(F, BD, U)                                                                     \
+  hipLaunchKernelGGL((k_berm_paths<F, BD, U>), dim3(blocks), dim3(BD), lds, st, variates,          \
+                     initial_rates, taus, displacements, pseudo_roots, strike, paths, rates, 1, \
+                     ex, basis_variables, exercise_values, numeraires)
 #define KOO_CASE(F)                                                                             \
   case F:                                                                                       \
-    hipLaunchKernelGGL(k_berm_paths<F>, dim3(blocks), dim3(threads), lds, st, variates,         \
-                       initial_rates, taus, displacements, pseudo_roots, strike, paths, rates, 1, \
-                       ex, basis_variables, exercise_values, numeraires);                       \
+    if (rates < kShortCurve)                                                                    \
+      KOO_PATHS(F, 256, 1);                                                                     \
+    else if (threads == 256)                                                                    \
+      KOO_PATHS(F, 256, kWindow<F>);                                                            \
+    else if (threads == 128)                                                                    \
+      KOO_PATHS(F, 128, kWindow<F>);                                                            \
+    else                                                                                        \
+      KOO_PATHS(F, 64, kWindow<F>);                                                             \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5) KOO_CASE(6) KOO_CASE(7)
     KOO_CASE(8)
 #undef KOO_CASE
+#undef KOO_PATHS
   }
   return check_launch("bermudan_paths_gpu");
 }

@@ -20,51 +20,54 @@ struct ExMap {
   int last;                          // last exercise step
 };
 
-template <int F>
+// One block (BD lanes): paths [block * BD, ...).  LDS: the states [N][lanes],
+// then the step table.
+template <int F, int BD, int U>
 __device__ __forceinline__ void berm_paths_block(const Model& m, const ExMap& ex,
                                                  float* __restrict__ bv, float* __restrict__ evo,
                                                  float* __restrict__ numo, int block) {
   extern __shared__ float lds[];
-  const int bd = blockDim.x;
-  const int p = block * bd + threadIdx.x;
-  const bool valid = p < m.P;
-  const int pc = valid ? p : m.P - 1;
-  float* L = lds + threadIdx.x;
-  float* ctab = lds + static_cast<size_t>(m.N) * bd;
-  const size_t P = static_cast<size_t>(m.P);
+  const BlockPaths b(m.P, block, BD);
+  const int N = m.N;
+  const LaneRows<BD> X{lds + threadIdx.x};
+  float* ctab = lds + static_cast<size_t>(N) * BD;
   fill_step_table<F>(m, ctab);
-  for (int r = 0; r < m.N; ++r) L[r * bd] = logf(m.f0[r] + m.disp[r]);
+  for (int r = 0; r < N; ++r) X.set(r, 0.0f);
   __syncthreads();
   float B = 1.0f;
+  const float* tab = ctab;
+  auto load = [&](int r) { return X.get(r); };
+  float zn[F];
+  load_z<F>(m, b, 0, zn);
+  Ahead<F, U> ahead;
+  pc_fetch<F, U>(ahead, m, 0, tab, load);
   for (int s = 0; s <= ex.last; ++s) {
-    float z[F], e[F], ep[F];
-    load_z<F>(m, s, pc, z);
-    pc_step<F>(m, s, ctab + s * m.N, z, e, ep, [&](int r) { return L[r * bd]; },
-               [&](int r, float v) { L[r * bd] = v; });
+    float z[F], y[F], d[F];
+#pragma unroll
+    for (int f = 0; f < F; ++f) z[f] = zn[f];
+    load_z<F>(m, b, min(s + 1, N - 1), zn);
+    const float xs = pc_step<F, U>(m, s, tab, ahead, z, y, d, load,
+                                [&](int r, float x) { X.set(r, x); });
+    if (s + 1 < N) pc_fetch<F, U>(ahead, m, s + 1, tab, load);
     const float tau = m.taus[s];
-    const float fs = fast_exp(L[s * bd]) - m.disp[s];
+    const float fs = fmaf(start_level(m, s), fast_exp2(xs), -m.disp[s]);
     const int ei = ex.e_of_step[s];
     if (ei >= 0) {
       // P_{r+1} = P_r / (1 + tau_r f_r) from P_s = 1; annuity sum tau_r P_{r+1};
       // swap rate as the annuity-weighted forward average, which equals
       // (1 - P_N) / annuity without its cancellation.
       float disc = 1.0f, ann = 0.0f, flt = 0.0f;
-      for (int r = s; r < m.N; ++r) {
-        const float fr = fast_exp(L[r * bd]) - m.disp[r];
-        const float tr = m.taus[r];
+      walk_curve<U, false>(m, s, X, [&](int, float, float fr, float tr) {
         disc *= fast_rcp(1.0f + tr * fr);
         ann += tr * disc;
         flt += tr * fr * disc;
-      }
+      });
       const float sr = flt / ann;
       const float v = (sr - m.strike) * ann;
-      if (valid) {
-        const size_t o = static_cast<size_t>(ei) * P + p;
-        bv[static_cast<size_t>(2 * ei) * P + p] = sr;
-        bv[static_cast<size_t>(2 * ei + 1) * P + p] = fs;
-        evo[o] = v > 0.0f ? v : 0.0f;
-        numo[o] = B;
-      }
+      b.row(bv, 2 * ei).store(sr);
+      b.row(bv, 2 * ei + 1).store(fs);
+      b.row(evo, ei).store(v > 0.0f ? v : 0.0f);
+      b.row(numo, ei).store(B);
     }
     B *= 1.0f + tau * fs;
   }

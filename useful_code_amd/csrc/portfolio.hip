@@ -190,7 +190,12 @@ __global__ void __launch_bounds__(kPfThreads, 3)
   case F:                                                                                      \
     for (int vb = t; vb < it.nvb; vb += T) {                                                   \
       __syncthreads();                                                                         \
-      berm_paths_block<F>(m, it.ex, gmem(it.bv), gmem(it.ev), gmem(it.num), vb);               \
+      if (it.N >= kShortCurve)                                                                 \
+        berm_paths_block<F, kPfThreads, kWindow<F>>(m, it.ex, gmem(it.bv), gmem(it.ev),        \
+                                                    gmem(it.num), vb);                         \
+      else                                                                                     \
+        berm_paths_block<F, kPfThreads, 1>(m, it.ex, gmem(it.bv), gmem(it.ev), gmem(it.num),   \
+                                           vb);                                                \
     }                                                                                          \
     break;
       KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
@@ -255,13 +260,26 @@ __global__ void __launch_bounds__(kPfThreads, 3)
   case F:                                                                                      \
     for (int vb = t; vb < it.nvb; vb += T) {                                                   \
       __syncthreads();                                                                         \
-      berm_fwd_block<F, true>(m, it.b, cf, gmem(it.ckpt), gmem(it.lamt), gmem(it.tau),         \
-                              gmem(it.vout), gmem(it.pfwd), vb);                               \
+      if (it.N >= kShortCurve)                                                                 \
+        berm_fwd_block<F, kPfThreads, kWindow<F>, true>(m, it.b, cf, gmem(it.ckpt),            \
+                                                        gmem(it.lamt), gmem(it.tau),           \
+                                                        gmem(it.vout), gmem(it.pfwd), vb);     \
+      else                                                                                     \
+        berm_fwd_block<F, kPfThreads, 1, true>(m, it.b, cf, gmem(it.ckpt), gmem(it.lamt),      \
+                                               gmem(it.tau), gmem(it.vout), gmem(it.pfwd),     \
+                                               vb);                                            \
     }                                                                                          \
     for (int vb = t; vb < it.nvb; vb += T) {                                                   \
       __syncthreads();                                                                         \
-      berm_bwd_block<F, true>(m, gmem(it.vols), gmem(it.ckpt), gmem(it.lamt), gmem(it.tau),    \
-                              gmem(it.vout), gmem(it.scratch), gmem(it.pbwd), vb);             \
+      if (it.N >= kShortCurve)                                                                 \
+        berm_bwd_block<F, kPfThreads, kWindow<F>, true>(m, gmem(it.vols), gmem(it.ckpt),       \
+                                                        gmem(it.lamt), gmem(it.tau),           \
+                                                        gmem(it.vout), gmem(it.scratch),       \
+                                                        gmem(it.pbwd), vb);                    \
+      else                                                                                     \
+        berm_bwd_block<F, kPfThreads, 1, true>(m, gmem(it.vols), gmem(it.ckpt),                \
+                                               gmem(it.lamt), gmem(it.tau), gmem(it.vout),     \
+                                               gmem(it.scratch), gmem(it.pbwd), vb);           \
     }                                                                                          \
     break;
       KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
@@ -339,8 +357,7 @@ int pf_nvb(int paths) { return (paths + kPfThreads - 1) / kPfThreads; }
 size_t pf_phase_lds(int N) {
   const size_t gen = sizeof(float) * static_cast<size_t>(N) * kPfThreads + sizeof(uint32_t) * 32 * N;
   size_t m = gen;
-  m = std::max(m, fwd_lds(N, kPfThreads));
-  m = std::max(m, bwd_lds(N, kPfThreads, true));
+  m = std::max(m, rows_lds(N, kPfThreads, true));
   m = std::max(m, sizeof(double) * static_cast<size_t>(kPfLsDoubles));
   return (m + 15) & ~static_cast<size_t>(15);
 }
