@@ -381,13 +381,13 @@ int koo_sum_f64(const double* in, long long n, double* workspace, double* out, v
  * tau_i max(f_i - K, 0) at T_{i+1} (product_aux = [K]).  Prices are in units
  * of the numeraire at T_0 (B_0 = 1).
  *
- * Forward: price (device double) and, when checkpoints != NULL, the
- * rates' state at the start of every checkpoint_every-th step plus the
- * numeraire there (with checkpoint_every == 1 also each step's final drift
- * sums, so the backward sweep recomputes nothing), then the model's step
- * table (fixed drifts and drift constants, rates*(rates+1) floats) that the
- * backward reads; all in the library's own format.  Backward: one reverse sweep per path from those
- * checkpoints (recomputing the steps in between into segment_scratch), giving
+ * Forward: price (device double) and, when checkpoints != NULL, what the
+ * backward sweep needs of the paths, in the library's own format, then the
+ * model's step table (fixed drifts and drift constants, rates*(rates+1)
+ * floats).  checkpoint_every sets the room it has: rates + 1 floats per path
+ * and checkpoint_every steps (with 1 also 2 factors floats a step, and nothing
+ * is recomputed).  Backward: one reverse sweep per path from those checkpoints
+ * (recomputing into segment_scratch the steps there was no room for), giving
  * greeks_out[0..N) = dV/df_i(0) and greeks_out[N..2N) = dV/dsigma_i with
  * A(s,i,f) proportional to sigma_i.  Sizes of all device buffers come from
  * lmm_price_workspace().  rates <= 90, factors <= 8.  product_aux is a HOST

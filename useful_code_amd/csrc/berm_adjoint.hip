@@ -28,29 +28,29 @@ using namespace lmm;
 template <int F, int BD, int U>
 __global__ void __launch_bounds__(BD)
     k_berm_fwd(KOO_MODEL_PARAMS, const BermArgs b, const double* __restrict__ coeffs,
-               float* __restrict__ ckpt, float* __restrict__ lamt, int* __restrict__ tau_out,
+               const float* __restrict__ tab, float* __restrict__ ckpt, float* __restrict__ lamt, int* __restrict__ tau_out,
                float* __restrict__ vout, double* __restrict__ part) {
   KOO_MODEL_LOCAL;
-  berm_fwd_block<F, BD, U>(m, b, CoefGlobal{coeffs}, ckpt, lamt, tau_out, vout, part, blockIdx.x);
+  berm_fwd_block<F, BD, U>(m, b, CoefGlobal{coeffs}, tab, ckpt, lamt, tau_out, vout, part, blockIdx.x);
 }
 
-template <int F, int BD, int U>
-__global__ void __launch_bounds__(BD)
-    k_berm_bwd(KOO_MODEL_PARAMS, const float* __restrict__ vols, const float* __restrict__ ckpt,
-               const float* __restrict__ lamt, const int* __restrict__ tau_in,
+template <int F, int BD, int U, int W>
+__global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
+    k_berm_bwd(KOO_MODEL_PARAMS, const float* __restrict__ vols, const float* __restrict__ tab,
+               float* __restrict__ ckpt, const float* __restrict__ lamt, const int* __restrict__ tau_in,
                const float* __restrict__ vin, float* __restrict__ scratch,
                double* __restrict__ part) {
   KOO_MODEL_LOCAL;
-  berm_bwd_block<F, BD, U>(m, vols, ckpt, lamt, tau_in, vin, scratch, part, blockIdx.x);
+  berm_bwd_block<F, BD, U>(m, vols, tab, ckpt, lamt, tau_in, vin, scratch, part, blockIdx.x);
 }
 
 // The step table (lmm_step.h) behind the checkpoints, which the forward and
 // the backward read with scalar loads.  One lane per entry of the square.
 template <int F>
-__global__ void __launch_bounds__(256) k_berm_step_table(KOO_MODEL_PARAMS, float* __restrict__ ckpt) {
+__global__ void __launch_bounds__(256) k_berm_step_table(KOO_MODEL_PARAMS, float* __restrict__ tab) {
   KOO_MODEL_LOCAL;
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < m.N * m.N) put_step_entry<F>(m, q, ckpt + berm_ckpt_floats<F>(m));
+  if (q < m.N * m.N) put_step_entry<F>(m, q, tab);
 }
 
 // ---------------------------------------------------------------------------
@@ -67,11 +67,11 @@ __global__ void __launch_bounds__(256) k_berm_step_table(KOO_MODEL_PARAMS, float
 struct BermItem {
   g_cfloat *z, *f0, *taus, *disp, *A, *vols;
   g_cdouble* coeffs;
-  g_float *ckpt, *lamt, *vout, *scratch;
+  g_float *ckpt, *tab, *lamt, *vout, *scratch;
   g_int* tau;
   g_double *part_fwd, *part_bwd, *price_out, *greeks_out;
   float strike;
-  int P, N, k, F, block0, blocks;
+  int P, N, S1, L, F, block0, blocks;
   BermArgs b;
 };
 
@@ -81,7 +81,7 @@ __device__ __forceinline__ const BermItem& find_item(const BermItem* items, int 
 
 __device__ __forceinline__ Model item_model(const BermItem& it) {
   return Model{gmem(it.z), cmem(it.f0), cmem(it.taus), cmem(it.disp), cmem(it.A), it.strike,
-               it.P, it.N, it.k};
+               it.P, it.N, it.S1, it.L};
 }
 
 // Every product's step table; grid (blocks of 256 entries, products).
@@ -93,14 +93,14 @@ __global__ void __launch_bounds__(256) k_berm_step_table_batch(const BermItem* _
   switch (it.F) {
 #define KOO_CASE(F)                                                      \
   case F:                                                                \
-    put_step_entry<F>(m, q, gmem(it.ckpt) + berm_ckpt_floats<F>(m));     \
+    put_step_entry<F>(m, q, gmem(it.tab));                               \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
 #undef KOO_CASE
   }
 }
 
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kAdjLanes)
     k_berm_fwd_batch(const BermItem* __restrict__ items, int n, int block_offset) {
   const int block = blockIdx.x + block_offset;
   const BermItem& it = find_item(items, n, block);
@@ -110,11 +110,11 @@ __global__ void __launch_bounds__(256)
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
     if (it.N >= kShortCurve)                                                                   \
-      berm_fwd_block<F, 256, kWindow<F>>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.ckpt),  \
+      berm_fwd_block<F, kAdjLanes, kWindow<F>>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.tab), gmem(it.ckpt),  \
                                          gmem(it.lamt), gmem(it.tau), gmem(it.vout),           \
                                          gmem(it.part_fwd), blk);                              \
     else                                                                                       \
-      berm_fwd_block<F, 256, 1>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.ckpt),           \
+      berm_fwd_block<F, kAdjLanes, 1>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.tab), gmem(it.ckpt),           \
                                 gmem(it.lamt), gmem(it.tau), gmem(it.vout), gmem(it.part_fwd), \
                                 blk);                                                          \
     break;
@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kAdjLanes) __attribute__((amdgpu_waves_per_eu(2, 4)))
     k_berm_bwd_batch(const BermItem* __restrict__ items, int n, int block_offset) {
   const int block = blockIdx.x + block_offset;
   const BermItem& it = find_item(items, n, block);
@@ -133,11 +133,11 @@ __global__ void __launch_bounds__(256)
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
     if (it.N >= kShortCurve)                                                                   \
-      berm_bwd_block<F, 256, kWindow<F>>(m, gmem(it.vols), gmem(it.ckpt), gmem(it.lamt),       \
+      berm_bwd_block<F, kAdjLanes, kWindow<F>>(m, gmem(it.vols), gmem(it.tab), gmem(it.ckpt), gmem(it.lamt),       \
                                          gmem(it.tau), gmem(it.vout), gmem(it.scratch),        \
                                          gmem(it.part_bwd), blk);                              \
     else                                                                                       \
-      berm_bwd_block<F, 256, 1>(m, gmem(it.vols), gmem(it.ckpt), gmem(it.lamt), gmem(it.tau),  \
+      berm_bwd_block<F, kAdjLanes, 1>(m, gmem(it.vols), gmem(it.tab), gmem(it.ckpt), gmem(it.lamt), gmem(it.tau),  \
                                 gmem(it.vout), gmem(it.scratch), gmem(it.part_bwd), blk);      \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
@@ -151,11 +151,13 @@ __global__ void __launch_bounds__(256)
     k_berm_finalize_batch(const BermItem* __restrict__ items, int fwd) {
   const BermItem& it = items[blockIdx.y];
   const double scale = 1.0 / static_cast<double>(it.P);
+  const int waves = wave_count(it.P);
   if (fwd) {
     if (blockIdx.x == 0)
-      finalize_col(gmem(it.part_fwd), it.blocks, 1, 0, scale, gmem(it.price_out));
+      finalize_col(gmem(it.part_fwd), waves, 1, 0, scale, gmem(it.price_out));
   } else if (static_cast<int>(blockIdx.x) < 2 * it.N) {
-    finalize_col(gmem(it.part_bwd), it.blocks, 2 * it.N, blockIdx.x, scale, gmem(it.greeks_out));
+    finalize_col(gmem(it.part_bwd) + static_cast<size_t>(blockIdx.x) * waves, waves, 1, 0, scale,
+                 gmem(it.greeks_out) + blockIdx.x);
   }
 }
 
@@ -171,18 +173,15 @@ extern "C" int bermudan_adjoint_workspace(int paths, int rates, int factors, int
     return e;
   const size_t P = static_cast<size_t>(paths);
   const int k = checkpoint_every;
-  const size_t nseg = (rates + k - 1) / k;
-  const size_t rows = k == 1 ? rates + 1 + 2 * factors : rates + 1;
-  // the checkpoints, then the step table the forward copies for the backward
-  if (checkpoint_bytes) *checkpoint_bytes = sizeof(float) * (nseg * rows * P + step_table_floats(rates));
+  // the checkpoints, then the step table
+  if (checkpoint_bytes)
+    *checkpoint_bytes = sizeof(float) * (ckpt_rows(rates, factors, k) * P + step_table_floats(rates));
   if (scratch_bytes)
-    *scratch_bytes = k == 1 ? sizeof(float)
-                            : sizeof(float) * static_cast<size_t>(k < rates ? k : rates) *
-                                  (rates + 1 + 2 * factors) * P;
+    *scratch_bytes = sizeof(float) * (k == 1 ? 1 : scratch_rows(rates, factors, k) * P);
   // payoff adjoints (rates x P floats), exercise step (P ints), value (P floats)
   if (path_bytes) *path_bytes = sizeof(float) * (static_cast<size_t>(rates) + 2) * P;
-  const int t = block_lanes(rates);
-  if (partial_bytes) *partial_bytes = sizeof(double) * ((P + t - 1) / t) * 2 * rates;
+  if (partial_bytes)
+    *partial_bytes = sizeof(double) * static_cast<size_t>(wave_count(paths)) * 2 * rates;
   return KOO_OK;
 }
 
@@ -206,34 +205,37 @@ extern "C" int bermudan_frozen_fwd(int paths, int rates, int factors, int checkp
   float* lamt = path_buffers;
   int* tau = reinterpret_cast<int*>(path_buffers + static_cast<size_t>(rates) * P);
   float* vout = path_buffers + static_cast<size_t>(rates + 1) * P;
-  const int threads = block_lanes(rates);
+  const int threads = fwd_lanes(paths, rates);
   const int blocks = (paths + threads - 1) / threads;
-  const size_t lds = rows_lds(rates, threads, false);
+  const size_t lds = rows_lds(rates, rates, threads, false);
+  const SweepPlan plan = sweep_plan(rates, factors, checkpoint_every);
+  float* tab =
+      checkpoints + static_cast<size_t>(ckpt_rows(rates, factors, checkpoint_every)) * paths;
   hipStream_t st = as_stream(stream);
   switch (factors) {
 #define KOO_FWD(F, BD, U)                                                                      \
   hipLaunchKernelGGL((k_berm_fwd<F, BD, U>), dim3(blocks), dim3(BD), lds, st, variates,           \
                      initial_rates, taus, displacements, pseudo_roots, strike, paths, rates,   \
-                     checkpoint_every, b, coefficients, checkpoints, lamt, tau, vout, partials)
+                     plan.S1, plan.L, b, coefficients, tab, checkpoints, lamt, tau, vout, partials)
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
     hipLaunchKernelGGL(k_berm_step_table<F>, dim3((rates * rates + 255) / 256), dim3(256), 0,  \
                        st, variates, initial_rates, taus, displacements, pseudo_roots, strike, \
-                       paths, rates, checkpoint_every, checkpoints);                           \
+                       paths, rates, plan.S1, plan.L, tab);                                    \
     if (threads == 64)                                                                         \
       KOO_FWD(F, 64, kWindow<F>);                                                               \
     else if (rates >= kShortCurve)                                                             \
-      KOO_FWD(F, 256, kWindow<F>);                                                              \
+      KOO_FWD(F, kAdjLanes, kWindow<F>);                                                         \
     else                                                                                       \
-      KOO_FWD(F, 256, 1);                                                                       \
+      KOO_FWD(F, kAdjLanes, 1);                                                                  \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5) KOO_CASE(6) KOO_CASE(7)
     KOO_CASE(8)
 #undef KOO_CASE
 #undef KOO_FWD
   }
-  hipLaunchKernelGGL(k_finalize_cols, dim3(1), dim3(256), 0, st, partials, blocks, 1,
-                     1.0 / static_cast<double>(paths), price_out);
+  hipLaunchKernelGGL(k_finalize_rows, dim3(1), dim3(finalize_lanes(wave_count(paths))), 0, st,
+                     partials, wave_count(paths), 1.0 / static_cast<double>(paths), price_out);
   return check_launch("bermudan_frozen_fwd");
 }
 
@@ -252,32 +254,37 @@ extern "C" int bermudan_frozen_bwd(int paths, int rates, int factors, int checkp
   const float* lamt = path_buffers;
   const int* tau = reinterpret_cast<const int*>(path_buffers + static_cast<size_t>(rates) * P);
   const float* vin = path_buffers + static_cast<size_t>(rates + 1) * P;
-  const int threads = block_lanes(rates);
+  const int threads = bwd_lanes(paths, rates);
   const int blocks = (paths + threads - 1) / threads;
-  const size_t lds = rows_lds(rates, threads, false);
+  const size_t lds = rows_lds(rates, 2 * rates, threads, false);
+  const SweepPlan plan = sweep_plan(rates, factors, checkpoint_every);
+  const float* tab =
+      checkpoints + static_cast<size_t>(ckpt_rows(rates, factors, checkpoint_every)) * paths;
   hipStream_t st = as_stream(stream);
   switch (factors) {
-#define KOO_BWD(F, BD, U)                                                                      \
-  hipLaunchKernelGGL((k_berm_bwd<F, BD, U>), dim3(blocks), dim3(BD), lds, st, variates,           \
+#define KOO_BWD(F, BD, U, W)                                                                     \
+  hipLaunchKernelGGL((k_berm_bwd<F, BD, U, W>), dim3(blocks), dim3(BD), lds, st, variates,           \
                      initial_rates, taus, displacements, pseudo_roots, strike, paths, rates,   \
-                     checkpoint_every, vols, checkpoints, lamt, tau, vin, segment_scratch,     \
+                     plan.S1, plan.L, vols, tab, const_cast<float*>(checkpoints), lamt, tau, vin, segment_scratch,     \
                      partials)
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
-    if (threads == 64)                                                                         \
-      KOO_BWD(F, 64, kWindow<F>);                                                               \
-    else if (rates >= kShortCurve)                                                             \
-      KOO_BWD(F, 256, kWindow<F>);                                                              \
+    if (rates < kShortCurve)                                                                   \
+      KOO_BWD(F, kAdjLanes, 1, 2);                                                             \
+    else if (threads == kAdjLanes)                                                             \
+      KOO_BWD(F, kAdjLanes, kWindow<F>, 2);                                                    \
+    else if (rates <= 64)                                                                      \
+      KOO_BWD(F, 64, kWindow<F>, 2);                                                           \
     else                                                                                       \
-      KOO_BWD(F, 256, 1);                                                                       \
+      KOO_BWD(F, 64, kWindow<F>, 1);                                                           \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5) KOO_CASE(6) KOO_CASE(7)
     KOO_CASE(8)
 #undef KOO_CASE
 #undef KOO_BWD
   }
-  hipLaunchKernelGGL(k_finalize_cols, dim3(2 * rates), dim3(256), 0, st, partials, blocks,
-                     2 * rates, 1.0 / static_cast<double>(paths), greeks_out);
+  hipLaunchKernelGGL(k_finalize_rows, dim3(2 * rates), dim3(finalize_lanes(wave_count(paths))), 0,
+                     st, partials, wave_count(paths), 1.0 / static_cast<double>(paths), greeks_out);
   return check_launch("bermudan_frozen_bwd");
 }
 
@@ -331,9 +338,13 @@ extern "C" int bermudan_portfolio_prepare(int n_products, const koo_berm_product
     it.strike = q.strike;
     it.P = q.paths;
     it.N = q.rates;
-    it.k = q.checkpoint_every;
+    const SweepPlan sweep = sweep_plan(q.rates, q.factors, q.checkpoint_every);
+    it.S1 = sweep.S1;
+    it.L = sweep.L;
+    it.tab = (g_float*)(q.checkpoints +
+                        static_cast<size_t>(ckpt_rows(q.rates, q.factors, q.checkpoint_every)) * P);
     it.F = q.factors;
-    it.blocks = (q.paths + 255) / 256;
+    it.blocks = (q.paths + kAdjLanes - 1) / kAdjLanes;
     // work ~ paths x rate updates up to the last exercise step
     double u = 0.0;
     for (int s = 0; s <= it.b.last; ++s) u += q.rates - s;
@@ -390,10 +401,10 @@ static int portfolio_launch(const char* who, bool fwd, const koo_portfolio_plan*
     if (nc < 1 || nc > N || nb < 1 || b0 < 0 || b0 + nb > plan->blocks)
       return set_error(KOO_ERR_INVALID, "%s: bad plan class %d", who, c);
     if (fwd)
-      hipLaunchKernelGGL(k_berm_fwd_batch, dim3(nb), dim3(256), rows_lds(nc, 256, false), st, items,
+      hipLaunchKernelGGL(k_berm_fwd_batch, dim3(nb), dim3(kAdjLanes), rows_lds(nc, nc, kAdjLanes, false), st, items,
                          plan->products, b0);
     else
-      hipLaunchKernelGGL(k_berm_bwd_batch, dim3(nb), dim3(256), rows_lds(nc, 256, false), st, items,
+      hipLaunchKernelGGL(k_berm_bwd_batch, dim3(nb), dim3(kAdjLanes), rows_lds(nc, 2 * nc, kAdjLanes, false), st, items,
                          plan->products, b0);
   }
   hipLaunchKernelGGL(k_berm_finalize_batch, dim3(fwd ? 1 : 2 * N, plan->products), dim3(256), 0,

@@ -18,20 +18,6 @@ struct BermArgs {
   float sh[kMaxBermDates][2], sc[kMaxBermDates][2];
 };
 
-__device__ __forceinline__ int wave_max_int(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-  return v;
-}
-
-// Floats of a product's checkpoint buffer before the step table that the
-// single-product and batched forwards copy behind them.
-template <int F>
-__device__ __forceinline__ size_t berm_ckpt_floats(const Model& m) {
-  const size_t rows = m.k == 1 ? m.N + 1 + 2 * F : m.N + 1;
-  return static_cast<size_t>((m.N + m.k - 1) / m.k) * rows * static_cast<size_t>(m.P);
-}
-
 // Coefficients of the frozen strategy, date ei, function j, as FP32: from
 // FP64 device memory (uniform addresses: scalar loads) or from an FP32 table.
 struct CoefGlobal {
@@ -43,13 +29,14 @@ struct CoefTable {
   __device__ float operator()(int ei, int j) const { return t[6 * ei + j]; }
 };
 
-// One block of the forward: paths [block * BD, ...) of product m.  Ctab: the
-// step table behind the checkpoints (scalar loads), or the block's own copy in
-// LDS behind its states (the persistent kernel, whose backward runs in the
-// same launch).  Agent: the block's price partial stored agent-coherent (the
-// persistent kernel).
+// One block of the forward: paths [block * BD, ...) of product m.  tab: the step
+// table (scalar loads); the persistent kernel (Agent) keeps its own in LDS
+// behind the states and stores the block's price partial agent-coherent.
+// The checkpoint rows are SweepPlan's, the 1/B row of the states at S1 holding
+// the number of steps the wavefront ran (as float) in its place.
 template <int F, int BD, int U, bool Agent = false, class Coef>
 __device__ __forceinline__ void berm_fwd_block(const Model& m, const BermArgs& b, const Coef& cf,
+                                               const float* __restrict__ tab,
                                                float* __restrict__ ckpt, float* __restrict__ lamt,
                                                int* __restrict__ tau_out,
                                                float* __restrict__ vout,
@@ -66,14 +53,22 @@ __device__ __forceinline__ void berm_fwd_block(const Model& m, const BermArgs& b
   if (Agent) __syncthreads();
   const auto ctab = [&]() {
     if constexpr (Agent) return static_cast<const float*>(ltab);
-    else return cmem(ckpt + berm_ckpt_floats<F>(m));
+    else return cmem(tab);
   }();
   float invB = 1.0f, V = 0.0f;
   int tau = -1;
   bool done = !valid;
-  const int rows = m.k == 1 ? N + 1 + 2 * F : N + 1;
-  auto slot = [&](int s) { return ckpt + static_cast<size_t>(s / m.k) * rows * bp.P; };
-  for (int r = 0; r < N; ++r) bp.row(slot(0), r).store(0.0f);
+  auto row = [&](int r) { return ckpt + static_cast<size_t>(r) * bp.P; };
+  int seg_step = m.S1, seg = 0;  // the next step whose states are kept
+  auto keep_states = [&](int s) {
+    const int lo = seg == 0 ? 0 : s;
+    dump_states(bp, X,
+                row(seg == 0 ? sweep_state_row(F, m.S1)
+                             : sweep_segment_row(N, F, m.S1, m.L, seg)),
+                lo, N);
+    ++seg;
+    seg_step += m.L;
+  };
   auto load = [&](int r) { return X.get(r); };
   float zn[F];
   load_z<F>(m, bp, 0, zn);
@@ -84,27 +79,18 @@ __device__ __forceinline__ void berm_fwd_block(const Model& m, const BermArgs& b
   const auto last_step = [&](int last) {
     return __builtin_amdgcn_readfirstlane(__builtin_amdgcn_ballot_w64(!done) != 0 ? last : -1);
   };
+  int steps = 0;  // run so far
   for (int s = 0, last = last_step(b.last); s <= last; ++s, last = last_step(last)) {
+    if (s == seg_step) keep_states(s);
     float z[F], y[F], d[F];
 #pragma unroll
     for (int f = 0; f < F; ++f) z[f] = zn[f];
     load_z<F>(m, bp, min(s + 1, N - 1), zn);
-    float xs;
-    if (s + 1 < N && (s + 1) % m.k == 0) {
-      const float* next = slot(s + 1);
-      xs = pc_step<F, U>(m, s, ctab, ahead, z, y, d, load, [&](int r, float x) {
-        X.set(r, x);
-        bp.row(next, r).store(x);
-      });
-    } else {
-      xs = pc_step<F, U>(m, s, ctab, ahead, z, y, d, load, [&](int r, float x) { X.set(r, x); });
-    }
+    const float xs = pc_step<F, U>(m, s, ctab, ahead, z, y, d, load,
+                                   [&](int r, float x) { X.set(r, x); });
+    steps = s + 1;
     if (s + 1 < N) pc_fetch<F, U>(ahead, m, s + 1, ctab, load);
-    if (s % m.k == 0) {
-      const float* c = slot(s) + static_cast<size_t>(N) * bp.P;
-      bp.row(c).store(invB);
-      if (m.k == 1) store_sums<F>(bp, c + bp.P, y, d);
-    }
+    if (s < m.S1) store_sums<F>(bp, row(2 * F * s), y, d);
     const float fs = fmaf(start_level(m, s), fast_exp2(xs), -m.disp[s]);
     const int ei = b.e_of_step[s];
     if (ei >= 0) {  // uniform: done lanes walk along
@@ -143,22 +129,27 @@ __device__ __forceinline__ void berm_fwd_block(const Model& m, const BermArgs& b
     }
     invB *= fast_rcp(1.0f + m.taus[s] * fs);
   }
+  if (seg == 0) keep_states(steps);  // stopped before step S1
+  bp.row(row(sweep_state_row(F, m.S1)), N).store(static_cast<float>(steps));
   if (valid) {
     tau_out[p] = tau;
     vout[p] = V;
   }
-  // (the states are done with: their rows hold the wavefronts' sums)
-  block_sum_to<Agent>(valid ? static_cast<double>(V) : 0.0, reinterpret_cast<double*>(lds),
-                      part + block);
+  const double sum = wave_sum_f64(valid ? static_cast<double>(V) : 0.0);
+  if ((threadIdx.x & 63) == 0)
+    put_partial<Agent>(part, wave_count(m.P), wave_index<BD>(block), 0, sum);
 }
 
-// One block of the backward (paths [block * BD, ...)).  Agent: the block's
-// partials stored agent-coherent (persistent kernel).  LDS: the state adjoints
-// [N][lanes], and the step table in the persistent kernel only (the others
-// read the forward's behind the checkpoints through the scalar cache).
+// One block of the backward (paths [block * BD, ...)).  LDS: the state adjoints
+// and the states, 2N rows of lanes.  Agent (the persistent kernel): the
+// partials stored agent-coherent; the step table in LDS behind the adjoints,
+// and the states in place in the rows that the forward kept them in (the next
+// run's forward writes those again), so that three blocks fit a CU as in its
+// other phases.
 template <int F, int BD, int U, bool Agent = false>
 __device__ __forceinline__ void berm_bwd_block(const Model& m, const float* __restrict__ vols,
-                                               const float* __restrict__ ckpt,
+                                               const float* __restrict__ tab,
+                                               float* __restrict__ ckpt,
                                                const float* __restrict__ lamt,
                                                const int* __restrict__ tau_in,
                                                const float* __restrict__ vin,
@@ -176,78 +167,86 @@ __device__ __forceinline__ void berm_bwd_block(const Model& m, const float* __re
   if (Agent) __syncthreads();
   const auto ctab = [&]() {
     if constexpr (Agent) return static_cast<const float*>(ltab);
-    else return cmem(ckpt + berm_ckpt_floats<F>(m));
+    else return cmem(tab);
   }();
   VegaSums<kVegaTiles<BD>> vegas;
   vegas.clear();
 
   const int tau = valid ? tau_in[p] : -1;
   const float V = valid ? vin[p] : 0.0f;
-  // The wavefront's last exercise step, made a scalar (the butterfly leaves
-  // it in every lane) so the loops below and their addresses are uniform.
-  const int s_top = __builtin_amdgcn_readfirstlane(wave_max_int(tau));
-  const size_t slot = static_cast<size_t>(N + 1 + 2 * F) * bp.P;
-  const bool every = m.k == 1;
-  Ahead<F, U> ahead;
-  for (int seg = s_top < 0 ? -1 : s_top / m.k; seg >= 0; --seg) {
-    const int s0 = seg * m.k;
-    const int s1 = min(s_top + 1, s0 + m.k);
-    const float* ck = ckpt + static_cast<size_t>(seg) * (every ? slot : (N + 1) * bp.P);
-    for (int s = s0; s < (every ? s0 : s1); ++s) {
-      const int j = s - s0;
-      const float* src = j == 0 ? ck : scratch + j * slot;
-      float* cur = scratch + j * slot;
-      float* dst = cur + slot;
-      const bool keep = s + 1 < s1;
+  auto row = [&](int r) { return ckpt + static_cast<size_t>(r) * bp.P; };
+  float* states = row(sweep_state_row(F, m.S1));
+  // the states, from their rows at `rows` (rates lo..N-1)
+  auto begin_states = [&](float* rows, int lo) {
+    if constexpr (Agent) {
+      return GlobalRows{bp, rows - static_cast<size_t>(lo) * bp.P};
+    } else {
+      const LaneRows<BD> X{lds + N * BD + threadIdx.x};
+      load_states(bp, X, rows, lo, N);
+      return X;
+    }
+  };
+  // The steps the wavefront's forward ran, which the kept states are after: a
+  // scalar, so that the loops below and their addresses are uniform.  (Lanes
+  // past the last path read 0; a wavefront of such lanes does nothing.)
+  const int top = __builtin_amdgcn_readfirstlane(static_cast<int>(bp.row(states, N).load()));
+  // Lanes past the last path have no exercise step: their adjoints stay zero.
+  auto seed = [&](int s) {
+    if (s == tau)  // the payoff adjoint recorded at exercise
+      for (int r = s; r < N; ++r) lam.set(r, bp.row(lamt, r).load());
+  };
+  auto fixing = [&](int s, float& lp, float x) {
+    // the fixing inside B_tau
+    const float xs = start_level(m, s) * fast_exp2(x);
+    const float ti = m.taus[s] * fast_rcp(1.0f + m.taus[s] * (xs - m.disp[s]));
+    if (s < tau) lp -= ti * V * xs * kLn2;
+  };
+  // The steps from S1 on: each segment run again, its sums to scratch, then
+  // reversed.
+  for (int seg = m.S1 < top ? (top - m.S1 - 1) / m.L : -1; seg >= 0; --seg) {
+    const int s0 = m.S1 + seg * m.L, s1 = min(top, s0 + m.L);
+    const auto X =
+        seg == 0 ? begin_states(states, 0)  // the rates that have fixed come first
+                 : begin_states(row(sweep_segment_row(N, F, m.S1, m.L, seg)), s0);
+    auto load = [&](int r) { return X.get(r); };
+    float zn[F];
+    load_z<F>(m, bp, s0, zn);
+    Ahead<F, U> ahead;
+    pc_fetch<F, U>(ahead, m, s0, ctab, load);
+    for (int s = s0; s < s1; ++s) {
       float z[F], y[F], d[F];
-      load_z<F>(m, bp, s, z);
-      auto load = [&](int r) { return bp.row(src, r).load(); };
-      if (j == 0) pc_fetch<F, U>(ahead, m, s, ctab, load);
-      const float xs = pc_step<F, U>(m, s, ctab, ahead, z, y, d, load, [&](int r, float x) {
-        bp.row(dst, r, keep).store(x);
-      });
-      if (keep)
-        pc_fetch<F, U>(ahead, m, s + 1, ctab, [&](int r) { return bp.row(dst, r).load(); });
-      store_sums<F>(bp, cur + static_cast<size_t>(N + 1) * bp.P, y, d);
-      if (keep) {
-        const float fs = fmaf(start_level(m, s), fast_exp2(xs), -m.disp[s]);
-        bp.row(dst, N).store(bp.row(src, N).load() * fast_rcp(1.0f + m.taus[s] * fs));
-      }
+#pragma unroll
+      for (int f = 0; f < F; ++f) z[f] = zn[f];
+      load_z<F>(m, bp, min(s + 1, N - 1), zn);
+      pc_step<F, U>(m, s, ctab, ahead, z, y, d, load, [&](int r, float x) { X.set(r, x); });
+      if (s + 1 < s1) pc_fetch<F, U>(ahead, m, s + 1, ctab, load);
+      store_sums<F>(bp, scratch + static_cast<size_t>(2 * F * (s - s0)) * bp.P, y, d);
     }
-    for (int s = s1 - 1; s >= s0; --s) {
-      const int j = s - s0;
-      const float* src = j == 0 ? ck : scratch + j * slot;
-      const float* sums = every ? ck : scratch + j * slot;
-      if (s == tau)  // seed lambda with the payoff adjoint recorded at exercise
-        for (int r = s; r < N; ++r) lam.set(r, bp.row(lamt, r).load());
-      auto load = [&](int r) { return bp.row(src, r).load(); };
-      reverse_fetch<F, U>(ahead, m, s, ctab, load, lam);
-      float y[F], d[F];
-      load_sums<F>(bp, sums + static_cast<size_t>(N + 1) * bp.P, y, d);
-      // Lanes past the last path read zeros and have no exercise step: their
-      // adjoints stay zero.
-      reverse_step<F, U>(
-          m, s, ctab, ahead, load, lam, y, d,
-          [&](float& lp, float x) {
-            // the fixing inside B_tau
-            const float xs = start_level(m, s) * fast_exp2(x);
-            const float ti = m.taus[s] * fast_rcp(1.0f + m.taus[s] * (xs - m.disp[s]));
-            if (s < tau) lp -= ti * V * xs * kLn2;
-          },
-          vegas);
-    }
+    reverse_steps<F, U>(m, bp, s1, s0, scratch, ctab, X, lam, seed, fixing, vegas);
   }
-  adjoint_sums<BD, Agent>(m, vols, lds, vegas, part + static_cast<size_t>(block) * 2 * N);
+  // The steps whose sums the forward kept, from the states there or those that
+  // segment 0 has gone back to (which are in place already).
+  const auto X = [&]() {
+    if constexpr (Agent) return GlobalRows{bp, states};
+    else return LaneRows<BD>{lds + N * BD + threadIdx.x};
+  }();
+  if (!Agent && top <= m.S1) load_states(bp, X, states, 0, N);
+  reverse_steps<F, U>(m, bp, min(top, m.S1), 0, ckpt, ctab, X, lam, seed, fixing, vegas);
+  adjoint_sums<BD, Agent>(m, vols, lam, vegas, part, block);
 }
 
-// Blocks of 256 lanes, as the batched and persistent kernels run (the same
-// sums bit for bit); of one wavefront for long curves, whose rows fill the LDS
-// in smaller pieces.
-int block_lanes(int N) { return N <= 45 ? 256 : 64; }
+// Lanes per block of the single-product kernels (the batched and persistent
+// ones run kAdjLanes).
+int fwd_lanes(int paths, int N) {
+  return N < kShortCurve || (N <= 2 * kAdjRates && paths >= 32768) ? kAdjLanes : 64;
+}
+int bwd_lanes(int paths, int N) {
+  return N < kShortCurve || (N <= kAdjRates && paths >= 32768) ? kAdjLanes : 64;
+}
 // lds_table: the persistent kernel, which keeps the step table in LDS.
-size_t rows_lds(int N, int lanes, bool lds_table) {
+size_t rows_lds(int N, int rows, int lanes, bool lds_table) {
   return sizeof(float) *
-         (static_cast<size_t>(N) * lanes + (lds_table ? step_table_floats(N) : 0));
+         (static_cast<size_t>(rows) * lanes + (lds_table ? step_table_floats(N) : 0));
 }
 
 // Host checks and the strategy argument.

@@ -95,8 +95,48 @@ struct Model {
   c_cfloat disp;      // N
   c_cfloat A;         // (S,N,F)
   float strike;
-  int P, N, k;
+  int P, N;
+  int S1, L;  // SweepPlan of the adjoint
 };
+
+// What the forward keeps for the reverse sweep, in the rows (of P) that the
+// checkpoint interval pays for.  The reverse of a step needs that step's final
+// sums and the states after it: it recovers the states before it from them
+// (reverse_step), so no step's states have to be kept but the last's.  Steps
+// 0..S1-1 keep their sums (2F rows each); as many as the checkpoint buffer
+// holds.  The later steps are run again in segments of L, whose sums the
+// segment scratch holds, from the states at S1, S1 + L, ...
+// Checkpoint rows: the sums; the N states when step S1 begins (those of rates
+// that have fixed as they fixed) and 1/B there; then per further segment the
+// alive states and 1/B when it begins.
+struct SweepPlan {
+  int S1, L;
+};
+__host__ __device__ constexpr int sweep_state_row(int F, int S1) { return 2 * F * S1; }
+// First row of segment i >= 1, which begins at step S1 + i L.
+__host__ __device__ constexpr int sweep_segment_row(int N, int F, int S1, int L, int i) {
+  return 2 * F * S1 + N + 1 + (i - 1) * (N - S1 + 1) - L * (i * (i - 1) / 2);
+}
+// Rows of the checkpoint buffer and of the segment scratch at interval k.
+inline int ckpt_rows(int N, int F, int k) {
+  return k == 1 ? N * (N + 1 + 2 * F) : (N + k - 1) / k * (N + 1);
+}
+inline int scratch_rows(int N, int F, int k) { return k == 1 ? 0 : (k < N ? k : N) * (N + 1 + 2 * F); }
+// (With S1 = 0 the segments are at least k long and fit the checkpoint rows:
+// a plan always exists.)
+inline SweepPlan sweep_plan(int N, int F, int k) {
+  if (k == 1) return {N, N};
+  const int room = ckpt_rows(N, F, k);
+  int L = scratch_rows(N, F, k) / (2 * F);
+  if (L > N) L = N;
+  int S1 = N;
+  for (; S1 > 0; --S1) {
+    const int more = (N - S1 + L - 1) / L;  // segments
+    const int rows = more > 1 ? sweep_segment_row(N, F, S1, L, more) : 2 * F * S1 + N + 1;
+    if (rows <= room) break;
+  }
+  return {S1, L};
+}
 
 // The step table: for every step s and alive rate r >= s the pair
 // {fixed drift c = -0.5 log2(e) sum_f A(s,r,f)^2, kr of drift_coeff}, steps one
@@ -185,6 +225,14 @@ struct BlockPaths {
   }
 };
 
+// The same in global memory (rows of P), for blocks whose LDS has no room.
+struct GlobalRows {
+  BlockPaths b;
+  float* rows;
+  __device__ __forceinline__ float get(int r) const { return b.row(rows, r).load(); }
+  __device__ __forceinline__ void set(int r, float v) const { b.row(rows, r).store(v); }
+};
+
 // Vega terms of a wavefront, summed over its lanes on the matrix cores: the
 // term of the rate j places from the top is the A operand of a 16x16x4 product
 // whose B is one in column j mod 16, so column j of tile j / 16 collects 16
@@ -215,8 +263,10 @@ struct VegaSums {
           acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u], one[u], acc[t], 0, 0, 0);
       }
   }
-  // out[j] (LDS) = the wavefront's sum of the rate j places from the top
-  __device__ __forceinline__ void sums(double* out, int rates) const {
+  // put(j, v): the wavefront's sum of the rate j places from the top, one lane
+  // per rate
+  template <class Put>
+  __device__ __forceinline__ void sums(int rates, Put put) const {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
@@ -224,10 +274,39 @@ struct VegaSums {
                  (static_cast<double>(acc[t][2]) + static_cast<double>(acc[t][3]));
       v += __shfl_xor(v, 16, 64);
       v += __shfl_xor(v, 32, 64);
-      if (lane < 16 && 16 * t + lane < rates) out[16 * t + lane] = v;
+      if (lane < 16 && 16 * t + lane < rates) put(16 * t + lane, v);
     }
   }
 };
+
+// The variates of step s.
+template <int F>
+__device__ __forceinline__ void load_z(const Model& m, const BlockPaths& b, int s, float (&z)[F]) {
+  const size_t P = b.stride();
+  const float* zs = m.z + static_cast<size_t>(s) * F * P;
+#pragma unroll
+  for (int f = 0; f < F; ++f, zs += P) z[f] = b.row(zs).load();
+}
+
+// A step's final sums y, d in the 2F rows at `rows`.
+template <int F>
+__device__ __forceinline__ void store_sums(const BlockPaths& b, const float* rows,
+                                           const float (&y)[F], const float (&d)[F]) {
+  const size_t P = b.stride();
+#pragma unroll
+  for (int f = 0; f < F; ++f, rows += P) b.row(rows).store(y[f]);
+#pragma unroll
+  for (int f = 0; f < F; ++f, rows += P) b.row(rows).store(d[f]);
+}
+template <int F>
+__device__ __forceinline__ void load_sums(const BlockPaths& b, const float* rows, float (&y)[F],
+                                          float (&d)[F]) {
+  const size_t P = b.stride();
+#pragma unroll
+  for (int f = 0; f < F; ++f, rows += P) y[f] = b.row(rows).load();
+#pragma unroll
+  for (int f = 0; f < F; ++f, rows += P) d[f] = b.row(rows).load();
+}
 
 // Rates per window of the step loops: a window's uniform data (pseudo-roots,
 // fixed drifts, drift constants) is contiguous and is fetched into scalar
@@ -282,23 +361,18 @@ __device__ __forceinline__ float keep_scalar(float x) {
   asm volatile("" : "+s"(i));
   return __int_as_float(i);
 }
-// A table in LDS is read into vector registers and stays there.
-template <int F, int U, class Tab>
-__device__ __forceinline__ Rows<F, U> scalar_rows(const Rows<F, U>& v) {
-  constexpr bool kScalarTab = std::is_same<Tab, c_cfloat>::value;
-  Rows<F, U> w;
+// (A table in LDS is read into vector registers and stays there.)
+template <class Tab, int F, int U>
+__device__ __forceinline__ void keep_scalar(Rows<F, U>& w) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
 #pragma unroll
-    for (int f = 0; f < F; ++f) w.a[u][f] = keep_scalar(v.a[u][f]);
-    w.c[u] = v.c[u];
-    w.kr[u] = v.kr[u];
-    if constexpr (kScalarTab) {
+    for (int f = 0; f < F; ++f) w.a[u][f] = keep_scalar(w.a[u][f]);
+    if constexpr (std::is_same<Tab, c_cfloat>::value) {
       w.c[u] = keep_scalar(w.c[u]);
       w.kr[u] = keep_scalar(w.kr[u]);
     }
   }
-  return w;
 }
 
 // Windows of the alive rates s..N-1.  Ascending, all but the first are full and
@@ -314,13 +388,24 @@ __device__ __forceinline__ int part_base(int N, int s) {
   return min(s, N - U);
 }
 
-// The first window of a step, fetched while the step before it ends.
+// A fetched window.  The step loops work on two in turn (no copies: a copy of
+// a register waits for the load into it), the first of a step fetched while
+// the step before it ends.
 template <int F, int U>
 struct Ahead {
   Rows<F, U> rows;
   float x[U];  // states
-  float l[U];  // their adjoints (the reverse)
+  float l[U];  // the adjoints (the reverse)
+
+  // Waits for the window, before the next one's loads are issued.
+  template <class Tab>
+  __device__ __forceinline__ void take() {
+    window_ready();
+    keep_scalar<Tab>(rows);
+  }
 };
+// Between the loads of the next window and the work on this one.
+__device__ __forceinline__ void loads_issued() { __builtin_amdgcn_sched_barrier(0); }
 
 // Fetches the first window of PC step s; `load(r)` gives the state of rate r.
 template <int F, int U, class Tab, class Load>
@@ -329,7 +414,7 @@ __device__ __forceinline__ void pc_fetch(Ahead<F, U>& h, const Model& m, int s, 
   const int base = part_base<U>(m.N, s);
   load_rows<F, U>(h.rows, m, tab, s, base);
 #pragma unroll
-  for (int i = 0; i < U; ++i) h.x[i] = load(max(base + i, s));
+  for (int i = 0; i < U; ++i) h.x[i] = load(base + i);
 }
 
 // One predictor-corrector step s over the alive rates.  In the state's units
@@ -372,83 +457,95 @@ __device__ __forceinline__ float pc_step(const Model& m, int s, Tab tab, Ahead<F
     store(r, xn);
     return xn;
   };
-  Rows<F, U> w;
-  float x[U], first = 0.0f;
-  // takes the fetched window and fetches the one at r
-  auto take = [&](int r) {
-    window_ready();
-    w = scalar_rows<F, U, Tab>(h.rows);
+  Ahead<F, U> g;
+  auto fetch = [&](Ahead<F, U>& to, int r) {
+    load_rows<F, U>(to.rows, m, tab, s, r);
 #pragma unroll
-    for (int u = 0; u < U; ++u) x[u] = h.x[u];
-    if (r < N) {
-      load_rows<F, U>(h.rows, m, tab, s, r);
+    for (int u = 0; u < U; ++u) to.x[u] = load(r + u);
+  };
+  auto window = [&](const Ahead<F, U>& w, int r0) {
+    loads_issued();
 #pragma unroll
-      for (int u = 0; u < U; ++u) h.x[u] = load(r + u);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    for (int u = 0; u < U; ++u) rate(w.rows, u, w.x[u], r0 + u);
   };
   const int base = part_base<U>(N, s), end = part_end<U>(N, s);
-  take(end);
+  float first = 0.0f;
+  h.template take<Tab>();
+  if (end < N) fetch(g, end);
+  loads_issued();
 #pragma unroll
   for (int i = 0; i < U; ++i)
     if (base + i >= s && base + i < end) {
-      const float v = rate(w, i, x[i], base + i);
+      const float v = rate(h.rows, i, h.x[i], base + i);
       if (base + i == s) first = v;
     }
-  for (int r0 = end; r0 < N; r0 += U) {
-    take(r0 + U);
-#pragma unroll
-    for (int u = 0; u < U; ++u) rate(w, u, x[u], r0 + u);
+  int r0 = end;
+  for (; r0 + U < N; r0 += 2 * U) {
+    g.template take<Tab>();
+    fetch(h, r0 + U);
+    window(g, r0);
+    h.template take<Tab>();
+    if (r0 + 2 * U < N) fetch(g, r0 + 2 * U);
+    window(h, r0 + U);
+  }
+  if (r0 < N) {
+    g.template take<Tab>();
+    window(g, r0);
   }
   return first;
 }
 
 // Fetches the first window of the reverse of step s (rates N-1, N-2, ...): a
 // full one, or the one with rate s.
-template <int F, int U, class Tab, class Src, class Lam>
+template <int F, int U, class Tab, class States, class Lanes>
 __device__ __forceinline__ void reverse_fetch(Ahead<F, U>& h, const Model& m, int s, Tab tab,
-                                              Src src, const Lam& lam) {
+                                              const States& X, const Lanes& lam) {
   load_rows<F, U>(h.rows, m, tab, s, m.N - U);
 #pragma unroll
   for (int i = 0; i < U; ++i) {
-    const int r = max(m.N - U + i, s);
-    h.x[i] = src(r);
-    h.l[i] = lam.get(r);
+    h.x[i] = X.get(m.N - U + i);
+    h.l[i] = lam.get(m.N - U + i);
   }
 }
 
-// Reverse of PC step s over the rates N-1..s.  On entry `lam.get(r)` holds the
-// adjoint of the end-of-step state r, on exit that of the start-of-step one
-// (`lam.set`).  `h`: reverse_fetch of this step.  y / d are the step's final
-// sums (un-accumulated here); `src(r)` gives the start state of rate r.
-// `fixing(lp, x')` adds the product's adjoint of the rate fixing at the end of
-// the step (r == s) to lp; `vegas` takes w = sum_f Abar(s,r,f) A(s,r,f) of the
-// step, which contracts to scalars the reverse already has: with the adjoint
-// sums D of d and Y of y (rates descending),
+// Reverse of PC step s over the rates N-1..s.  On entry `X` holds the states
+// and `lam` their adjoints after the step, on exit those before it; y / d are
+// the step's final sums.  With the sums after rate r (un-accumulated as the
+// rates descend) the step runs backwards by itself,
+//   xh_r = x'_r - 0.5 sum a d,   x_r = xh_r - c_r - sum a y,
+// so the states before the step need not be kept.  (Each step back rounds
+// the states once more, about as the step forward does.)  `h`: reverse_fetch
+// of this step.  `fixing(lp, x')` adds the product's adjoint of the rate
+// fixing at the end of the step (r == s) to lp; `vegas` takes
+// w = sum_f Abar(s,r,f) A(s,r,f) of the step, which contracts to scalars the
+// reverse already has: with the adjoint sums D of d and Y of y (rates
+// descending),
 //   D_f += 0.5 lp a_f, q = sum a D;   xhb = lp + q dGh/dx
 //   Y_f += xhb a_f,    p = sum a Y;   lam = xhb + (p - q) dG/dx
 //   w = 0.5 lp sum a d + (Gh - G) q + G p + xhb (sum a y + 2 c).
-template <int F, int U, class Tab, class Src, class Lam, class Fixing, class Vegas>
+template <int F, int U, class Tab, class States, class Lanes, class Fixing, class Vegas>
 __device__ __forceinline__ void reverse_step(const Model& m, int s, Tab tab, Ahead<F, U>& h,
-                                             Src src, const Lam& lam, float (&y)[F],
+                                             const States& X, const Lanes& lam, float (&y)[F],
                                              float (&d)[F], Fixing fixing, Vegas& vegas) {
   const int N = m.N;
   float D[F], Y[F];
 #pragma unroll
   for (int f = 0; f < F; ++f) D[f] = Y[f] = 0.0f;
-  auto rate = [&](const Rows<F, U>& v, int u, float x, float lp, int r, bool may_fix) {
+  auto rate = [&](const Rows<F, U>& v, int u, float xe, float lp, int r, bool may_fix) {
     const float c = v.c[u];
-    const float G = drift_coeff(x, v.kr[u]);
     float my = 0.0f, md = 0.0f;
 #pragma unroll
     for (int f = 0; f < F; ++f) {
-      my = fmaf(v.a[u][f], y[f], my);
       md = fmaf(v.a[u][f], d[f], md);
+      my = fmaf(v.a[u][f], y[f], my);
     }
+    const float xh = fmaf(-0.5f, md, xe);
     const float mc = my + c;
-    const float xh = x + mc;
+    const float x = xh - mc;
     const float Gh = drift_coeff(xh, v.kr[u]);
-    if (may_fix && r == s) fixing(lp, fmaf(0.5f, md, xh));
+    const float G = drift_coeff(x, v.kr[u]);
+    X.set(r, x);
+    if (may_fix && r == s) fixing(lp, xe);
     const float lh = 0.5f * lp;
     float q = 0.0f;
 #pragma unroll
@@ -474,44 +571,91 @@ __device__ __forceinline__ void reverse_step(const Model& m, int s, Tab tab, Ahe
     }
     return fmaf(xhb, mc + c, fmaf(lh, md, uh + ug));
   };
-  Rows<F, U> v;
-  float x[U], l[U];
-  // takes the fetched window; then fetches the one at r, if any
-  auto take = [&](bool more, int r) {
-    window_ready();
-    v = scalar_rows<F, U, Tab>(h.rows);
+  Ahead<F, U> g;
+  auto fetch = [&](Ahead<F, U>& to, int r) {
+    load_rows<F, U>(to.rows, m, tab, s, r);
 #pragma unroll
     for (int i = 0; i < U; ++i) {
-      x[i] = h.x[i];
-      l[i] = h.l[i];
+      to.x[i] = X.get(r + i);
+      to.l[i] = lam.get(r + i);
     }
-    if (more) {
-      load_rows<F, U>(h.rows, m, tab, s, r);
-#pragma unroll
-      for (int i = 0; i < U; ++i) {
-        h.x[i] = src(max(r + i, s));
-        h.l[i] = lam.get(max(r + i, s));
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
   };
-  const int base = part_base<U>(N, s), end = part_end<U>(N, s);
-  // full windows [r0, r0 + U); the window after the last of them is at base
-  for (int r0 = N - U; r0 >= end; r0 -= U) {
-    take(true, r0 - U >= end ? r0 - U : base);
+  auto window = [&](const Ahead<F, U>& v, int r0) {
+    loads_issued();
     float w[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) w[u] = rate(v, U - 1 - u, x[U - 1 - u], l[U - 1 - u], r0 + U - 1 - u, false);
+    for (int u = 0; u < U; ++u)
+      w[u] = rate(v.rows, U - 1 - u, v.x[U - 1 - u], v.l[U - 1 - u], r0 + U - 1 - u, false);
     vegas.add(N - U - r0, w);
+  };
+  // full windows [r0, r0 + U); the window after the last of them is at base
+  const int base = part_base<U>(N, s), end = part_end<U>(N, s);
+  int r0 = N - U;
+  for (; r0 - U >= end; r0 -= 2 * U) {
+    h.template take<Tab>();
+    fetch(g, r0 - U);
+    window(h, r0);
+    g.template take<Tab>();
+    fetch(h, r0 - 2 * U >= end ? r0 - 2 * U : base);
+    window(g, r0 - U);
+  }
+  if (r0 >= end) {
+    h.template take<Tab>();
+    fetch(g, base);
+    window(h, r0);
+    h = g;
   }
   // the window with rate s
-  take(false, 0);
+  h.template take<Tab>();
+  loads_issued();
 #pragma unroll
   for (int i = U - 1; i >= 0; --i)
     if (base + i >= s && base + i < end) {
-      const float w[1] = {rate(v, i, x[i], l[i], base + i, true)};
+      const float w[1] = {rate(h.rows, i, h.x[i], h.l[i], base + i, true)};
       vegas.add(N - 1 - base - i, w);
     }
+}
+
+// Reverses the steps hi - 1 .. lo, whose sums are the 2F rows per step from
+// `sums` (step lo's first), fetched a step ahead.
+template <int F, int U, class Tab, class States, class Lanes, class Before, class Fixing,
+          class Vegas>
+__device__ __forceinline__ void reverse_steps(const Model& m, const BlockPaths& b, int hi, int lo,
+                                              const float* sums, Tab tab, const States& X,
+                                              const Lanes& lam, Before before, Fixing fixing,
+                                              Vegas& vegas) {
+  if (hi <= lo) return;
+  const size_t step_rows = 2 * F * b.P;
+  float yn[F], dn[F];
+  load_sums<F>(b, sums + (hi - 1 - lo) * step_rows, yn, dn);
+  Ahead<F, U> ahead;
+  for (int s = hi - 1; s >= lo; --s) {
+    before(s);
+    reverse_fetch<F, U>(ahead, m, s, tab, X, lam);
+    float y[F], d[F];
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      y[f] = yn[f];
+      d[f] = dn[f];
+    }
+    if (s > lo) load_sums<F>(b, sums + (s - 1 - lo) * step_rows, yn, dn);
+    reverse_step<F, U>(m, s, tab, ahead, X, lam, y, d,
+                       [&](float& lp, float x) { fixing(s, lp, x); }, vegas);
+  }
+}
+
+// Copies rows [lo, hi) of the states to or from the rows at `rows`.
+template <class Lanes>
+__device__ __forceinline__ void dump_states(const BlockPaths& b, const Lanes& X, const float* rows,
+                                            int lo, int hi) {
+#pragma unroll 4
+  for (int r = lo; r < hi; ++r) b.row(rows, r - lo).store(X.get(r));
+}
+template <class Lanes>
+__device__ __forceinline__ void load_states(const BlockPaths& b, const Lanes& X, const float* rows,
+                                            int lo, int hi) {
+#pragma unroll 4
+  for (int r = lo; r < hi; ++r) X.set(r, b.row(rows, r - lo).load());
 }
 
 // Walks the alive rates s..N-1 of a curve, upwards or downwards, in windows
@@ -527,7 +671,7 @@ __device__ __forceinline__ void walk_curve(const Model& m, int s, const Lanes& X
       f0n[i] = m.f0[r + i];
       dn[i] = m.disp[r + i];
       tn[i] = m.taus[r + i];
-      xn[i] = X.get(max(r + i, s));
+      xn[i] = X.get(r + i);
     }
   };
   auto take = [&](bool more, int r) {
@@ -572,74 +716,62 @@ __device__ __forceinline__ void walk_curve(const Model& m, int s, const Lanes& X
   }
 }
 
-// Tiles of VegaSums: blocks of 256 lanes take up to 45 rates, those of one
-// wavefront up to kMaxRates.
+// Lanes of the adjoint's blocks.  Four wavefronts: a CU spreads those over its
+// four SIMDs, where blocks of one or two that fill its LDS are left uneven (at
+// 2^20 paths and 40 rates, 128-lane blocks took 2.93 ms in the backward, 256
+// lanes 2.37, with the same eight wavefronts per CU).  One wavefront for few
+// paths and for curves whose rows leave no room for two such blocks.
+constexpr int kAdjLanes = 256, kAdjRates = 40;
+// Rates that the batched and persistent kernels take.
+constexpr int kBatchRates = 45;
 template <int BD>
-constexpr int kVegaTiles = BD == 256 ? 3 : (kMaxRates + 15) / 16;
+constexpr int kVegaTiles = (BD == kAdjLanes ? kBatchRates + 15 : kMaxRates + 15) / 16;
 
-// A block's sums of the state adjoints (rows of BD lanes in LDS) and vega
-// terms, as deltas (d/df0_r = log2(e) lam_r / (f0_r + d_r)) and vegas (over
-// sigma_r) into out[0..N) and out[N..2N).  Overwrites the LDS rows.  Agent: the
-// stores are agent-coherent.
-template <int BD, bool Agent = false, class Vegas>
+// Wavefronts of `paths` paths, and this one's index: every wavefront writes its
+// own partial sums (so they do not depend on the block size), column after
+// column: column c of wavefront w at part[c * waves + w].
+__host__ __device__ constexpr int wave_count(int paths) { return (paths + 63) >> 6; }
+template <int BD>
+__device__ __forceinline__ int wave_index(int block) {
+  return block * (BD / 64) + static_cast<int>(threadIdx.x >> 6);
+}
+template <bool Agent>
+__device__ __forceinline__ void put_partial(double* part, int waves, int w, int col, double v) {
+  double* o = part + static_cast<size_t>(col) * waves + w;
+  if (w >= waves) return;
+  if (Agent) store_agent(o, v);
+  else *o = v;
+}
+
+// A wavefront's sums of the state adjoints and vega terms, as deltas
+// (d/df0_r = log2(e) lam_r / (f0_r + d_r)) and vegas (over sigma_r): columns
+// 0..N-1 and N..2N-1.  Agent: the stores are agent-coherent.
+template <int BD, bool Agent = false, class Lanes, class Vegas>
 __device__ __forceinline__ void adjoint_sums(const Model& m, const float* __restrict__ vols,
-                                             float* lds, const Vegas& vegas, double* out) {
-  const int N = m.N, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  constexpr int W = BD / 64;
-  auto put = [&](double* o, double v) {
-    if (Agent) store_agent(o, v);
-    else *o = v;
-  };
-  __syncthreads();
-  // a wavefront sums whole rows
-  for (int r = wave; r < N; r += W) {
-    double v = 0.0;
+                                             const Lanes& lam, const Vegas& vegas, double* part,
+                                             int block) {
+  const int N = m.N, lane = threadIdx.x & 63;
+  const int waves = wave_count(m.P), w = wave_index<BD>(block);
+  // four rates at a time, so that their butterflies overlap
+  for (int r0 = 0; r0 < N; r0 += 4) {
+    double v[4];
 #pragma unroll
-    for (int i = 0; i < W; ++i) v += static_cast<double>(lds[r * BD + 64 * i + lane]);
-    v = wave_sum_f64(v);
-    if (lane == 0)
-      put(out + r, v * static_cast<double>(kLog2e) / static_cast<double>(start_level(m, r)));
+    for (int i = 0; i < 4; ++i) v[i] = static_cast<double>(lam.get(min(r0 + i, N - 1)));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += __shfl_xor(v[i], o, 64);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (lane == i && r0 + i < N)
+        put_partial<Agent>(part, waves, w, r0 + i,
+                           v[i] * static_cast<double>(kLog2e) /
+                               static_cast<double>(start_level(m, r0 + i)));
   }
-  __syncthreads();
-  double* red = reinterpret_cast<double*>(lds);  // [W][N]
-  vegas.sums(red + wave * N, N);
-  __syncthreads();
-  for (int j = threadIdx.x; j < N; j += BD) {
-    double v = 0.0;
-#pragma unroll
-    for (int i = 0; i < W; ++i) v += red[i * N + j];
+  vegas.sums(N, [&](int j, double v) {
     const int r = N - 1 - j;
-    put(out + N + r, v / static_cast<double>(vols[r]));
-  }
-}
-
-// The variates of step s.
-template <int F>
-__device__ __forceinline__ void load_z(const Model& m, const BlockPaths& b, int s, float (&z)[F]) {
-  const size_t P = b.stride();
-  const float* zs = m.z + static_cast<size_t>(s) * F * P;
-#pragma unroll
-  for (int f = 0; f < F; ++f, zs += P) z[f] = b.row(zs).load();
-}
-
-// A step's final sums y, d in the 2F rows at `rows`.
-template <int F>
-__device__ __forceinline__ void store_sums(const BlockPaths& b, const float* rows,
-                                           const float (&y)[F], const float (&d)[F]) {
-  const size_t P = b.stride();
-#pragma unroll
-  for (int f = 0; f < F; ++f, rows += P) b.row(rows).store(y[f]);
-#pragma unroll
-  for (int f = 0; f < F; ++f, rows += P) b.row(rows).store(d[f]);
-}
-template <int F>
-__device__ __forceinline__ void load_sums(const BlockPaths& b, const float* rows, float (&y)[F],
-                                          float (&d)[F]) {
-  const size_t P = b.stride();
-#pragma unroll
-  for (int f = 0; f < F; ++f, rows += P) y[f] = b.row(rows).load();
-#pragma unroll
-  for (int f = 0; f < F; ++f, rows += P) d[f] = b.row(rows).load();
+    put_partial<Agent>(part, waves, w, N + r, v / static_cast<double>(vols[r]));
+  });
 }
 
 // The model arrays are separate __restrict__ kernel arguments (not members of
@@ -647,9 +779,9 @@ __device__ __forceinline__ void load_sums(const BlockPaths& b, const float* rows
 #define KOO_MODEL_PARAMS                                                                  \
   const float* __restrict__ z_, const float* __restrict__ f0_,                            \
       const float* __restrict__ taus_, const float* __restrict__ disp_,                   \
-      const float* __restrict__ A_, float strike_, int P_, int N_, int k_
+      const float* __restrict__ A_, float strike_, int P_, int N_, int S1_, int L_
 #define KOO_MODEL_LOCAL \
-  const Model m{z_, cmem(f0_), cmem(taus_), cmem(disp_), cmem(A_), strike_, P_, N_, k_}
+  const Model m{z_, cmem(f0_), cmem(taus_), cmem(disp_), cmem(A_), strike_, P_, N_, S1_, L_}
 
 // Batched kernels read the pointers of their device descriptor tables as
 // global-memory pointers (address space 1), so accesses through them are
@@ -700,13 +832,23 @@ __device__ __forceinline__ void finalize_col(const double* __restrict__ part, in
   __shared__ double sv[16], sc[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   // per lane: Neumaier over a strided slice of the blocks
+  // (eight loads in flight: one at a time took 30 us for 2^14 blocks)
   double s = 0.0, c = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-    const double x = Agent ? load_agent(part + static_cast<size_t>(b) * ncols + col)
-                           : part[static_cast<size_t>(b) * ncols + col];
-    const double t = s + x;
-    c += (fabs(s) >= fabs(x)) ? (s - t) + x : (x - t) + s;
-    s = t;
+  for (int b0 = threadIdx.x; b0 < nb; b0 += 8 * blockDim.x) {
+    double v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int b = b0 + i * static_cast<int>(blockDim.x);
+      const double* src = part + static_cast<size_t>(b < nb ? b : 0) * ncols + col;
+      const double x = Agent ? load_agent(src) : *src;
+      v[i] = b < nb ? x : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const double x = v[i], t = s + x;
+      c += (fabs(s) >= fabs(x)) ? (s - t) + x : (x - t) + s;
+      s = t;
+    }
   }
   // wavefront butterfly with error-free additions (TwoSum), then the waves
 #pragma unroll
@@ -738,6 +880,15 @@ __global__ void __launch_bounds__(256)
     k_finalize_cols(const double* __restrict__ part, int nb, int ncols, double scale,
                     double* __restrict__ out) {
   finalize_col(part, nb, ncols, blockIdx.x, scale, out);
+}
+
+// The same for partials stored column after column (put_partial); as many
+// lanes as finalize_lanes.
+inline int finalize_lanes(int nb) { return nb <= 2048 ? 256 : 1024; }
+__global__ void __launch_bounds__(1024)
+    k_finalize_rows(const double* __restrict__ part, int nb, double scale,
+                    double* __restrict__ out) {
+  finalize_col(part + static_cast<size_t>(blockIdx.x) * nb, nb, 1, 0, scale, out + blockIdx.x);
 }
 
 }  // namespace

@@ -535,7 +535,7 @@ __global__ void __launch_bounds__(256)
   const int block = blockIdx.x + block_offset;
   const LsItem& it = items[find_block_owner(items, n, block, &LsItem::paths_block0)];
   const Model m{gmem(it.z), cmem(it.f0), cmem(it.taus), cmem(it.disp), cmem(it.A), it.strike,
-                it.P, it.N, 1};
+                it.P, it.N, 0, 0};
   const int blk = block - it.paths_block0;
   switch (it.F) {
 #define KOO_CASE(F)                                                                            \
@@ -772,8 +772,8 @@ extern "C" int bermudan_paths_gpu(int paths, int rates, int factors, const float
   switch (factors) {
 #define KOO_PATHS(F, BD, U)                                                                     \
   hipLaunchKernelGGL((k_berm_paths<F, BD, U>), dim3(blocks), dim3(BD), lds, st, variates,          \
-                     initial_rates, taus, displacements, pseudo_roots, strike, paths, rates, 1, \
-                     ex, basis_variables, exercise_values, numeraires)
+                     initial_rates, taus, displacements, pseudo_roots, strike, paths, rates, 0, \
+                     0, ex, basis_variables, exercise_values, numeraires)
 #define KOO_CASE(F)                                                                             \
   case F:                                                                                       \
     if (rates < kShortCurve)                                                                    \

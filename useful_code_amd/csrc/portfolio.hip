@@ -48,7 +48,7 @@ struct PfItem {
   g_float* z;
   g_cfloat *f0, *taus, *disp, *A, *vols;
   float strike;
-  int P, N, F, k;
+  int P, N, F, S1, L;
   // LS first pass (two variables per date, the cross basis)
   ExMap ex;
   int E, itm_only;
@@ -64,9 +64,9 @@ struct PfItem {
   int team0, team, nvb;
 };
 
-__device__ __forceinline__ Model pf_model(const PfItem& it, int k) {
+__device__ __forceinline__ Model pf_model(const PfItem& it) {
   return Model{gmem(it.z), cmem(it.f0), cmem(it.taus), cmem(it.disp), cmem(it.A), it.strike,
-               it.P, it.N, k};
+               it.P, it.N, it.S1, it.L};
 }
 
 // The arguments of round r of the product's first pass (as item_round_args
@@ -104,10 +104,9 @@ __device__ __forceinline__ int pf_round_entries(const PfItem& it, int r) {
   return it.E - 1 - r >= 0 ? tri_count(7) : 1;
 }
 
-// Waits until no entry part[b * ncols + col], b < nb, holds kUnsetBits (agent
+// Waits until no entry part[b], b < nb, holds kUnsetBits (agent
 // loads, bounded); false on every lane if a wait gave up.  Contains barriers.
-__device__ __forceinline__ bool wait_column(const double* part, int nb, int ncols, int col,
-                                            int* flag_lds) {
+__device__ __forceinline__ bool wait_column(const double* part, int nb, int* flag_lds) {
   if (threadIdx.x == 0) *flag_lds = 1;
   __syncthreads();
   bool ok = true;
@@ -116,7 +115,7 @@ __device__ __forceinline__ bool wait_column(const double* part, int nb, int ncol
     unsigned polls = 0;
     for (;;) {
       const bool mine =
-          b >= nb || !is_unset(load_agent(part + static_cast<size_t>(b) * ncols + col));
+          b >= nb || !is_unset(load_agent(part + b));
       if (__all(mine)) break;
       if (++polls >= kBarrierPolls) {
         ok = false;
@@ -184,7 +183,7 @@ __global__ void __launch_bounds__(kPfThreads, 3)
 
   // 2. path quantities (basis variables, exercise values, numeraires)
   {
-    const Model m = pf_model(it, 1);
+    const Model m = pf_model(it);
     switch (it.F) {
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
@@ -253,7 +252,7 @@ __global__ void __launch_bounds__(kPfThreads, 3)
 
   // 4. frozen-strategy forward and 5. adjoint backward
   {
-    const Model m = pf_model(it, it.k);
+    const Model m = pf_model(it);
     const CoefTable cf{tab};
     switch (it.F) {
 #define KOO_CASE(F)                                                                            \
@@ -261,23 +260,25 @@ __global__ void __launch_bounds__(kPfThreads, 3)
     for (int vb = t; vb < it.nvb; vb += T) {                                                   \
       __syncthreads();                                                                         \
       if (it.N >= kShortCurve)                                                                 \
-        berm_fwd_block<F, kPfThreads, kWindow<F>, true>(m, it.b, cf, gmem(it.ckpt),            \
+        berm_fwd_block<F, kPfThreads, kWindow<F>, true>(m, it.b, cf, nullptr, gmem(it.ckpt),   \
                                                         gmem(it.lamt), gmem(it.tau),           \
                                                         gmem(it.vout), gmem(it.pfwd), vb);     \
       else                                                                                     \
-        berm_fwd_block<F, kPfThreads, 1, true>(m, it.b, cf, gmem(it.ckpt), gmem(it.lamt),      \
+        berm_fwd_block<F, kPfThreads, 1, true>(m, it.b, cf, nullptr, gmem(it.ckpt),            \
+                                               gmem(it.lamt),                                  \
                                                gmem(it.tau), gmem(it.vout), gmem(it.pfwd),     \
                                                vb);                                            \
     }                                                                                          \
     for (int vb = t; vb < it.nvb; vb += T) {                                                   \
       __syncthreads();                                                                         \
       if (it.N >= kShortCurve)                                                                 \
-        berm_bwd_block<F, kPfThreads, kWindow<F>, true>(m, gmem(it.vols), gmem(it.ckpt),       \
+        berm_bwd_block<F, kPfThreads, kWindow<F>, true>(m, gmem(it.vols), nullptr,             \
+                                                        gmem(it.ckpt),                         \
                                                         gmem(it.lamt), gmem(it.tau),           \
                                                         gmem(it.vout), gmem(it.scratch),       \
                                                         gmem(it.pbwd), vb);                    \
       else                                                                                     \
-        berm_bwd_block<F, kPfThreads, 1, true>(m, gmem(it.vols), gmem(it.ckpt),                \
+        berm_bwd_block<F, kPfThreads, 1, true>(m, gmem(it.vols), nullptr, gmem(it.ckpt),       \
                                                gmem(it.lamt), gmem(it.tau), gmem(it.vout),     \
                                                gmem(it.scratch), gmem(it.pbwd), vb);           \
     }                                                                                          \
@@ -292,13 +293,15 @@ __global__ void __launch_bounds__(kPfThreads, 3)
   // block c mod T (each once all its partials are in)
   {
     const double scale = 1.0 / static_cast<double>(P);
+    const int waves = wave_count(P);
     if (t == 0) {
-      if (!wait_column(gmem(it.pfwd), it.nvb, 1, 0, &flag)) goto fail;
-      finalize_col<true>(gmem(it.pfwd), it.nvb, 1, 0, scale, gmem(it.price));
+      if (!wait_column(gmem(it.pfwd), waves, &flag)) goto fail;
+      finalize_col<true>(gmem(it.pfwd), waves, 1, 0, scale, gmem(it.price));
     }
     for (int c = t; c < 2 * it.N; c += T) {
-      if (!wait_column(gmem(it.pbwd), it.nvb, 2 * it.N, c, &flag)) goto fail;
-      finalize_col<true>(gmem(it.pbwd), it.nvb, 2 * it.N, c, scale, gmem(it.greeks));
+      const double* col = gmem(it.pbwd) + static_cast<size_t>(c) * waves;
+      if (!wait_column(col, waves, &flag)) goto fail;
+      finalize_col<true>(col, waves, 1, 0, scale, gmem(it.greeks) + c);
     }
   }
   if (threadIdx.x == 0) ticks[blockIdx.x] = __builtin_amdgcn_s_memrealtime() - t_start;
@@ -318,8 +321,8 @@ fail:
 __global__ void __launch_bounds__(256) k_portfolio_arm(const PfItem* __restrict__ items) {
   const PfItem& it = items[blockIdx.x];
   const size_t nx = 3 * static_cast<size_t>(kTriMax) * it.team;
-  const size_t nf = it.nvb;
-  const size_t nbw = static_cast<size_t>(it.nvb) * 2 * it.N;
+  const size_t nf = wave_count(it.P);
+  const size_t nbw = nf * 2 * it.N;
   unsigned long long* x = reinterpret_cast<unsigned long long*>(gmem(it.xbuf));
   unsigned long long* pf = reinterpret_cast<unsigned long long*>(gmem(it.pfwd));
   unsigned long long* pb = reinterpret_cast<unsigned long long*>(gmem(it.pbwd));
@@ -329,7 +332,7 @@ __global__ void __launch_bounds__(256) k_portfolio_arm(const PfItem* __restrict_
 }
 
 // Device buffer: the items, the bridge tables, the forward price partials
-// (one column per product, nvb doubles each), the error word.
+// (one column per product, a double per wavefront), the error word.
 constexpr int kPfMaxGrid = 4096;
 
 struct PfLayout {
@@ -352,12 +355,12 @@ int pf_nvb(int paths) { return (paths + kPfThreads - 1) / kPfThreads; }
 
 // Dynamic LDS (bytes) of the phases of a product: generation (S bridge
 // points per lane and the S dimensions' direction numbers), path quantities
-// and forward (the curve and the step table), backward (plus the vega slots),
-// the LS rounds (kPfLsDoubles).
+// and forward (the states and the step table), backward (adjoints and step
+// table), the LS rounds (kPfLsDoubles).
 size_t pf_phase_lds(int N) {
   const size_t gen = sizeof(float) * static_cast<size_t>(N) * kPfThreads + sizeof(uint32_t) * 32 * N;
   size_t m = gen;
-  m = std::max(m, rows_lds(N, kPfThreads, true));
+  m = std::max(m, rows_lds(N, N, kPfThreads, true));
   m = std::max(m, sizeof(double) * static_cast<size_t>(kPfLsDoubles));
   return (m + 15) & ~static_cast<size_t>(15);
 }
@@ -384,7 +387,7 @@ using namespace koo;
 extern "C" size_t bermudan_portfolio_persistent_bytes(int n_products, const int* paths) {
   if (n_products < 1 || !paths) return 0;
   size_t f = 0;
-  for (int i = 0; i < n_products; ++i) f += pf_nvb(paths[i] < 1 ? 1 : paths[i]);
+  for (int i = 0; i < n_products; ++i) f += wave_count(paths[i] < 1 ? 1 : paths[i]);
   return pf_layout(n_products, f).total;
 }
 
@@ -455,7 +458,9 @@ extern "C" int bermudan_portfolio_persistent_prepare(int n_products, const koo_g
     it.P = q.paths;
     it.N = q.rates;
     it.F = q.factors;
-    it.k = q.checkpoint_every;
+    const SweepPlan sweep = sweep_plan(q.rates, q.factors, q.checkpoint_every);
+    it.S1 = sweep.S1;
+    it.L = sweep.L;
     for (int s = 0; s < kMaxRates; ++s) it.ex.e_of_step[s] = -1;
     for (int e = 0; e < q.n_ex; ++e) {
       const int s = l.exercise_steps[e];
@@ -490,7 +495,7 @@ extern "C" int bermudan_portfolio_persistent_prepare(int n_products, const koo_g
     it.price = (g_double*)q.price_out;
     it.greeks = (g_double*)q.greeks_out;
     it.nvb = pf_nvb(q.paths);
-    pf_total += it.nvb;
+    pf_total += wave_count(q.paths);
     lds_main = std::max(lds_main, pf_phase_lds(q.rates));
     max_e = std::max(max_e, q.n_ex);
     cost[i] = work ? work[i] : pf_cost(q, it.ex.last, it.gen);
@@ -505,7 +510,7 @@ extern "C" int bermudan_portfolio_persistent_prepare(int n_products, const koo_g
       per_cu < 1)
     return set_error(KOO_ERR_INVALID, "%s: no block of %zu bytes of LDS can be resident", who, lds);
   // every block must be resident at once; bound the occupancy figure by the
-  // residency measured on gfx950 for 256-lane blocks (LDS per block incl.
+  // residency measured on gfx950 (LDS per block incl.
   // static: <= 40 KiB: 4 per CU, <= 53 120 B: 3, <= 80 KiB: 2), since the
   // query has allowed a block more than fits just below the 3-per-CU limit
   {
@@ -527,7 +532,7 @@ extern "C" int bermudan_portfolio_persistent_prepare(int n_products, const koo_g
     return set_error(KOO_ERR_INVALID, "%s: %d products exceed the %d resident blocks", who,
                      n_products, R);
   // team sizes: proportional to the work, at least 1, at most one block per
-  // 256-path chunk and per LS partial column, summing to at most R
+  // chunk of kPfThreads paths and per LS partial column, summing to at most R
   double tot = 0.0;
   for (double c : cost) tot += c;
   std::vector<int> team(n_products);
@@ -568,7 +573,7 @@ extern "C" int bermudan_portfolio_persistent_prepare(int n_products, const koo_g
     it.team = team[i];
     b0 += team[i];
     it.pfwd = (g_double*)(buf + lay.pfwd) + fo;
-    fo += it.nvb;
+    fo += wave_count(it.P);
     if (it.gen)
       it.tables = (const BridgeTables KOO_GLOBAL*)(buf + lay.tables) + i;
   }
