@@ -98,6 +98,36 @@ def test_fused_sobol_bridge_equals_staged(torch_cuda, S, F, P, off):
     assert torch.allclose(fused, staged, rtol=0, atol=2e-6)
 
 
+@pytest.mark.parametrize("S,F", [(1, 2), (3, 1), (4, 3), (5, 2), (63, 1), (64, 2), (65, 2), (127, 1),
+                                 (128, 2)])
+@pytest.mark.parametrize("P,off", [(1, 0), (63, 0), (64, 63), (65, 62), (129, 1), (20003, 130)])
+def test_fused_sobol_bridge_chunks_and_rows(torch_cuda, S, F, P, off):
+    """Path counts that end inside either chunk of a pair, first points at
+    every place in a group of 64, and step counts around the groups of four
+    dimensions and the two-register split, against the stages; the word behind
+    the last path keeps its value.
+
+    Both sides form a bridge point with three roundings from points at most
+    log2(S) + 1 levels above it (a convex combination, which does not amplify
+    their errors) and difference two of them."""
+    torch = torch_cuda
+    D = S * F
+    dirs = dev(torch, koo.sobol_directions(D))
+    scr = dev(torch, np.random.RandomState(5).randint(0, 2**32, D, dtype=np.uint64).astype(np.uint32))
+    alloc = dev(torch, O.bridge_allocate_diagonal(F, S))
+    normals = torch.empty(D * P, dtype=torch.float32, device="cuda")
+    koo.sobol_scramble_normal_gpu(P, D, off, dirs, scr, D, normals)
+    staged = torch.empty(D * P, dtype=torch.float32, device="cuda")
+    koo.brownian_bridge_gpu(S, alloc, normals, staged, P, F)
+    fused = torch.full((D * P + 64,), 7.0, dtype=torch.float32, device="cuda")
+    koo.sobol_bridge_gpu(P, off, S, F, dirs, scr, D, alloc, fused)
+    assert bool((fused[D * P:] == 7.0).all())
+    w = staged.double().reshape(S, F, P).cumsum(0).abs().max().item()
+    levels = int(np.ceil(np.log2(S))) + 1
+    bound = 2 * 2 * 3 * levels * 2.0**-24 * w  # two sides, two points, three roundings a level
+    assert (fused[:D * P] - staged).abs().max().item() <= bound
+
+
 def test_fused_sobol_bridge_vs_fp64_oracle(torch_cuda):
     torch = torch_cuda
     S, F, P = 40, 5, 8192

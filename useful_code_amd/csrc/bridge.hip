@@ -4,11 +4,11 @@
 //
 // One lane owns one (path, factor) pair and every global load/store is a
 // contiguous 256-byte row of the path-minor layouts ([D][P] in, (S,F,P)
-// out).  For S <= 64 steps the construction order is a compile-time constant
-// and the S bridge points of a lane live in VGPRs; longer bridges keep them
-// in LDS laid out [step][lane] (bank-conflict free).  The construction
-// weights travel in the kernel arguments (scalar loads), so a call allocates
-// nothing.
+// out).  The generator for every step count and the stand-alone bridge for
+// S <= 64 take the construction order as a compile-time constant and hold the S
+// bridge points of a lane in VGPRs; longer stand-alone bridges keep them in LDS
+// laid out [step][lane] (bank-conflict free).  The construction weights travel
+// in the kernel arguments (scalar loads), so a call allocates nothing.
 #include <array>
 #include <cmath>
 #include <mutex>
@@ -34,39 +34,14 @@ __global__ void __launch_bounds__(kBridgeThreads)
               [&](int i) { return in[static_cast<size_t>(idx[i]) * paths + p]; }, out);
 }
 
-// Fused generator, general steps: the bridge variate i of factor f is the
-// normal quantile of Sobol dimension d = alloc(f, i) at Gray index p + off1,
-// scrambled when d < number_scrambled.  Direction numbers of the block's S
-// dimensions sit in LDS behind the path storage.
-__global__ void __launch_bounds__(kBridgeThreads)
-    k_sobol_bridge(const BridgeTables T, int steps, int factors, int paths, uint32_t off1,
-                   const uint32_t* __restrict__ dirs, const uint32_t* __restrict__ scr,
-                   int number_scrambled, const int* __restrict__ alloc, float* __restrict__ out) {
-  extern __shared__ float lds[];
-  uint32_t* v = reinterpret_cast<uint32_t*>(lds + steps * blockDim.x);
-  const int* idx = alloc + blockIdx.y * steps;
-  for (int w = threadIdx.x; w < steps * 32; w += blockDim.x)
-    v[w] = dirs[static_cast<size_t>(idx[w >> 5]) * 32 + (w & 31)];
-  __syncthreads();
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= paths) return;
-  const uint32_t n = static_cast<uint32_t>(p) + off1;
-  bridge_lane(T, steps, factors, paths, p, blockIdx.y, lds,
-              [&](int i) {
-                const int d = idx[i];
-                const uint32_t s = d < number_scrambled ? scr[d] : 0u;
-                return invnorm_u32(sobol_point(v + 32 * i, n) ^ s);
-              },
-              out);
-}
-
 // ---------------------------------------------------------------------------
-// Register-resident bridge for S <= kRegSteps.  The construction order
-// depends on S only, so for a compile-time S every index is a constant and
-// the S bridge points of a lane stay in VGPRs (no LDS path storage, which
-// held occupancy to one or two waves per SIMD).  The stand-alone bridge
-// reads its weights from the kernel arguments (uniform, scalar loads); the
-// fused generator, which loops over chunks, from an LDS copy (LdsWeights).
+// Register-resident bridge (stand-alone for S <= kRegSteps, the generator for
+// every S).  The construction order depends on S only, so for a compile-time S
+// every index is a constant and the S bridge points of a lane stay in VGPRs (no
+// LDS path storage, which held occupancy to one or two waves per SIMD).  The
+// stand-alone bridge reads its weights from the kernel arguments (uniform,
+// scalar loads); the fused generator, which loops over chunks, from an LDS copy
+// (LdsWeights).
 // ---------------------------------------------------------------------------
 constexpr int kRegSteps = 64;
 
@@ -111,7 +86,8 @@ struct LdsWeights {
   }
 };
 
-// V is float (one path) or f32x4 (four paths; the scalar weights broadcast).
+// V is float (one path), f32x2 or f32x4 (two, four paths; the scalar weights
+// broadcast).
 template <int S, int I, class V, class Z, class W>
 __device__ __forceinline__ void bridge_point(V (&w)[S], const W& wt, Z& z) {
   constexpr BridgeOrder<S> M{};
@@ -159,24 +135,6 @@ __device__ __forceinline__ void bridge_points_loaded(V (&w)[S], const BridgeTabl
   (bridge_point_inplace<S, I>(w, T), ...);
 }
 
-// Builds the lane's path from z(i) (bridge variate i, i a constant) and
-// stores its increments to (S,F,P) at path p when `live`.
-template <int S, class Z, class W>
-__device__ __forceinline__ void bridge_store(const W& wt, Z z, int factors, int f, int paths,
-                                             int p, bool live, float* __restrict__ out) {
-  float w[S];
-  bridge_points<S>(w, wt, z, std::make_integer_sequence<int, S>{});
-  // the step index offset by the weights' opaque zero, so the S step
-  // offsets are formed where they are stored rather than hoisted into
-  // scalar registers across the chunk loop
-  float prev = 0.0f;
-#pragma unroll
-  for (int i = 0; i < S; ++i) {
-    if (live) out[(static_cast<size_t>(i + wt.z) * factors + f) * paths + p] = w[i] - prev;
-    prev = w[i];
-  }
-}
-
 template <int S>
 __global__ void __launch_bounds__(kBridgeThreads)
     k_bridge_reg(const BridgeTables T, int factors, int paths, const int* __restrict__ alloc,
@@ -221,24 +179,34 @@ __global__ void __launch_bounds__(kBridgeThreads)
   }
 }
 
-// Fused generator on the register bridge.  Each wavefront walks a contiguous
-// run of 64-path chunks of one factor.  With n = G + l (G a multiple of 64,
-// l < 64) the Gray code splits, gray(n) = gray(G) ^ gray(l), so the
-// scrambled Sobol integer is X(G) ^ T(l) with X(G) = scrambler ^ XOR of the
-// direction numbers over the set bits of gray(G).  A lane's l is the same in
-// every chunk; T(l) sits in LDS.  X(G) lives one dimension per lane: from
-// G = 64m to 64(m+1) gray flips bits 5 and 6 + ctz(m+1), so advancing costs
-// two XORs; a chunk (lanes at n = 64c + off1 + lane) spans G and G + 64, so
-// both are formed and read out by readlane.
+// Fused generator on the register bridge, every step count.  Each wavefront
+// walks a contiguous run of 64-path chunks of one factor, two at a time.  With
+// n = G + l (G a multiple of 64, l < 64) the Gray code splits, gray(n) =
+// gray(G) ^ gray(l), so the scrambled Sobol integer is X(G) ^ T(l) with X(G) =
+// scrambler ^ XOR of the direction numbers over the set bits of gray(G).  A
+// lane's l is the same in every chunk; T(l) sits in LDS.  X(G) is kept one
+// dimension per lane (two registers beyond 64 steps): from G = 64m to 64(m+1)
+// gray flips bits 5 and 6 + ctz(m+1), so advancing costs two XORs.  A chunk
+// (lanes at n = 64c + off1 + lane) spans G and G + 64, two chunks three values:
+// the wavefront writes them to rows of its own in LDS, from which each lane
+// reads those of its group, four dimensions to a read.
+// Bound by the vector instructions, 26 a point, most of them the quantile; 43
+// with one chunk at a time, X(G) read out by readlane and 64-bit store
+// addresses.  2^20 paths: 40 steps x 5 factors 232 -> 175 us, 64 x 32 2.59 ->
+// 1.93 ms (4.4 TB/s of stores).  Step counts above 64 kept the points in LDS
+// and walked the bits of the Gray code for each: 2^17 x 80 x 2 238 -> 43 us.
 template <int S>
 __global__ void __launch_bounds__(kBridgeThreads)
     k_sobol_bridge_reg(const BridgeTables T, int factors, int paths, uint32_t off1,
                        const uint32_t* __restrict__ dirs, const uint32_t* __restrict__ scr,
                        int number_scrambled, const int* __restrict__ alloc,
                        float* __restrict__ out) {
-  __shared__ uint32_t vall[S * 32];  // direction numbers [bridge variate][bit]
-  __shared__ uint32_t tlo[S * 64];   // T(l) [bridge variate][l]
-  __shared__ f32x4 wts[S];           // construction weights {rw, lw, sd, 0}
+  constexpr int R = (S + 63) / 64;  // dimensions per lane in the X(G) bookkeeping
+  constexpr int Q = (S + 3) / 4;    // groups of four dimensions
+  __shared__ uint32_t vall[S * 32];                      // direction numbers [bridge variate][bit]
+  __shared__ u32x4 tlo[Q * 64];                          // T(l) [group][l]
+  __shared__ u32x4 xrows[(kBridgeThreads / 64) * 3 * Q]; // X(G), X(G+64), X(G+128) per wavefront
+  __shared__ f32x4 wts[S];                               // construction weights {rw, lw, sd, 0}
   const int f = blockIdx.y;
   const int* idx = alloc + f * S;
   for (int q = threadIdx.x; q < S * 32; q += blockDim.x)
@@ -252,51 +220,93 @@ __global__ void __launch_bounds__(kBridgeThreads)
 #pragma unroll
     for (int bit = 0; bit < 6; ++bit)
       if ((g >> bit) & 1u) x ^= vv[bit];
-    tlo[q] = x;
+    reinterpret_cast<uint32_t*>(tlo)[(q >> 8) * 256 + l * 4 + ((q >> 6) & 3)] = x;
   }
   __syncthreads();
 
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t waves = static_cast<int64_t>(gridDim.x) * (blockDim.x >> 6);
-  const int64_t wv = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int64_t wv = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave;
   const int64_t chunks = (static_cast<int64_t>(paths) + 63) >> 6;
-  const int c0 = static_cast<int>(wv * chunks / waves);
-  const int c1 = static_cast<int>((wv + 1) * chunks / waves);
+  // scalars: the loop below and its addresses are uniform
+  const int c0 = __builtin_amdgcn_readfirstlane(static_cast<int>(wv * chunks / waves));
+  const int c1 = __builtin_amdgcn_readfirstlane(static_cast<int>((wv + 1) * chunks / waves));
   if (c0 >= c1) return;
 
-  // this lane's dimension for the X(G) bookkeeping
-  const int dl = lane < S ? lane : S - 1;
-  const uint32_t* vd = vall + dl * 32;
   const uint32_t r = off1 & 63u;
-  const bool upper = r + static_cast<uint32_t>(lane) >= 64u;  // lane sits in G + 64
   const uint32_t l = (r + static_cast<uint32_t>(lane)) & 63u;
   uint32_t m = static_cast<uint32_t>(c0) + (off1 >> 6);  // G = 64 m for chunk c0
-  uint32_t xc;
-  {
+  // this lane's dimensions for the X(G) bookkeeping
+  const uint32_t* vd[R];
+  uint32_t x[R], v5[R];
+  uint32_t* xw = reinterpret_cast<uint32_t*>(xrows + wave * 3 * Q) + lane;
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int dl = 64 * k + lane < S ? 64 * k + lane : S - 1;
+    vd[k] = vall + dl * 32;
     const int d = idx[dl];
-    xc = d < number_scrambled ? scr[d] : 0u;
+    x[k] = d < number_scrambled ? scr[d] : 0u;
     const uint32_t G = m << 6, g = G ^ (G >> 1);
     for (int b = 5; b < 32; ++b)
-      if ((g >> b) & 1u) xc ^= vd[b];
+      if ((g >> b) & 1u) x[k] ^= vd[k][b];
+    v5[k] = vd[k][5];
   }
-  const uint32_t v5 = vd[5];
-  for (int c = c0; c < c1; ++c, ++m) {
-    const int t = 6 + __builtin_ctz(m + 1u);
-    const uint32_t xn = xc ^ v5 ^ (t < 32 ? vd[t] : 0u);
-    const int p = c * 64 + lane;
+  auto put = [&](int row) {
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if (64 * k + lane < S) xw[row * 4 * Q + 64 * k] = x[k];
+  };
+  // bits 5 and t of gray, t = 6 + ctz of the next m
+  auto advance = [&] {
+    const int t = 6 + __builtin_ctz(++m);
+#pragma unroll
+    for (int k = 0; k < R; ++k) x[k] ^= v5[k] ^ (t < 32 ? vd[k][t] : 0u);
+  };
+  const u32x4* tl = tlo + l;
+  // the lane's own group of the first chunk; of the second, a row further
+  const u32x4* xl = xrows + wave * 3 * Q + (r + static_cast<uint32_t>(lane) >= 64u ? Q : 0);
+  // the wavefront's paths as a buffer per step: stores past its last path are
+  // dropped (the second chunk of the last pair, lanes past the last path)
+  const int bytes = 4 * min(paths - c0 * 64, (c1 - c0) * 64);
+  float* first = out + static_cast<size_t>(f) * paths + static_cast<size_t>(c0) * 64;
+  for (int c = c0; c < c1; c += 2) {
+    // a wavefront's LDS operations keep their order, and the rows are its own
+    put(0);
+    advance();
+    put(1);
+    advance();
+    put(2);
+    __builtin_amdgcn_wave_barrier();
+    u32x4 t, a, b;
     auto z = [&](int i) {
-      const uint32_t xa = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(xc), i));
-      const uint32_t xb = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(xn), i));
-      return invnorm_u32((upper ? xb : xa) ^ tlo[i * 64 + l]);
+      if (i % 4 == 0) {
+        t = tl[(i >> 2) * 64];
+        a = xl[i >> 2];
+        b = xl[Q + (i >> 2)];
+      }
+      return f32x2{invnorm_u32(t[i & 3] ^ a[i & 3]), invnorm_u32(t[i & 3] ^ b[i & 3])};
     };
-    // every lane computes (the readlanes see whole-wave values); only the
-    // lanes inside the path range store.  The weights come from LDS at an
-    // offset made opaque each chunk (a zero from s_mov), so their reads stay
-    // in the loop.
+    // The weights come from LDS at an offset, and the rows of the steps from a
+    // stride, made opaque each time (a zero from s_mov), so that their reads
+    // and sums stay in the loop.
     int zero;
     asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
-    bridge_store<S>(LdsWeights{wts, zero}, z, factors, f, paths, p, p < paths, out);
-    xc = xn;
+    f32x2 w[S];
+    const LdsWeights wt{wts, zero};
+    bridge_points<S>(w, wt, z, std::make_integer_sequence<int, S>{});
+    const size_t stride = (static_cast<size_t>(factors) + zero) * paths;
+    float* row = first;
+    const int byte = (c - c0) * 256 + lane * 4;
+    f32x2 prev = {0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < S; ++i, row += stride) {
+      const auto rs = __builtin_amdgcn_make_buffer_rsrc(row, 0, bytes, 0x00027000);
+      const f32x2 dz = w[i] - prev;
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz.x), rs, byte, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz.y), rs, byte + 256, 0, 0);
+      prev = w[i];
+    }
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -320,7 +330,7 @@ constexpr auto reg_bridge4_table(std::integer_sequence<int, I...>) {
 }
 const auto kRegBridge = reg_bridge_table(std::make_integer_sequence<int, kRegSteps>{});
 const auto kRegBridge4 = reg_bridge4_table(std::make_integer_sequence<int, kRegSteps4>{});
-const auto kRegGen = reg_gen_table(std::make_integer_sequence<int, kRegSteps>{});
+const auto kRegGen = reg_gen_table(std::make_integer_sequence<int, kBridgeMaxSteps>{});
 
 // ---------------------------------------------------------------------------
 // Power-of-two bridge (the reference's legacy BrownianBridge<D>,
@@ -566,43 +576,34 @@ extern "C" int sobol_bridge_gpu(int paths, unsigned path_offset, int steps, int 
     return set_error(KOO_ERR_INVALID, "sobol_bridge_gpu: null pointer");
   if (static_cast<uint64_t>(path_offset) + 1u + static_cast<uint64_t>(paths) > (1ull << 32))
     return set_error(KOO_ERR_INVALID, "sobol_bridge_gpu: path_offset + paths exceeds 2^32 - 1");
-  if (steps <= kRegSteps) {
-    // One block set that is resident at once (blocks per CU from the
-    // occupancy calculator), split evenly over the factors; each wavefront
-    // then walks its own run of chunks, so there is no tail of late blocks.
-    static std::array<int, kRegSteps> resident{};
-    static std::mutex mu;
-    int per_cu;
-    {
-      std::lock_guard<std::mutex> lock(mu);
-      if (!resident[steps - 1]) {
-        int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &nb, reinterpret_cast<const void*>(kRegGen[steps - 1]), kBridgeThreads, 0) !=
-                hipSuccess ||
-            nb < 1)
-          nb = 1;
-        resident[steps - 1] = nb;
-      }
-      per_cu = resident[steps - 1];
+  // One block set that is resident at once (blocks per CU from the
+  // occupancy calculator), split evenly over the factors; each wavefront
+  // then walks its own run of chunks, so there is no tail of late blocks.
+  static std::array<int, kBridgeMaxSteps> resident{};
+  static std::mutex mu;
+  int per_cu;
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (!resident[steps - 1]) {
+      int nb = 0;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+              &nb, reinterpret_cast<const void*>(kRegGen[steps - 1]), kBridgeThreads, 0) !=
+              hipSuccess ||
+          nb < 1)
+        nb = 1;
+      resident[steps - 1] = nb;
     }
-    const int64_t chunks = (static_cast<int64_t>(paths) + 63) / 64;
-    int64_t per_factor = (static_cast<int64_t>(per_cu) * device_cu_count()) / factors;
-    const int64_t most = (chunks + kBridgeThreads / 64 - 1) / (kBridgeThreads / 64);
-    if (per_factor > most) per_factor = most;
-    if (per_factor < 1) per_factor = 1;
-    hipLaunchKernelGGL(kRegGen[steps - 1], dim3(static_cast<unsigned>(per_factor), factors),
-                       dim3(kBridgeThreads), 0, as_stream(stream), tables_for(steps), factors,
-                       paths, path_offset + 1u, d_directions, scramblers, number_scrambled,
-                       allocation_indices, out);
-    return check_launch("sobol_bridge_gpu");
+    per_cu = resident[steps - 1];
   }
-  const int threads = bridge_threads(steps);
-  const size_t lds = sizeof(float) * steps * threads + sizeof(uint32_t) * 32 * steps;
-  hipLaunchKernelGGL(k_sobol_bridge, dim3((paths + threads - 1) / threads, factors), dim3(threads),
-                     lds, as_stream(stream), tables_for(steps), steps,
-                     factors, paths, path_offset + 1u, d_directions, scramblers,
-                     number_scrambled, allocation_indices, out);
+  const int64_t chunks = (static_cast<int64_t>(paths) + 63) / 64;
+  int64_t per_factor = (static_cast<int64_t>(per_cu) * device_cu_count()) / factors;
+  const int64_t most = (chunks + kBridgeThreads / 64 - 1) / (kBridgeThreads / 64);
+  if (per_factor > most) per_factor = most;
+  if (per_factor < 1) per_factor = 1;
+  hipLaunchKernelGGL(kRegGen[steps - 1], dim3(static_cast<unsigned>(per_factor), factors),
+                     dim3(kBridgeThreads), 0, as_stream(stream), tables_for(steps), factors, paths,
+                     path_offset + 1u, d_directions, scramblers, number_scrambled,
+                     allocation_indices, out);
   return check_launch("sobol_bridge_gpu");
 }
 

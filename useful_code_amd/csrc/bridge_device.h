@@ -79,6 +79,10 @@ constexpr int kBridgeThreads = 256;
 __device__ __forceinline__ float bridge_fma(float a, float b, float c) {
   return __builtin_fmaf(a, b, c);
 }
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ f32x2 bridge_fma(float a, f32x2 b, f32x2 c) {
+  return f32x2{__builtin_fmaf(a, b.x, c.x), __builtin_fmaf(a, b.y, c.y)};
+}
 __device__ __forceinline__ f32x4 bridge_fma(float a, f32x4 b, f32x4 c) {
   return __builtin_elementwise_fma(f32x4{a, a, a, a}, b, c);
 }

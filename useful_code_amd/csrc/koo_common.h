@@ -66,13 +66,13 @@ __device__ __forceinline__ float invnorm_u32(uint32_t x) {
   const float Q2 = 2.0795584360534589311f, Q3 = 1.2499328117341603014f,
               Q4 = 0.23668431621373705623f, Q5 = 0.0120098270559197768f,
               Q6 = 0.00010590620919921025259f;
-  const bool upper = x >= 0x80000000u;
-  const uint32_t t = upper ? (0u - x) : x;
-  const float tf = (t == 0u) ? 0.5f : static_cast<float>(t);
+  // As a signed number x is its own tail with the side as the sign: |x| is x
+  // below 2^31 and 2^32 - x above, and converting rounds both signs alike.
+  const float side = static_cast<float>(static_cast<int>(x));
   // w = t * 2^-31 lies in [2^-32, 1]: always a normal number, so the
   // hardware log2 (v_log_f32) needs none of logf's range handling;
   // z = -ln(w) = -ln2 * log2(w).
-  const float w = tf * 4.656612873077392578125e-10f;
+  const float w = fmaxf(fabsf(side) * 4.656612873077392578125e-10f, 2.3283064365386962890625e-10f);
   const float z = __builtin_amdgcn_logf(w) * -0.693147180559945309417f;
   // Horner with the multiply-adds written out, so every kernel that inlines
   // this rounds alike (the same bits from the staged, fused and persistent
@@ -85,7 +85,8 @@ __device__ __forceinline__ float invnorm_u32(uint32_t x) {
   const float rq = __builtin_amdgcn_rcpf(q);
   const float r0 = n * rq;
   const float r = fmaf(fmaf(-q, r0, n), rq, r0);
-  return upper ? r : -r;
+  // negative below 2^31 (r >= 0)
+  return __uint_as_float(__float_as_uint(r) ^ (~x & 0x80000000u));
 }
 
 // Error-free sum: s + e == a + b exactly (Knuth's TwoSum).

@@ -156,7 +156,7 @@ __global__ void __launch_bounds__(kPfThreads, 3)
 
   // 1. generation: the bridge variates of the block's paths, factor by factor
   // (the direction numbers of the factor's S dimensions in LDS behind the
-  // path storage, as k_sobol_bridge)
+  // path storage)
   if (it.gen) {
     const int S = it.N;
     uint32_t* v = reinterpret_cast<uint32_t*>(lds + S * kPfThreads);
