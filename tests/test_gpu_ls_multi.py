@@ -190,6 +190,22 @@ def test_multi_first_pass_many_exact_zero_net_values(torch_cuda):
     check(got, want, 1)
 
 
+@pytest.mark.parametrize("P", [70, 1023, 1025, 3000])
+@pytest.mark.parametrize("m", [1e-6, 0.5, 0.999])
+def test_multi_first_pass_blocks_chains_and_collinear_variables(torch_cuda, P, m):
+    """One block, a block with one path and several; a growth chain that leaves
+    the range of its quick quotient (1e-6: beyond 1e300), one inside it, and one
+    whose search passes the ladder (0.999); and on one date two proportional
+    variables, whose normal equations take the truncated eigen-solve."""
+    c = f32(M.ls_multi_case(23, E=4, P=P, max_vars=2, last_vars=1))
+    c["bv"][1, 1] = 2.0 * c["bv"][1, 0]
+    sel = M.SELECTOR[:3] + (m,)
+    got = run_gpu(torch_cuda, c, 1, 2, 1, selector=sel)
+    want = O.ls_multi_first_pass(c["bv"], c["ves"], c["cash"], c["ev"], c["num"], 1, 2, 10,
+                                 *sel, normalise=1)
+    check(got, want, 1)
+
+
 def test_multi_first_pass_is_deterministic(torch_cuda):
     c = f32(M.ls_multi_case(7, E=6, P=20000, max_vars=2, last_vars=1))
     a = run_gpu(torch_cuda, c, 1, 3, 1)

@@ -23,15 +23,17 @@
 //                   bits, which order like the values; non-members get a
 //                   sentinel above every key) and FP64 sums of net and net^2.
 //   k_multi_ladder  a histogram of the member keys against the ladder of cuts
-//                   the selector's search can ask for (one pass, LDS bins).
-//   k_multi_select  one block: the selector's band search (grow, shrink,
-//                   bisect on a symmetric band) on the exact ladder counts;
-//                   the cuts and the next depth's member count, or the
-//                   interval of a bisection.
+//                   the selector's search can ask for (one pass, LDS bins);
+//                   then, on the last block, the selector's band search
+//                   (grow, shrink, bisect on a symmetric band) on the exact
+//                   ladder counts: the cuts and the next depth's member
+//                   count, or the interval of a bisection.
 //   k_multi_tree    a histogram of the keys inside the bisection interval
-//                   against every guess of the next ten bisection steps.
-//   k_multi_bisect  one block: the bisection on those counts (two stages of
-//                   tree + bisection cover twenty steps).
+//                   against every guess of the next ten bisection steps;
+//                   then, on the last block, the bisection on those counts
+//                   (two such launches cover twenty steps).
+// Bound by the latency of this chain of small launches (2^17 paths, ten dates,
+// three depths: 30 regressions of six launches), not by bytes or operations.
 // The whole pass computes in FP64 from the FP32 inputs, so the band search
 // takes the same steps as the FP64 gold: counts are exact and the net
 // values agree to rounding.  Depths past the last active one return at once;
@@ -46,7 +48,6 @@ namespace {
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMultiThreads = 1024;  // multi-block kernels (16 wavefronts)
-constexpr int kSearchThreads = 1024;  // single-block search kernels (16 wavefronts)
 constexpr int kMaxDepth = 8;         // regressions per exercise date
 constexpr int kSelectMaxSteps = 1000;
 constexpr unsigned long long kKeySentinel = 0x7FFFFFFFFFFFFFFFull;
@@ -93,16 +94,33 @@ __device__ __forceinline__ size_t norm_at(int e, int R, int d, int which, int ma
   return ((static_cast<size_t>(e) * R + d) * 2 + which) * max_vars;
 }
 
-// Normalised variables of one path at (date q, depth d): (x - mean) / sd,
+// One path's inputs at a date.  The kernels load their lane's first path before
+// the cross-block sums they begin with, so that its latency overlaps them.
+struct PathIn {
+  float bv[kMaxBasisVars];
+  float ev, cash;
+};
+
+__device__ __forceinline__ PathIn load_path(const float* __restrict__ bv,
+                                            const float* __restrict__ ev,
+                                            const float* __restrict__ cash, int q, int max_vars,
+                                            int v, size_t P, int p) {
+  PathIn in;
+#pragma unroll
+  for (int i = 0; i < kMaxBasisVars; ++i)
+    in.bv[i] = i < v ? bv[(static_cast<size_t>(q) * max_vars + i) * P + p] : 0.0f;
+  in.ev = ev ? ev[static_cast<size_t>(q) * P + p] : 0.0f;
+  in.cash = cash ? cash[static_cast<size_t>(q) * P + p] : 0.0f;
+  return in;
+}
+
+// Normalised variables of one path at a date and depth: (x - mean) / sd,
 // FP64 as in the gold (GenerateLSRegressionMatrixSelectivelyNormalisingVariables_gold).
-__device__ __forceinline__ void norm_vars(const float* __restrict__ bv, int q, int max_vars,
-                                          size_t P, int p, int v, const double* m,
+__device__ __forceinline__ void norm_vars(const PathIn& in, int v, const double* m,
                                           const double* sd, double* x) {
 #pragma unroll
   for (int i = 0; i < kMaxBasisVars; ++i)
-    x[i] = i < v ? (static_cast<double>(bv[(static_cast<size_t>(q) * max_vars + i) * P + p]) -
-                    m[i]) / sd[i]
-                 : 0.0;
+    x[i] = i < v ? (static_cast<double>(in.bv[i]) - m[i]) / sd[i] : 0.0;
 }
 
 __device__ __forceinline__ double basis_dot(int v, int k, bool cross, const double* x,
@@ -118,23 +136,19 @@ __device__ __forceinline__ double basis_dot(int v, int k, bool cross, const doub
 // value exceeds the last estimate, else add the date's cash flow.
 // dec = the date's coefficients [R][maxd], norm [R][2][max_vars] and cuts
 // [R] (lower, upper), in LDS.
-__device__ __forceinline__ double decide(const MultiArgs& a, int q, int v, int k,
-                                         const float* __restrict__ bv,
-                                         const float* __restrict__ cash,
-                                         const float* __restrict__ ev, size_t P, int p, double y,
-                                         const double* beta, const double* nrm, const double* lo,
-                                         const double* hi) {
-  const double exv = static_cast<double>(ev[static_cast<size_t>(q) * P + p]);
+__device__ __forceinline__ double decide(const MultiArgs& a, int v, int k, const PathIn& in,
+                                         double y, const double* beta, const double* nrm,
+                                         const double* lo, const double* hi) {
+  const double exv = static_cast<double>(in.ev);
   double est = 0.0, nv = 0.0;
   double x[kMaxBasisVars];
   for (int d = 0; d == 0 || (d < a.R && nv > lo[d - 1] && nv < hi[d - 1]); ++d) {
-    norm_vars(bv, q, a.max_vars, P, p, v, nrm + (2 * d) * a.max_vars,
-              nrm + (2 * d + 1) * a.max_vars, x);
+    norm_vars(in, v, nrm + (2 * d) * a.max_vars, nrm + (2 * d + 1) * a.max_vars, x);
     est = basis_dot(v, k, a.cross != 0, x, beta + d * a.maxd);
     nv = est - exv;
   }
   if (exv > est) return exv;
-  return y + static_cast<double>(cash[static_cast<size_t>(q) * P + p]);
+  return y + static_cast<double>(in.cash);
 }
 
 // Loads date q's decision data into LDS (every thread calls; contains a
@@ -189,6 +203,28 @@ __device__ __forceinline__ void multi_prep_body(const MultiArgs a, int depth, co
   __shared__ double red[16 * 8];
   const size_t P = static_cast<size_t>(a.P);
   unsigned long long cutbits = 0;
+  const bool later = depth == 0 && a.e + 1 < a.E;
+  struct Inputs {
+    PathIn next;  // the later date's, for its decision
+    PathIn here;  // this date's variables, for the sums
+    double y, num0, num1;
+    unsigned long long key;
+  };
+  auto load = [&](int p) {
+    Inputs in;
+    if (later) {
+      in.next = load_path(bv, ev, cash, a.e + 1, a.max_vars, a.vn, P, p);
+      in.y = Y[p];
+      in.num0 = static_cast<double>(num[static_cast<size_t>(a.e) * P + p]);
+      in.num1 = static_cast<double>(num[static_cast<size_t>(a.e + 1) * P + p]);
+    }
+    in.key = depth ? ld_ag(keys + p) : 0ull;
+    if (a.normalise) in.here = load_path(bv, nullptr, nullptr, a.e, a.max_vars, a.v, P, p);
+    return in;
+  };
+  const int p0 = blk * blockDim.x + threadIdx.x;
+  Inputs in;
+  if (p0 < a.P) in = load(p0);
   if (depth == 0) {
     if (blk == 0 && threadIdx.x == 0) {
       st_ag(&state[0].active, 1);
@@ -203,28 +239,27 @@ __device__ __forceinline__ void multi_prep_body(const MultiArgs a, int depth, co
   double sums[2 * kMaxBasisVars];
 #pragma unroll
   for (int i = 0; i < 2 * kMaxBasisVars; ++i) sums[i] = 0.0;
-  for (int p = blk * blockDim.x + threadIdx.x; p < a.P; p += nblk * blockDim.x) {
+  for (int p = p0; p < a.P; p += nblk * blockDim.x) {
+    if (p != p0) in = load(p);
     bool member;
     if (depth == 0) {
       double y = 0.0;
-      if (a.e + 1 < a.E) {
-        y = decide(a, a.e + 1, a.vn, a.kn, bv, cash, ev, P, p, Y[p], beta, nrm, lo, hi);
+      if (later) {
+        y = decide(a, a.vn, a.kn, in.next, in.y, beta, nrm, lo, hi);
         // updateDeflationOfContinuationValues_gold (gold/LS_regression.cpp:98-115)
-        y *= static_cast<double>(num[static_cast<size_t>(a.e) * P + p]) /
-             static_cast<double>(num[static_cast<size_t>(a.e + 1) * P + p]);
+        y *= in.num0 / in.num1;
       }
       Y[p] = y;
       member = true;
     } else {
-      member = ld_ag(keys + p) <= cutbits;
+      member = in.key <= cutbits;
     }
     mem[p] = member ? 1 : 0;
     if (a.normalise && member) {
 #pragma unroll
       for (int i = 0; i < kMaxBasisVars; ++i)
         if (i < a.v) {
-          const double x =
-              static_cast<double>(bv[(static_cast<size_t>(a.e) * a.max_vars + i) * P + p]);
+          const double x = static_cast<double>(in.here.bv[i]);
           sums[2 * i] += x;
           sums[2 * i + 1] += x * x;
         }
@@ -289,6 +324,23 @@ __device__ __forceinline__ void multi_gram_body(const MultiArgs a, int depth, co
   __shared__ double msd[2 * kMaxBasisVars];
   if (!ld_ag(&state[depth].active)) return;
   const double n_pre = static_cast<double>(ld_ag(&state[depth].n_pre));
+  const size_t P = static_cast<size_t>(a.P);
+  struct Inputs {
+    PathIn in;
+    double y;
+    bool member;
+  };
+  auto load = [&](int p) {
+    Inputs r;
+    r.member = p < a.P && mem[p];
+    if (r.member) {
+      r.in = load_path(bv, nullptr, cash, a.e, a.max_vars, a.v, P, p);
+      r.y = Y[p];
+    }
+    return r;
+  };
+  const int p0 = blk * blockDim.x + threadIdx.x;
+  Inputs r = load(p0);
   if (a.normalise && a.v > 0) reduce_partials<true>(stats_part, nblk, 2 * a.v, sums);
   if (threadIdx.x < kMaxBasisVars) {
     const int i = threadIdx.x;
@@ -311,7 +363,6 @@ __device__ __forceinline__ void multi_gram_body(const MultiArgs a, int depth, co
   __syncthreads();
   constexpr int kPathsPerOp = 4 * GROUPS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const size_t P = static_cast<size_t>(a.P);
   const bool cross = a.cross != 0;
   const int n = a.k + 1;
   const int j = GROUPS == 2 ? (lane & 7) : (lane & 15);
@@ -319,12 +370,12 @@ __device__ __forceinline__ void multi_gram_body(const MultiArgs a, int depth, co
   doublex4 acc = {0.0, 0.0, 0.0, 0.0};
   const int stride = nblk * nw * 64;
   for (int base = (blk * nw + wave) * 64; base < a.P; base += stride) {
-    const int p = base + lane;
+    if (base + lane != p0) r = load(base + lane);
     double x[kMaxBasisVars] = {0.0, 0.0, 0.0, 0.0};
     double t = 0.0, w = 0.0;
-    if (p < a.P && mem[p]) {
-      norm_vars(bv, a.e, a.max_vars, P, p, a.v, msd, msd + kMaxBasisVars, x);
-      t = static_cast<double>(cash[static_cast<size_t>(a.e) * P + p]) + Y[p];
+    if (r.member) {
+      norm_vars(r.in, a.v, msd, msd + kMaxBasisVars, x);
+      t = static_cast<double>(r.in.cash) + r.y;
       w = 1.0;
     }
     // 64 paths of this wave -> 64 / (4 GROUPS) MFMAs; lane l takes row j of path `sub`.
@@ -363,7 +414,7 @@ __global__ void __launch_bounds__(kMultiThreads)
 // smallest eigenvalue against an upper bound of the largest -- no eigenvalue
 // is below tol times the largest, the truncated solve keeps every direction
 // and equals the Cholesky solution.  Otherwise the truncated Jacobi solve.
-// Single lane; A, V are 16 x 16 LDS scratch, b and z 16.
+// A, V are 16 x 16 LDS scratch, b and z 16.
 // The Cholesky branch of solve_multi with the factor in registers (K known
 // at compile time): the same operations in the same order (divisions by the
 // pivots, not reciprocals), so the same bits.  Returns false where
@@ -423,6 +474,69 @@ __device__ bool cholesky_multi_reg(const double* G, int ld, double inv, double* 
   return true;
 }
 
+// jacobi_truncated (ls_common.h) on one wavefront: the same rotations in the
+// same order.  Every lane forms a rotation's angle; the rows of A (lanes 0-15)
+// and of V (lanes 16-31) take the column rotation side by side, then the columns of
+// A the row rotation, so each element goes through the same operations and
+// keeps its bits.  k = 6 with two collinear variables: the solve 145 -> 45 us.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ void jacobi_truncated_wave(int k, double* A, double* V, const double* b, double tol,
+                                      double* x) {
+  const int lane = threadIdx.x & 63, r = lane & 15;
+  const bool rows = lane < 32 && r < k, cols = lane < 16 && r < k;
+  double* M = (lane & 16) ? V : A;
+  if (cols)
+    for (int j = 0; j < k; ++j) V[r * 16 + j] = r == j ? 1.0 : 0.0;
+  wave_lds_fence();
+  for (int sweep = 0; sweep < 100; ++sweep) {
+    double off = 0.0, tot = 0.0;
+    for (int i = 0; i < k; ++i)
+      for (int j = 0; j < k; ++j) {
+        const double q = A[i * 16 + j] * A[i * 16 + j];
+        tot += q;
+        if (i != j) off += q;
+      }
+    if (off <= 1e-30 * tot) break;
+    for (int p = 0; p < k - 1; ++p)
+      for (int q = p + 1; q < k; ++q) {
+        const double apq = A[p * 16 + q];
+        if (apq == 0.0) continue;
+        const double tau = (A[q * 16 + q] - A[p * 16 + p]) / (2.0 * apq);
+        const double t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
+        const double c = 1.0 / sqrt(1.0 + t * t), s = t * c;
+        if (rows) {
+          const double mp = M[r * 16 + p], mq = M[r * 16 + q];
+          M[r * 16 + p] = c * mp - s * mq;
+          M[r * 16 + q] = s * mp + c * mq;
+        }
+        wave_lds_fence();
+        if (cols) {
+          const double mp = A[p * 16 + r], mq = A[q * 16 + r];
+          A[p * 16 + r] = c * mp - s * mq;
+          A[q * 16 + r] = s * mp + c * mq;
+        }
+        wave_lds_fence();
+      }
+  }
+  double lmax = 0.0;
+  for (int i = 0; i < k; ++i) lmax = fmax(lmax, fabs(A[i * 16 + i]));
+  double xr = 0.0;
+  for (int i = 0; i < k; ++i) {
+    const double l = A[i * 16 + i];
+    if (!(lmax > 0.0) || fabs(l) < tol * lmax) continue;
+    double e = 0.0;
+    for (int q = 0; q < k; ++q) e += V[q * 16 + i] * b[q];
+    e /= l;
+    if (cols) xr += e * V[r * 16 + i];
+  }
+  if (cols) x[r] = xr;
+}
+
+// Whole wavefront; every lane runs the Cholesky branches (the same values).
 __device__ void solve_multi(const double* G, int k, double n, double* beta, double* A, double* V,
                             double* b, double* z) {
   const int ld = k + 1;
@@ -443,8 +557,9 @@ __device__ void solve_multi(const double* G, int k, double n, double* beta, doub
     for (int j = 0; j < k; ++j) A[i * 16 + j] = G[i * ld + j] * inv;
     b[i] = G[i * ld + k] * inv;
   }
+  wave_lds_fence();
   if (reg) {
-    jacobi_truncated(k, A, V, b, kSvdTolerance, beta);
+    jacobi_truncated_wave(k, A, V, b, kSvdTolerance, beta);
     return;
   }
   // Cholesky into V (lower triangle)
@@ -491,7 +606,7 @@ __device__ void solve_multi(const double* G, int k, double n, double* beta, doub
       return;
     }
   }
-  jacobi_truncated(k, A, V, b, kSvdTolerance, beta);
+  jacobi_truncated_wave(k, A, V, b, kSvdTolerance, beta);
 }
 
 __device__ __forceinline__ void multi_net_body(const MultiArgs a, int depth, const float* __restrict__ bv,
@@ -510,21 +625,23 @@ __device__ __forceinline__ void multi_net_body(const MultiArgs a, int depth, con
   // the lane's first path's inputs are loaded before the Gram sums and the
   // solve, so their latency overlaps them
   const int p0 = blk * blockDim.x + threadIdx.x;
-  unsigned char m0 = 0;
-  float raw0[kMaxBasisVars], ev0 = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kMaxBasisVars; ++i) raw0[i] = 0.0f;
-  if (p0 < a.P) {
-    m0 = mem[p0];
-#pragma unroll
-    for (int i = 0; i < kMaxBasisVars; ++i)
-      if (i < a.v) raw0[i] = bv[(static_cast<size_t>(a.e) * a.max_vars + i) * P + p0];
-    ev0 = ev[static_cast<size_t>(a.e) * P + p0];
-  }
+  struct Inputs {
+    PathIn in;
+    bool member;
+  };
+  auto load = [&](int p) {
+    Inputs r;
+    r.member = mem[p] != 0;
+    r.in = load_path(bv, ev, nullptr, a.e, a.max_vars, a.v, P, p);
+    return r;
+  };
+  Inputs r;
+  if (p0 < a.P) r = load(p0);
   reduce_partials<true>(gram_part, nblk, n * n, gram);
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 64) {
     solve_multi(gram, a.k, static_cast<double>(ld_ag(&state[depth].n_pre)), beta, A, V, rhs, tmp);
-    if (blk == 0)
+    wave_lds_fence();
+    if (blk == 0 && threadIdx.x == 0)
       for (int i = 0; i < a.maxd; ++i)
         st_ag(coeffs + (static_cast<size_t>(a.e) * a.R + depth) * a.maxd + i,
               i < a.k ? beta[i] : 0.0);
@@ -540,18 +657,12 @@ __device__ __forceinline__ void multi_net_body(const MultiArgs a, int depth, con
   double s[2] = {0.0, 0.0};
   for (int p = p0; p < a.P; p += nblk * blockDim.x) {
     unsigned long long key = kKeySentinel;
-    const bool first = p == p0;
-    if (first ? m0 != 0 : mem[p] != 0) {
+    if (p != p0) r = load(p);
+    if (r.member) {
       double x[kMaxBasisVars];
-      if (first) {
-#pragma unroll
-        for (int i = 0; i < kMaxBasisVars; ++i)
-          x[i] = i < a.v ? (static_cast<double>(raw0[i]) - msd[i]) / msd[kMaxBasisVars + i] : 0.0;
-      } else {
-        norm_vars(bv, a.e, a.max_vars, P, p, a.v, msd, msd + kMaxBasisVars, x);
-      }
-      const double net = basis_dot(a.v, a.k, a.cross != 0, x, beta) -
-                         static_cast<double>(first ? ev0 : ev[static_cast<size_t>(a.e) * P + p]);
+      norm_vars(r.in, a.v, msd, msd + kMaxBasisVars, x);
+      const double net =
+          basis_dot(a.v, a.k, a.cross != 0, x, beta) - static_cast<double>(r.in.ev);
       s[0] += net;
       s[1] += net * net;
       key = static_cast<unsigned long long>(__double_as_longlong(fabs(net)));
@@ -579,23 +690,21 @@ __global__ void __launch_bounds__(kMultiThreads)
 // G_j = G_0 / m^j, the shrink steps G_0 m^(i+1) and the first shrink step
 // G_j m after j growth steps -- and then bisects between two of them.
 // k_multi_ladder histograms every member key against the whole ladder (one
-// pass), k_multi_select replays the search on those exact counts, and when
+// pass) and its last block replays the search on those exact counts, and when
 // it ends in a bisection, k_multi_tree histograms the keys against every
-// guess of the first bisection steps and k_multi_bisect replays those.  A search that runs
-// past the ladder (kLadder steps either way) continues in k_multi_select with
+// guess of the first bisection steps and its last block replays those.  A search
+// that runs past the ladder (kLadder steps either way) continues there with
 // block-wide counts over all keys, so every count the gold would take is
 // taken exactly.
 // ---------------------------------------------------------------------------
 constexpr int kLadder = 64;                   // growth / shrink steps held
-constexpr int kLadderSlots = 256;             // >= 3 kLadder - 1
-static_assert(3 * kLadder - 1 <= kLadderSlots, "ladder slots");
-// ladder_build uses lanes 0 and 64; block sums use one LDS slot per wavefront
-static_assert(kSearchThreads >= 256 && kMultiThreads >= 256,
-              "ladder needs 128 lanes, the selection's sums 4 wavefronts");
-static_assert(kSearchThreads <= 1024 && kMultiThreads <= 1024, "16 wavefront slots");
+constexpr int kLadderBins = 192;              // >= 3 kLadder - 1, whole wavefronts
+static_assert(3 * kLadder - 1 <= kLadderBins && 4 * kLadderBins <= kMultiThreads - 64 &&
+                  kMultiThreads <= 1024,
+              "four groups of bins and a wavefront beside them; 16 wavefront slots");
 constexpr unsigned long long kEmpty = ~0ull;  // a cut that counts no path
 
-// Bisection hand-over from k_multi_select to k_multi_tree / k_multi_bisect.
+// Bisection hand-over from k_multi_ladder to k_multi_tree and on to the next stage.
 struct SelectState {
   double low, high;
   long long count_low;
@@ -673,16 +782,6 @@ __device__ __forceinline__ double net_sd(const double* sums, long long n_pre) {
   return sqrt(sums[1] / np - mean * mean);
 }
 
-// Number of ladder values ladder_build makes for n_pre members: it depends
-// on the selector and the member count only, not on the net values.
-__device__ __forceinline__ int ladder_count(const MultiArgs& a, long long n_pre) {
-  const double np = static_cast<double>(n_pre);
-  const long long lowerT = static_cast<long long>(np * a.lower_frac);
-  const long long upperT = static_cast<long long>(np * a.upper_frac);
-  if (a.selector == 1 || (n_pre > lowerT && n_pre < upperT)) return 1;
-  return 3 * kLadder - 1;
-}
-
 // The ladder of raw cut values v[0..n) and their key bounds tb (a member
 // counts at cut t when key <= tb[t]; kEmpty counts none).  Layout: fraction
 // selector with the pre-selected count inside the window: v[0] = 10000;
@@ -691,17 +790,36 @@ __device__ __forceinline__ int ladder_count(const MultiArgs& a, long long n_pre)
 // 1] = G_j m (1 <= j < L); standard-deviation selector: v[0] = sd_guess sd
 // with the open bound.  Whole block; returns n.
 // The growth steps v[0..L) (G_0 divided by m again and again) and the shrink
-// steps v[L..2L) (G_0 m multiplied by m again and again), as ladder_build
-// forms them.  One lane; sums in LDS.
-__device__ void ladder_chains(const MultiArgs& a, long long n_pre, const double* sums, double* v) {
+// steps v[L..2L) (G_0 m multiplied by m again and again), as the gold forms
+// them, each a serial chain.  One lane each; sums in LDS.
+// A quotient g / m with y = 1 / m correctly rounded: q = g y, once corrected by
+// its remainder, is within one unit in the last place of g / m, and then a
+// second correction (exact remainder, same y) rounds correctly (P. Markstein,
+// "Computation of elementary functions on the IBM RISC System/6000 processor",
+// 1990), where nothing under- or overflows: five dependent operations in place
+// of a division's range handling (the chain 4.6 -> 1.3 us).  A chain that leaves
+// the safe range is formed again with divisions.
+__device__ __forceinline__ void ladder_growth(const MultiArgs& a, double sd, double* v) {
   const int L = kLadder;
-  const double sd = net_sd(sums, n_pre);
-  double g = sd * a.sd_guess;
+  const double m = a.multiplier, y = 1.0 / m, g0 = sd * a.sd_guess;
+  double g = g0;
   v[0] = g;
   for (int j = 1; j < L; ++j) {
-    g /= a.multiplier;
+    double q = g * y;
+    q = fma(fma(-q, m, g), y, q);
+    g = fma(fma(-q, m, g), y, q);
     v[j] = g;
   }
+  if (g0 > 1e-250 && g < 1e250 && m > 1e-250) return;
+  g = g0;
+  for (int j = 1; j < L; ++j) {
+    g /= m;
+    v[j] = g;
+  }
+}
+
+__device__ __forceinline__ void ladder_shrink(const MultiArgs& a, double sd, double* v) {
+  const int L = kLadder;
   double lo = (sd * a.sd_guess) * a.multiplier;
   v[L] = lo;
   for (int i = 1; i < L; ++i) {
@@ -710,10 +828,8 @@ __device__ void ladder_chains(const MultiArgs& a, long long n_pre, const double*
   }
 }
 
-// chains_done: ladder_chains has already filled v[0..2L) (the full ladder
-// case only).
 __device__ int ladder_build(const MultiArgs& a, long long n_pre, const double* sums, double* v,
-                            unsigned long long* tb, bool chains_done = false) {
+                            unsigned long long* tb) {
   const int t = threadIdx.x, L = kLadder;
   const double sd = net_sd(sums, n_pre);
   const double np = static_cast<double>(n_pre);
@@ -735,22 +851,8 @@ __device__ int ladder_build(const MultiArgs& a, long long n_pre, const double* s
     }
   } else {
     n = 3 * L - 1;
-    if (chains_done) {
-    } else if (t == 0) {
-      double g = sd * a.sd_guess;
-      v[0] = g;
-      for (int j = 1; j < L; ++j) {
-        g /= a.multiplier;
-        v[j] = g;
-      }
-    } else if (t == 64) {  // the kernels run at least 128 lanes
-      double lo = (sd * a.sd_guess) * a.multiplier;
-      v[L] = lo;
-      for (int i = 1; i < L; ++i) {
-        lo *= a.multiplier;
-        v[L + i] = lo;
-      }
-    }
+    if (t == 0) ladder_growth(a, sd, v);
+    if (t == 64) ladder_shrink(a, sd, v);  // the kernels run at least 128 lanes
     __syncthreads();
     for (int j = 1 + t; j < L; j += blockDim.x) v[2 * L + j - 1] = v[j] * a.multiplier;
     __syncthreads();
@@ -760,17 +862,35 @@ __device__ int ladder_build(const MultiArgs& a, long long n_pre, const double* s
   return n;
 }
 
+// The ladder of the current regression and the counts on it, in LDS: built by
+// multi_ladder_body, read by multi_select_body in the same block.
+struct LadderLds {
+  double sums[2];
+  double v[kLadderBins];
+  unsigned long long tb[kLadderBins], ts[kLadderBins];
+  int rank[kLadderBins];
+  int part[4][kLadderBins];  // of the ranks
+  int n;
+};
+
 // Stable ranks of the key bounds: ts (ascending) and rank[t] = position of
-// tb[t] in ts.  Whole block.
-__device__ __forceinline__ void ladder_sort(int n, const unsigned long long* tb,
-                                            unsigned long long* ts, int* rank) {
-  for (int t = threadIdx.x; t < n; t += blockDim.x) {
-    const unsigned long long x = tb[t];
+// tb[t] in ts.  Whole block: four groups of lanes each compare with a quarter
+// of the bounds (with one group the comparisons took 2.2 us).
+__device__ __forceinline__ void ladder_sort(LadderLds& s) {
+  const int n = s.n, g = threadIdx.x / kLadderBins, t = threadIdx.x - g * kLadderBins;
+  if (g < 4 && t < n) {
+    const unsigned long long x = s.tb[t];
+    const int q = (n + 3) / 4, u1 = min(n, (g + 1) * q);
     int r = 0;
 #pragma unroll 8
-    for (int u = 0; u < n; ++u) r += (tb[u] < x || (tb[u] == x && u < t)) ? 1 : 0;
-    ts[r] = x;
-    if (rank) rank[t] = r;
+    for (int u = g * q; u < u1; ++u) r += (s.tb[u] < x || (s.tb[u] == x && u < t)) ? 1 : 0;
+    s.part[g][t] = r;
+  }
+  __syncthreads();
+  if (g == 0 && t < n) {
+    const int r = s.part[0][t] + s.part[1][t] + s.part[2][t] + s.part[3][t];
+    s.ts[r] = s.tb[t];
+    s.rank[t] = r;
   }
   __syncthreads();
 }
@@ -789,33 +909,47 @@ __device__ __forceinline__ int ladder_bin(const unsigned long long* ts, int n,
   return lo;
 }
 
-// Histogram of the member keys over the ladder: hist_part[bin * nb + block]
-// (FP64, exact) counts the members whose first bound >= key is bin.
+// Adds a block's LDS counts to the pass's counts in memory (zero between
+// searches).  A row of counts per block, summed by the block that searches,
+// took 3 us (192 bins) and 7 us (1024) more at 128 blocks.
+__device__ __forceinline__ void add_counts(const int* lds, int n, int* __restrict__ counts) {
+  for (int t = threadIdx.x; t < n; t += blockDim.x)
+    if (lds[t])
+      __hip_atomic_fetch_add(counts + t, lds[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Reads count t and sets it back to zero.
+__device__ __forceinline__ int take_count(int* __restrict__ counts, int t) {
+  const int c = ld_ag(counts + t);
+  st_ag(counts + t, 0);
+  return c;
+}
+
+// Histogram of the member keys over the ladder: hist[bin] counts the members
+// whose first bound >= key is bin.
 __device__ __forceinline__ void multi_ladder_body(const MultiArgs a, int depth, const unsigned long long* __restrict__ keys,
                    const double* __restrict__ net_part, int nb_net,
-                   const DepthState* __restrict__ state, double* __restrict__ hist_part,
-                   KeyExtent* __restrict__ ext_part, int blk, int nblk) {
-  __shared__ double sums[2];
-  __shared__ double v[kLadderSlots];
-  __shared__ unsigned long long tb[kLadderSlots], ts[kLadderSlots];
-  __shared__ int hist[kLadderSlots];
+                   const DepthState* __restrict__ state, int* __restrict__ counts,
+                   KeyExtent* __restrict__ ext_part, LadderLds& s, int blk, int nblk) {
+  __shared__ int hist[kLadderBins];
   __shared__ KeyExtent wext[16];
   if (!ld_ag(&state[depth].active)) return;
   // the lane's first key is loaded before the ladder is built, so its
   // latency overlaps the net-value sums
   const int p0 = blk * blockDim.x + threadIdx.x;
   const unsigned long long key0 = p0 < a.P ? ld_ag(keys + p0) : kKeySentinel;
-  reduce_partials<true>(net_part, nb_net, 2, sums);
-  const int n = ladder_build(a, ld_ag(&state[depth].n_pre), sums, v, tb);
-  ladder_sort(n, tb, ts, nullptr);
+  reduce_partials<true>(net_part, nb_net, 2, s.sums);
+  const int n = ladder_build(a, ld_ag(&state[depth].n_pre), s.sums, s.v, s.tb);
+  if (threadIdx.x == 0) s.n = n;
   for (int t = threadIdx.x; t < n; t += blockDim.x) hist[t] = 0;
   __syncthreads();
+  ladder_sort(s);
   unsigned long long mn = ~0ull, mx = 0ull;
   long long nz = 0, nv = 0;
   for (int p = p0; p < a.P; p += nblk * blockDim.x) {
     const unsigned long long key = p == p0 ? key0 : ld_ag(keys + p);
     if (key != kKeySentinel) {
-      const int b = ladder_bin(ts, n, key);
+      const int b = ladder_bin(s.ts, n, key);
       if (b < n) atomicAdd(&hist[b], 1);
       if (key <= kInfKey) {  // not NaN
         ++nv;
@@ -837,9 +971,8 @@ __device__ __forceinline__ void multi_ladder_body(const MultiArgs a, int depth, 
   }
   if ((threadIdx.x & 63) == 0) wext[threadIdx.x >> 6] = KeyExtent{mn, mx, nz, nv};
   __syncthreads();
-  for (int t = threadIdx.x; t < n; t += blockDim.x)
-    st_ag(hist_part + static_cast<size_t>(t) * nblk + blk, static_cast<double>(hist[t]));
-  if (threadIdx.x == 0) {
+  add_counts(hist, n, counts);
+  if (threadIdx.x == blockDim.x - 1) {
     KeyExtent e = wext[0];
     for (int w = 1; w < static_cast<int>(blockDim.x >> 6); ++w) {
       e.minpos = wext[w].minpos < e.minpos ? wext[w].minpos : e.minpos;
@@ -853,15 +986,6 @@ __device__ __forceinline__ void multi_ladder_body(const MultiArgs a, int depth, 
     st_ag(&ext_part[blk].nvalid, e.nvalid);
   }
 }
-
-__global__ void __launch_bounds__(kMultiThreads)
-    k_multi_ladder(const MultiArgs a, int depth, const unsigned long long* __restrict__ keys,
-                   const double* __restrict__ net_part, int nb_net,
-                   const DepthState* __restrict__ state, double* __restrict__ hist_part,
-                   KeyExtent* __restrict__ ext_part) {
-  multi_ladder_body(a, depth, keys, net_part, nb_net, state, hist_part, ext_part, blockIdx.x, gridDim.x);
-}
-
 
 // Count of member keys <= key_of(g) for g >= 0 from the extents when they
 // decide it, else -1.
@@ -877,9 +1001,16 @@ __device__ __forceinline__ long long extent_count(const KeyExtent& x, double g) 
 __device__ long long block_count(const unsigned long long* __restrict__ keys, long long n,
                                  unsigned long long gb, long long* red /* [16] */) {
   long long c = 0;
-  for (long long i = threadIdx.x; i < n; i += blockDim.x) {
-    const unsigned long long k = ld_ag(keys + i);
-    c += (k != kKeySentinel && k <= gb) ? 1 : 0;
+  constexpr int kInFlight = 16;
+  for (long long i0 = threadIdx.x; i0 < n; i0 += static_cast<long long>(kInFlight) * blockDim.x) {
+    unsigned long long k[kInFlight];
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) {
+      const long long i = i0 + static_cast<long long>(u) * blockDim.x;
+      k[u] = i < n ? ld_ag(keys + i) : kKeySentinel;
+    }
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) c += (k[u] != kKeySentinel && k[u] <= gb) ? 1 : 0;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
@@ -912,50 +1043,65 @@ __device__ __forceinline__ void finish_select(const MultiArgs& a, int depth, dou
   }
 }
 
+// x times f (or divided by f) n times over, on one wavefront (sixteen of them
+// at it took 15 us for 900 steps); every lane returns it.  Whole block.
+template <bool Divide>
+__device__ double repeat_scale(double x, double f, int n) {
+  __shared__ double out;
+  if (threadIdx.x < 64) {
+#pragma unroll 8
+    for (int i = 0; i < n; ++i) x = Divide ? x / f : x * f;
+    if (threadIdx.x == 0) out = x;
+  }
+  __syncthreads();
+  x = out;
+  __syncthreads();
+  return x;
+}
+
 // The band search on the ladder counts (RegressionSelector_gold_Fraction::Select,
 // Regression_Selector_concrete_gold.cpp:13-183; RegressionSelectorStandardDeviations,
 // RegressionSelectorConcrete.cu:19-90).  One block; every thread runs the same
 // search on LDS values so the block-wide fallback counts stay uniform.
 __device__ __forceinline__ void multi_select_body(const MultiArgs a, int depth, const unsigned long long* __restrict__ keys,
-                   const double* __restrict__ net_part, int nb,
-                   const double* __restrict__ hist_part, const KeyExtent* __restrict__ ext_part,
+                   int* __restrict__ counts, const KeyExtent* __restrict__ ext_part,
                    int nh, DepthState* __restrict__ state, SelectState* __restrict__ sel,
-                   double* __restrict__ lower, double* __restrict__ upper, int blk, int nblk) {
-  __shared__ double sums[2];
-  __shared__ double v[kLadderSlots], cnt[kLadderSlots];
-  __shared__ unsigned long long tb[kLadderSlots], ts[kLadderSlots];
-  __shared__ int rank[kLadderSlots];
+                   double* __restrict__ lower, double* __restrict__ upper, LadderLds& s) {
+  __shared__ double cnt[kLadderBins];
   __shared__ long long red[16];
   __shared__ KeyExtent ext;
-  if (!ld_ag(&state[depth].active)) {
-    if (threadIdx.x == 0) {
-      st_ag(&sel->bisect, 0);
-      if (depth + 1 < a.R) st_ag(&state[depth + 1].active, 0);
-    }
-    return;
-  }
   const long long n_pre = ld_ag(&state[depth].n_pre);
-  // the three cross-block sums at once, on disjoint wavefronts: the ladder's
-  // bin counts (cnt[k]: members in bin k), the net-value sums, the extents
-  // (the net-value wavefront then builds the ladder's two serial chains
-  // while the bin counts are still being summed)
-  const int nw = blockDim.x >> 6;
-  const int nlad = ladder_count(a, n_pre);
-  reduce_partials_waves<true>(hist_part, nh, nlad, cnt, 0, nw - 2);
-  reduce_partials_waves<true>(net_part, nb, 2, sums, nw - 2, 1);
-  if (nlad > 1 && threadIdx.x == (nw - 2) * 64) ladder_chains(a, n_pre, sums, v);
-  reduce_extents_wave(ext_part, nh, &ext, nw - 1);
+  const int n = s.n;
+  const double* v = s.v;
+  const unsigned long long* tb = s.tb;
+  const int* rank = s.rank;
+  if (threadIdx.x < n) cnt[threadIdx.x] = static_cast<double>(take_count(counts, threadIdx.x));
+  reduce_extents_wave(ext_part, nh, &ext, (blockDim.x >> 6) - 1);
   __syncthreads();
-  const int n = ladder_build(a, n_pre, sums, v, tb, nlad > 1);
-  ladder_sort(n, tb, ts, rank);
-  if (threadIdx.x == 0) {
-    // running count in a register, so the bins' loads are independent of
-    // the additions (the counts are integers, exact in FP64)
-    double run = cnt[0];
-#pragma unroll 8
-    for (int k = 1; k < n; ++k) {
-      run += cnt[k];
-      cnt[k] = run;
+  if (threadIdx.x < 64) {
+    // running count: each lane sums a run of kRun bins, the sums are scanned
+    // across the wavefront (the counts are integers, exact in FP64)
+    constexpr int kRun = (kLadderBins + 63) / 64;
+    const int lane = threadIdx.x;
+    double c[kRun], sum = 0.0;
+#pragma unroll
+    for (int q = 0; q < kRun; ++q) {
+      const int t = lane * kRun + q;
+      c[q] = t < n ? cnt[t] : 0.0;
+      sum += c[q];
+    }
+    double incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    double run = incl - sum;
+#pragma unroll
+    for (int q = 0; q < kRun; ++q) {
+      const int t = lane * kRun + q;
+      run += c[q];
+      if (t < n) cnt[t] = run;
     }
   }
   __syncthreads();
@@ -1006,7 +1152,7 @@ __device__ __forceinline__ void multi_select_body(const MultiArgs a, int depth, 
         if (guess >= 0.0 && key_of(guess) >= ext.maxval && ext.nvalid < lowerT) {
           // every later guess is larger, so the count stays at nvalid: the
           // gold's loop runs out its steps (the same divisions, no counts)
-          while (it++ < kSelectMaxSteps) guess /= m;
+          if (it < kSelectMaxSteps) guess = repeat_scale<true>(guess, m, kSelectMaxSteps - it);
           count = ext.nvalid;
           break;
         }
@@ -1048,7 +1194,7 @@ __device__ __forceinline__ void multi_select_body(const MultiArgs a, int depth, 
           if (low >= 0.0 && key_of(low) < ext.minpos && ext.nzero > upperT) {
             // every later cut is smaller, so the count stays at the zero
             // count: the gold's loop runs out its steps (same products)
-            while (it++ < kSelectMaxSteps) low *= m;
+            if (it < kSelectMaxSteps) low = repeat_scale<false>(low, m, kSelectMaxSteps - it);
             count = ext.nzero;
             break;
           }
@@ -1079,13 +1225,47 @@ __device__ __forceinline__ void multi_select_body(const MultiArgs a, int depth, 
   }
 }
 
-__global__ void __launch_bounds__(kSearchThreads)
-    k_multi_select(const MultiArgs a, int depth, const unsigned long long* __restrict__ keys,
-                   const double* __restrict__ net_part, int nb,
-                   const double* __restrict__ hist_part, const KeyExtent* __restrict__ ext_part,
-                   int nh, DepthState* __restrict__ state, SelectState* __restrict__ sel,
+// Whether this block is the last of the grid to get here (a counter that the
+// last block sets back to 0).  What the blocks hand over is stored and loaded
+// agent-coherent, and each wave's stores are performed before its block
+// counts itself in.  Every lane; contains barriers.
+__device__ __forceinline__ bool last_block(unsigned* counter) {
+  __shared__ int last;
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+           gridDim.x - 1;
+    if (last) st_ag(counter, 0u);
+  }
+  __syncthreads();
+  return last != 0;
+}
+
+// Depth not reached: neither is the next, and there is no search.  One lane.
+__device__ __forceinline__ void skip_select(const MultiArgs& a, int depth, DepthState* state,
+                                            SelectState* sel) {
+  st_ag(&sel->bisect, 0);
+  if (depth + 1 < a.R) st_ag(&state[depth + 1].active, 0);
+}
+
+// The histogram, then the search on the last block (its ladder is in LDS
+// already): 15.5 us; 37 with the search in a launch of its own, rows of counts
+// per block and one lane's chains of divisions.
+__global__ void __launch_bounds__(kMultiThreads)
+    k_multi_ladder(const MultiArgs a, int depth, const unsigned long long* __restrict__ keys,
+                   const double* __restrict__ net_part, int nb_net, DepthState* state,
+                   SelectState* sel, int* counts, KeyExtent* ext_part, unsigned* counter,
                    double* __restrict__ lower, double* __restrict__ upper) {
-  multi_select_body(a, depth, keys, net_part, nb, hist_part, ext_part, nh, state, sel, lower, upper, blockIdx.x, gridDim.x);
+  __shared__ LadderLds s;
+  if (!ld_ag(&state[depth].active)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) skip_select(a, depth, state, sel);
+    return;
+  }
+  multi_ladder_body(a, depth, keys, net_part, nb_net, state, counts, ext_part, s, blockIdx.x,
+                    gridDim.x);
+  if (last_block(counter))
+    multi_select_body(a, depth, keys, counts, ext_part, gridDim.x, state, sel, lower, upper, s);
 }
 
 
@@ -1106,16 +1286,18 @@ __device__ __forceinline__ int tree_rank(int i) {
   return (2 * (i - (1 << k)) + 1) * (1 << (kTreeDepth - 1 - k)) - 1;
 }
 
-// Per block: cumulative counts, in in-order position, of the member keys in
-// (low, high] that are <= each tree guess: cum_part[rank * nb + block].
+// Counts, by in-order position, of the member keys in (low, high]
+// whose first guess >= key it is, added to counts.
 __device__ __forceinline__ void multi_tree_body(const MultiArgs a, int depth, const unsigned long long* __restrict__ keys,
                  const DepthState* __restrict__ state, const SelectState* __restrict__ sel,
-                 int* __restrict__ cum_part, int blk, int nblk) {
+                 int* __restrict__ counts, int blk, int nblk) {
   __shared__ double lo[kTreeNodes + 1], hi[kTreeNodes + 1];
   __shared__ unsigned long long ts[kTreeNodes];
   __shared__ int hist[kTreeNodes + 1];
   if (!ld_ag(&state[depth].active) || !ld_ag(&sel->bisect)) return;
   const double low = ld_ag(&sel->low), high = ld_ag(&sel->high);
+  const int p0 = blk * blockDim.x + threadIdx.x;
+  const unsigned long long key0 = p0 < a.P ? ld_ag(keys + p0) : kKeySentinel;
   for (int k = 0; k < kTreeDepth; ++k) {
     for (int i = (1 << k) + threadIdx.x; i < (2 << k); i += blockDim.x) {
       double l = low, h = high;
@@ -1139,99 +1321,53 @@ __device__ __forceinline__ void multi_tree_body(const MultiArgs a, int depth, co
   for (int t = threadIdx.x; t < kTreeNodes; t += blockDim.x) hist[t] = 0;
   __syncthreads();
   const unsigned long long lb = key_of(low), hb = key_of(high);
-  for (int p = blk * blockDim.x + threadIdx.x; p < a.P; p += nblk * blockDim.x) {
-    const unsigned long long key = ld_ag(keys + p);
+  for (int p = p0; p < a.P; p += nblk * blockDim.x) {
+    const unsigned long long key = p == p0 ? key0 : ld_ag(keys + p);
     if (key != kKeySentinel && key > lb && key <= hb) {
       const int b = ladder_bin(ts, kTreeNodes, key);
       if (b < kTreeNodes) atomicAdd(&hist[b], 1);
     }
   }
   __syncthreads();
-  if (threadIdx.x < 64) {
-    // inclusive prefix over the in-order bins on one wavefront: each lane
-    // sums a run of kScanRun bins, the lanes' sums are scanned across the
-    // wavefront, then each lane writes its run's prefixes (integer counts,
-    // so the order of the additions does not matter)
-    constexpr int kScanRun = (kTreeNodes + 63) / 64;
-    const int lane = threadIdx.x;
-    int v[kScanRun];
-    int sum = 0;
+  add_counts(hist, kTreeNodes, counts);
+}
+
+// Counts of the member keys in (low, high] that are <= each tree guess, by
+// in-order position, into cum: a prefix sum of the counts (integers, so the
+// order of the additions does not matter).  Whole block, barriers.
+__device__ void tree_counts(int* __restrict__ counts, int* cum) {
+  static_assert(kTreeNodes + 1 == kMultiThreads, "one lane per position");
+  __shared__ int wave_sum[kMultiThreads / 64];
+  const int t = threadIdx.x, lane = t & 63;
+  int c = t < kTreeNodes ? take_count(counts, t) : 0;
 #pragma unroll
-    for (int q = 0; q < kScanRun; ++q) {
-      const int t = lane * kScanRun + q;
-      v[q] = t < kTreeNodes ? hist[t] : 0;
-      sum += v[q];
-    }
-    int incl = sum;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += y;
-    }
-    int run = incl - sum;
-#pragma unroll
-    for (int q = 0; q < kScanRun; ++q) {
-      const int t = lane * kScanRun + q;
-      run += v[q];
-      if (t < kTreeNodes) hist[t] = run;
-    }
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(c, o, 64);
+    if (lane >= o) c += y;
   }
+  if (lane == 63) wave_sum[t >> 6] = c;
   __syncthreads();
-  for (int t = threadIdx.x; t < kTreeNodes; t += blockDim.x)
-    st_ag(cum_part + static_cast<size_t>(t) * nblk + blk, hist[t]);
-}
-
-__global__ void __launch_bounds__(kMultiThreads)
-    k_multi_tree(const MultiArgs a, int depth, const unsigned long long* __restrict__ keys,
-                 const DepthState* __restrict__ state, const SelectState* __restrict__ sel,
-                 int* __restrict__ cum_part) {
-  multi_tree_body(a, depth, keys, state, sel, cum_part, blockIdx.x, gridDim.x);
-}
-
-
-// Sums over the blocks of the counts of the tree nodes in the kSubtreeLevels
-// levels of the subtree rooted at `root` (heap order; nodes past the tree
-// are skipped) into sub[local], local = 2^l - 1 + j for node root 2^l + j:
-// one wavefront per node, all in flight at once.  Whole block, barrier.
-constexpr int kSubtreeLevels = 4;
-constexpr int kSubtreeNodes = (1 << kSubtreeLevels) - 1;
-static_assert(kSubtreeNodes <= kSearchThreads / 64 && kSubtreeNodes <= kMultiThreads / 64,
-              "one wavefront per subtree node");
-
-__device__ void subtree_counts(const int* __restrict__ cum_part, int nb, int root,
-                               long long* sub) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  __syncthreads();  // every lane has read the previous subtree's counts
-  if (w < kSubtreeNodes) {
-    const int l = 31 - __builtin_clz(w + 1);   // level below the root
-    const int node = (root << l) + (w + 1 - (1 << l));
-    long long c = 0;
-    if (node <= kTreeNodes) {
-      const size_t row = static_cast<size_t>(tree_rank(node)) * nb;
-      for (int b = lane; b < nb; b += 64) c += ld_ag(cum_part + row + b);
-    }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-    if (lane == 0) sub[w] = c;
-  }
+  for (int w = 0; w < kMultiThreads / 64; ++w) c += w < (t >> 6) ? wave_sum[w] : 0;
+  cum[t] = c;
   __syncthreads();
 }
 
 // The gold's bisection loop on the tree counts.  Count at a guess g in
 // [low, high] = count at low + keys in (low, g].  A stage that runs past its
 // tree hands (low, high, count at low, step counter) to the next stage
-// (k_multi_tree + k_multi_bisect again); the last stage continues with
+// (k_multi_tree again); the last stage continues with
 // block-wide counts over all keys.
 __device__ __forceinline__ void multi_bisect_body(const MultiArgs a, int depth, DepthState* __restrict__ state,
                    SelectState* __restrict__ sel, const unsigned long long* __restrict__ keys,
-                   const int* __restrict__ cum_part, const KeyExtent* __restrict__ ext_part,
+                   int* __restrict__ counts, const KeyExtent* __restrict__ ext_part,
                    int nb, double* __restrict__ lower, double* __restrict__ upper,
-                   int last_stage, int blk, int nblk) {
+                   int last_stage) {
   __shared__ long long red[16];
-  __shared__ long long sub[kSubtreeNodes];
+  __shared__ int cum[kTreeNodes + 1];
   __shared__ KeyExtent ext;
   if (!ld_ag(&state[depth].active) || !ld_ag(&sel->bisect)) return;
-  reduce_extents(ext_part, nb, &ext);
+  bool have_ext = false;  // the extents are needed past the tree only
   const long long n_pre = ld_ag(&state[depth].n_pre);
   const double np = static_cast<double>(n_pre);
   const long long lowerT = static_cast<long long>(np * a.lower_frac);
@@ -1241,20 +1377,12 @@ __device__ __forceinline__ void multi_bisect_body(const MultiArgs a, int depth, 
   int it = ld_ag(&sel->it);
   int node = 1;
   const long long c0 = c_low;  // the tree counts keys in (low, high] of this stage
-  // the counts of a subtree of nodes are summed together, so kSubtreeLevels
-  // steps of the walk take one round of cross-block loads
-  int sub_root = 0;
+  tree_counts(counts, cum);
   auto count_at = [&](double g) -> long long {
-    if (node <= kTreeNodes) {
-      const int dl = sub_root ? (31 - __builtin_clz(node)) - (31 - __builtin_clz(sub_root)) : -1;
-      if (dl < 0 || dl >= kSubtreeLevels || (node >> dl) != sub_root) {
-        sub_root = node;
-        subtree_counts(cum_part, nb, sub_root, sub);
-        return c0 + sub[0];
-      }
-      return c0 + sub[(1 << dl) - 1 + (node - (sub_root << dl))];
-    }
+    if (node <= kTreeNodes) return c0 + cum[tree_rank(node)];
     if (!(g >= 0.0)) return 0;
+    if (!have_ext) reduce_extents(ext_part, nb, &ext);
+    have_ext = true;
     const long long c = extent_count(ext, g);
     return c >= 0 ? c : block_count(keys, a.P, key_of(g), red);
   };
@@ -1289,13 +1417,18 @@ __device__ __forceinline__ void multi_bisect_body(const MultiArgs a, int depth, 
   }
 }
 
-__global__ void __launch_bounds__(kSearchThreads)
-    k_multi_bisect(const MultiArgs a, int depth, DepthState* __restrict__ state,
-                   SelectState* __restrict__ sel, const unsigned long long* __restrict__ keys,
-                   const int* __restrict__ cum_part, const KeyExtent* __restrict__ ext_part,
-                   int nb, double* __restrict__ lower, double* __restrict__ upper,
-                   int last_stage) {
-  multi_bisect_body(a, depth, state, sel, keys, cum_part, ext_part, nb, lower, upper, last_stage, blockIdx.x, gridDim.x);
+// The tree's histogram, then the bisection on the last block: 14 us, 18 with
+// the bisection in a launch of its own; without a search to end, 4.5 for 9.
+__global__ void __launch_bounds__(kMultiThreads)
+    k_multi_tree(const MultiArgs a, int depth, const unsigned long long* __restrict__ keys,
+                 DepthState* state, SelectState* sel, int* counts, const KeyExtent* ext_part,
+                 unsigned* counter, double* __restrict__ lower, double* __restrict__ upper,
+                 int last_stage) {
+  if (!ld_ag(&state[depth].active) || !ld_ag(&sel->bisect)) return;
+  multi_tree_body(a, depth, keys, state, sel, counts, blockIdx.x, gridDim.x);
+  if (last_block(counter))
+    multi_bisect_body(a, depth, state, sel, keys, counts, ext_part, gridDim.x, lower, upper,
+                      last_stage);
 }
 
 
@@ -1313,7 +1446,8 @@ __device__ __forceinline__ void multi_final_body(const MultiArgs a, const float*
   const size_t P = static_cast<size_t>(a.P);
   double s = 0.0;
   for (int p = blk * blockDim.x + threadIdx.x; p < a.P; p += nblk * blockDim.x) {
-    const double y = decide(a, 0, a.v, a.k, bv, cash, ev, P, p, Y[p], beta, nrm, lo, hi);
+    const PathIn in = load_path(bv, ev, cash, 0, a.max_vars, a.v, P, p);
+    const double y = decide(a, a.v, a.k, in, Y[p], beta, nrm, lo, hi);
     s += y / static_cast<double>(num[p]);
   }
   block_sum_to<true>(s, red, part + blk);
@@ -1329,10 +1463,27 @@ __global__ void __launch_bounds__(kMultiThreads)
 }
 
 
-__global__ void k_fill_zero(double* __restrict__ a, size_t n) {
-  for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < n;
-       i += static_cast<size_t>(gridDim.x) * blockDim.x)
-    a[i] = 0.0;
+// Outputs start at zero (depths never reached stay zero), and the counter of
+// last_block.
+struct ZeroSpans {
+  double* p[6];
+  size_t n[6];
+};
+
+__device__ __forceinline__ void zero_counts(int* hist, int* cum) {
+  for (int t = threadIdx.x; t < kLadderBins; t += blockDim.x) st_ag(hist + t, 0);
+  for (int t = threadIdx.x; t <= kTreeNodes; t += blockDim.x) st_ag(cum + t, 0);
+}
+
+__global__ void k_multi_zero(const ZeroSpans z, unsigned* counter, int* hist, int* cum) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) *counter = 0u;
+    zero_counts(hist, cum);
+  }
+  for (int k = 0; k < 6; ++k)
+    for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < z.n[k];
+         i += static_cast<size_t>(gridDim.x) * blockDim.x)
+      z.p[k][i] = 0.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1383,11 +1534,13 @@ __global__ void __launch_bounds__(kMultiThreads)
                  const float* __restrict__ num, double* coeffs, double* lower, double* upper,
                  double* norm, double* means, double* sds, double* Y, unsigned char* mem,
                  unsigned long long* keys, int* cum, double* stats, double* gram, double* net,
-                 double* hist, KeyExtent* ext, double* price_part, DepthState* state,
+                 int* hist, KeyExtent* ext, double* price_part, DepthState* state,
                  SelectState* sel, unsigned* bar, double* price_out) {
+  __shared__ LadderLds lad;
   const int blk = blockIdx.x, G = gridDim.x;
   const bool cross = a.cross != 0;
   unsigned phase = 0;
+  if (blk == 0) zero_counts(hist, cum);
   // outputs start at zero (depths never reached stay zero)
   {
     const size_t ncoef = static_cast<size_t>(a.E) * a.R * a.maxd, ncut = static_cast<size_t>(a.E) * a.R;
@@ -1432,10 +1585,9 @@ __global__ void __launch_bounds__(kMultiThreads)
       if (blk < nb)
         multi_net_body(a, d, bv, ev, mem, state, norm, gram, coeffs, keys, net, blk, nb);
       if (!multi_grid_sync(bar + 2, ++phase)) goto fail;
-      if (blk < nh) multi_ladder_body(a, d, keys, net, nb, state, hist, ext, blk, nh);
+      if (blk < nh) multi_ladder_body(a, d, keys, net, nb, state, hist, ext, lad, blk, nh);
       if (!multi_grid_sync(bar + 2, ++phase)) goto fail;
-      if (blk == 0)
-        multi_select_body(a, d, keys, net, nb, hist, ext, nh, state, sel, lower, upper, 0, 1);
+      if (blk == 0) multi_select_body(a, d, keys, hist, ext, nh, state, sel, lower, upper, lad);
       if (!multi_grid_sync(bar + 2, ++phase)) goto fail;
       for (int stage = 0; stage < kBisectStages; ++stage) {
         if (!ld_ag(&sel->bisect)) break;  // the search ended without (more) bisection
@@ -1443,7 +1595,7 @@ __global__ void __launch_bounds__(kMultiThreads)
         if (!multi_grid_sync(bar + 2, ++phase)) goto fail;
         if (blk == 0)
           multi_bisect_body(a, d, state, sel, keys, cum, ext, nh, lower, upper,
-                            stage + 1 == kBisectStages ? 1 : 0, 0, 1);
+                            stage + 1 == kBisectStages ? 1 : 0);
         if (!multi_grid_sync(bar + 2, ++phase)) goto fail;
       }
     }
@@ -1497,7 +1649,7 @@ MultiLayout multi_layout(int paths) {
   l.keys = o;
   o += al256(8 * P);
   l.cum = o;
-  o += al256(4 * static_cast<size_t>(kTreeNodes) * nb);
+  o += al256(4 * (kTreeNodes + 1));
   l.stats = o;
   o += al256(8 * 2 * kMaxBasisVars * nb);
   l.gram = o;
@@ -1505,7 +1657,7 @@ MultiLayout multi_layout(int paths) {
   l.net = o;
   o += al256(8 * 2 * nb);
   l.hist = o;
-  o += al256(8 * kLadderSlots * nb);
+  o += al256(4 * kLadderBins);
   l.ext = o;
   o += al256(sizeof(KeyExtent) * nb);
   l.price = o;
@@ -1586,7 +1738,7 @@ extern "C" int ls_multi_first_pass_gpu(
   double* stats = reinterpret_cast<double*>(ws + lay.stats);
   double* gram = reinterpret_cast<double*>(ws + lay.gram);
   double* net = reinterpret_cast<double*>(ws + lay.net);
-  double* hist = reinterpret_cast<double*>(ws + lay.hist);
+  int* hist = reinterpret_cast<int*>(ws + lay.hist);
   KeyExtent* ext = reinterpret_cast<KeyExtent*>(ws + lay.ext);
   double* price_part = reinterpret_cast<double*>(ws + lay.price);
   double* norm = reinterpret_cast<double*>(ws + lay.norm);
@@ -1613,10 +1765,9 @@ extern "C" int ls_multi_first_pass_gpu(
 
   // With KOO_LS_MULTI_PERSISTENT=1, one persistent launch (after zeroing
   // its barrier words) when all nb blocks can be resident: the same bodies
-  // and blocks, bit for bit the same results.  Not the default: on the
-  // config-3 path quantities it measures 5.0 ms per pass against 3.7 ms for
-  // the launch per phase, the one-block band searches running 16 wavefronts
-  // of the same serial search where their own launches run 4.
+  // and blocks, bit for bit the same results.  Not the default: 2^17 paths,
+  // ten dates, three depths take 2.5 ms against 1.77 ms for the launch per
+  // phase (2.7 before the searches moved to the last block of the histograms).
   {
     int per_cu = 0;
     const char* persistent = getenv("KOO_LS_MULTI_PERSISTENT");
@@ -1636,21 +1787,13 @@ extern "C" int ls_multi_first_pass_gpu(
     }
   }
 
-  // outputs start at zero (depths never reached stay zero)
   const size_t ncoef = static_cast<size_t>(n_ex) * R * maxd, ncut = static_cast<size_t>(n_ex) * R;
   const size_t nvar = static_cast<size_t>(n_ex) * R * max_vars;
-  hipLaunchKernelGGL(k_fill_zero, dim3(grid_for(ncoef, 256, 256)), dim3(256), 0, st, coefficients,
-                     ncoef);
-  hipLaunchKernelGGL(k_fill_zero, dim3(grid_for(ncut, 256, 256)), dim3(256), 0, st, lower_cuts,
-                     ncut);
-  hipLaunchKernelGGL(k_fill_zero, dim3(grid_for(ncut, 256, 256)), dim3(256), 0, st, upper_cuts,
-                     ncut);
-  hipLaunchKernelGGL(k_fill_zero, dim3(grid_for(2 * nvar + 1, 256, 256)), dim3(256), 0, st, norm,
-                     2 * nvar + 1);
-  if (means && nvar)
-    hipLaunchKernelGGL(k_fill_zero, dim3(grid_for(nvar, 256, 256)), dim3(256), 0, st, means, nvar);
-  if (sds && nvar)
-    hipLaunchKernelGGL(k_fill_zero, dim3(grid_for(nvar, 256, 256)), dim3(256), 0, st, sds, nvar);
+  unsigned* counter = reinterpret_cast<unsigned*>(ws + lay.bar);
+  const ZeroSpans zs{{coefficients, lower_cuts, upper_cuts, norm, means, sds},
+                     {ncoef, ncut, ncut, 2 * nvar + 1, means ? nvar : 0, sds ? nvar : 0}};
+  hipLaunchKernelGGL(k_multi_zero, dim3(grid_for(ncoef + 2 * nvar + 1, 256, 256)), dim3(256), 0, st, zs,
+                     counter, hist, cum);
 
   for (int e = n_ex - 1; e >= 0; --e) {
     a.e = e;
@@ -1674,16 +1817,11 @@ extern "C" int ls_multi_first_pass_gpu(
                          basis_variables, exercise_values, mem, state, norm, gram, coefficients,
                          keys, net);
       hipLaunchKernelGGL(k_multi_ladder, dim3(nh), dim3(kMultiThreads), 0, st, a, d, keys, net, nb,
-                         state, hist, ext);
-      hipLaunchKernelGGL(k_multi_select, dim3(1), dim3(kSearchThreads), 0, st, a, d, keys, net,
-                         nb, hist, ext, nh, state, sel, lower_cuts, upper_cuts);
-      for (int stage = 0; stage < kBisectStages; ++stage) {
+                         state, sel, hist, ext, counter, lower_cuts, upper_cuts);
+      for (int stage = 0; stage < kBisectStages; ++stage)
         hipLaunchKernelGGL(k_multi_tree, dim3(nh), dim3(kMultiThreads), 0, st, a, d, keys, state,
-                           sel, cum);
-        hipLaunchKernelGGL(k_multi_bisect, dim3(1), dim3(kSearchThreads), 0, st, a, d, state, sel,
-                           keys, cum, ext, nh, lower_cuts, upper_cuts,
+                           sel, cum, ext, counter, lower_cuts, upper_cuts,
                            stage + 1 == kBisectStages ? 1 : 0);
-      }
     }
   }
   a.e = 0;
