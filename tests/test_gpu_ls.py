@@ -637,6 +637,29 @@ def test_persistent_portfolio_equals_stage_calls(torch_cuda, seed, paths):
         assert abs(pr.price1.item() - p1) <= 1e-12 * abs(p1), j
 
 
+@pytest.mark.parametrize("paths", [257, 1 << 16, (1 << 16) + 300])
+def test_persistent_teams_of_a_block_per_chunk(torch_cuda, paths):
+    """Teams of as many blocks as the product has 256-path chunks, up to 256
+    (the most columns of the first pass's partials): two chunks with one path
+    in the second, exactly 256, and 258 (two blocks take two).  The first pass
+    sums its partials over other blocks than the single call: 1e-12, as above."""
+    torch = torch_cuda
+    prods = configs.bermudan_portfolio(n_products=2, paths=paths, seed=83)
+    pf = pipeline.PortfolioPricer(prods, checkpoint_every=4, n_streams=2)
+    assert pf.persistent
+    print(f"persistent teams, 2 products x {paths} paths", flush=True)
+    pf.run(capture=False)
+    torch.cuda.synchronize()
+    got = pf.results()
+    for j, pr in enumerate(pf.pricers):
+        assert pf.pplan.team_blocks[j] == min((paths + 255) // 256, 256)
+        p1, p2, g = got[j]
+        assert np.isfinite(p2) and np.all(np.isfinite(g))
+        pr.regress()
+        torch.cuda.synchronize()
+        assert abs(pr.price1.item() - p1) <= 1e-12 * abs(p1), j
+
+
 def test_portfolio_persistent_ls_equals_per_round_launches(torch_cuda):
     """The portfolio's LS first passes as one persistent launch (resident
     blocks walking all products' blocks, the partials exchanged through

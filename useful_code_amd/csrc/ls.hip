@@ -458,13 +458,21 @@ struct LsLayout {
   size_t y, part, xbuf, bar, total;
 };
 
+// Columns of the first pass's partial slots: the blocks of the per-round
+// launches, and, for the teams of a persistent portfolio, one for each of
+// their blocks of 256 paths up to the 256 columns that a round's sum reads in
+// one go (every block of the team sums them all).
+int xbuf_columns(int paths) {
+  return std::max(gram_blocks(paths), std::min((paths + 255) / 256, 256));
+}
+
 LsLayout ls_layout(int paths) {
   LsLayout l;
   l.y = 0;
   l.part = align256(sizeof(float) * static_cast<size_t>(paths));
   const int nb = ls_blocks(paths) > gram_blocks(paths) ? ls_blocks(paths) : gram_blocks(paths);
   l.xbuf = l.part + align256(sizeof(double) * kMaxGram * kMaxGram * nb);
-  l.bar = l.xbuf + align256(sizeof(double) * 3 * kTriMax * gram_blocks(paths));
+  l.bar = l.xbuf + align256(sizeof(double) * 3 * kTriMax * xbuf_columns(paths));
   l.total = l.bar + 256;
   return l;
 }
@@ -732,7 +740,7 @@ fail:
 
 namespace koo {
 size_t ls_workspace_xbuf_offset(int paths) { return ls_layout(paths).xbuf; }
-int ls_workspace_xbuf_columns(int paths) { return gram_blocks(paths); }
+int ls_workspace_xbuf_columns(int paths) { return xbuf_columns(paths); }
 }  // namespace koo
 
 using namespace koo;
