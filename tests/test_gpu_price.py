@@ -246,3 +246,53 @@ def test_windows_blocks_and_intervals_vs_fp64_adjoint(torch_cuda, P, N, F, k):
     assert abs(alone / pp.mean() - 1) < 2e-5
     assert np.all(np.abs(g - g64)[:N] <= 2e-5 * np.max(np.abs(d / P)))
     assert np.all(np.abs(g - g64)[N:] <= 2e-5 * np.max(np.abs(v / P)))
+
+
+@pytest.mark.parametrize("P,N,F,k", [
+    (1, 4, 1, 1), (17, 16, 8, 2), (33, 17, 2, 1), (9, 32, 7, 4), (5, 33, 6, 1), (7, 64, 5, 8),
+    (16384, 16, 3, 4), (12288, 20, 4, 3), (8192, 40, 5, 8),
+    (16385, 5, 6, 3), (16390, 12, 1, 1), (12289, 20, 4, 3), (8200, 46, 5, 8)])
+def test_rates_across_lanes_and_single_wavefront_blocks(torch_cuda, P, N, F, k):
+    """Few paths run with a path's rates across 16, 32 or 64 lanes: the
+    smallest and largest curve of each, one path and counts that leave part of
+    a wavefront and of a block idle, and the most paths of each; and just above
+    those, single-wavefront blocks of a path per lane.
+
+    Rounding moves each path's Greek by at most 4 units of 2^-24 of its size a
+    step (as above), so the mean by 4 N 2^-24 of the paths' mean size -- not of
+    the mean itself, which may cancel: struck at zero, the caplets' vegas do
+    over the paths.  The mean size from 32 of the paths, doubled for that."""
+    rng = np.random.RandomState(100 * N + F)
+    f0 = 0.04 + 0.01 * rng.uniform(size=N)
+    taus = np.full(N, 0.5)
+    vols = rng.uniform(0.1, 0.2, N)
+    A = (vols[None, :, None] * np.sqrt(0.5 / F) * rng.uniform(0.5, 1.0, size=(N, N, F)))
+    f0, vols, A = (x.astype(np.float32).astype(np.float64) for x in (f0, vols, A))
+    w = configs.LMMWorkload("across", P, N, F, 0.5, f0, vols, 0.5 * np.arange(1, N + 2), A, 0.0,
+                            "caplets", np.zeros(N * F, np.uint32), checkpoint_every=k,
+                            displacements=np.full(N, 0.0078125))
+    pr = pipeline.LMMPricer(w)
+    z = rng.normal(size=(N, F, P)).astype(np.float32)
+    pr.z.copy_(torch_cuda.from_numpy(z.reshape(-1)))
+
+    def fp64(zz):
+        n = zz.shape[2]
+        return O.caplet_adjoint_paths(
+            O.caplet_model(f0, taus, w.disp(), A, vols, w.strike, n), zz.astype(np.float64))
+
+    pp, d, v = fp64(z)
+    few = [fp64(np.ascontiguousarray(z[:, :, p:p + 1])) for p in range(min(P, 32))]
+    size = [2 * np.mean([np.abs(x[i]) for x in few], axis=0).max() for i in (1, 2)]
+    pr.price_kernel(checkpoints=False)
+    alone = pr.price_out.item()
+    pr.price_kernel(checkpoints=True)
+    pr.greeks_kernel()
+    g = pr.greeks_out.cpu().numpy()
+    err = np.abs(g - np.concatenate([d, v]) / P)
+    print(f"P={P} N={N} F={F} k={k}: price rel {alone / pp.mean() - 1:.2e}, deltas "
+          f"{err[:N].max() / size[0]:.2e}, vegas {err[N:].max() / size[1]:.2e}", flush=True)
+    bound = 4 * N * 2.0**-24
+    assert alone == pr.price_out.item()
+    assert abs(alone / pp.mean() - 1) <= bound
+    assert np.all(err[:N] <= bound * size[0])
+    assert np.all(err[N:] <= bound * size[1])

@@ -21,6 +21,10 @@
 // partial sums are formed in FP64 and a final single pass sums them with
 // compensation.
 //
+// Few paths take the form with a path's rates across the lanes instead
+// (lmm_across.h; k_price_fwd_across, k_price_bwd_across): it keeps nothing
+// between forward and backward, which runs the steps again.
+//
 // Both kernels issue vector instructions most of the time, so they got faster
 // by having fewer: the step in the state's units (relative, base 2), the
 // diffusion carried along with the predictor drift, buffer addressing, the vega
@@ -28,10 +32,12 @@
 // and k = 8 those of 300 of the 820 rate updates; all of them while each step's
 // states were kept in scratch, 14.8 GB of traffic).  At 2^20 paths, 40 rates, 5
 // factors and k = 8: forward with checkpoints 1250 -> 845 us, backward 3655 ->
-// 2440 us; at k = 8 and 4096 paths 188 -> 107 and 535 -> 230 us; price of 2^17
-// paths, 80 rates, 2 factors 1525 -> 365 us (its step table was in LDS and left
+// 2440 us; at k = 8 and 4096 paths 188 -> 107 and 535 -> 230 us, 51 and 107 with
+// the rates across the lanes; price of 2^17 paths, 80 rates, 2 factors 1525 -> 365 us (its step table was in LDS and left
 // room for three wavefronts per CU).
-#include "lmm_step.h"
+#include <algorithm>
+
+#include "lmm_across.h"
 
 namespace koo {
 
@@ -188,6 +194,115 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
   adjoint_sums<BD>(m, vols, lam, vegas, part, blockIdx.x);
 }
 
+// Few paths: the rates of a path across W lanes (lmm_across.h).  Once the paths
+// have fixed, every lane values its own caplet: 1/B as a product scan, and for
+// the adjoint the value of the later caplets as a sum scan.
+struct Fixing {
+  float inv, before, v;  // 1 / (1 + tau f), 1/B before the step, deflated value
+};
+template <int W>
+__device__ __forceinline__ Fixing across_fixing(const Model& m, const AcrossLane<W>& at, float x) {
+  Fixing o{1.0f, 0.0f, 0.0f};
+  float f = 0.0f, tau = 0.0f;
+  if (at.live) {
+    tau = m.taus[at.r];
+    f = fmaf(start_level(m, at.r), fast_exp2(x), -m.disp[at.r]);
+    o.inv = fast_rcp(1.0f + tau * f);
+  }
+  const float upto = __shfl_up(scan_mul<W>(o.inv), 1, W);
+  o.before = at.r ? upto : 1.0f;
+  if (at.live) o.v = caplet_value(f, tau, m.strike, o.inv) * o.before;
+  return o;
+}
+
+template <int F, int W>
+__global__ void __launch_bounds__(kAcrossLanes)
+    k_price_fwd_across(KOO_MODEL_PARAMS, double* __restrict__ part) {
+  KOO_MODEL_LOCAL;
+  __shared__ double red[kAcrossLanes / 64];
+  const AcrossLane<W> at(m, blockIdx.x);
+  const float kr = at.rate ? rate_kr(m, at.r) : 1.0f;
+  const float x = across_steps<F, W>(m, at, kr, [](int, float, float, float) {});
+  block_sum_to(static_cast<double>(across_fixing<W>(m, at, x).v), red, part + blockIdx.x);
+}
+
+// The forward again with what the reverse needs in LDS, then the reverse.
+template <int F, int W>
+__global__ void __launch_bounds__(kAcrossLanes)
+    k_price_bwd_across(KOO_MODEL_PARAMS, const float* __restrict__ vols,
+                       double* __restrict__ part) {
+  KOO_MODEL_LOCAL;
+  extern __shared__ float lds[];
+  const AcrossLane<W> at(m, blockIdx.x);
+  const int N = m.N, path = static_cast<int>(threadIdx.x) / W, tri = across_tri(N);
+  float* mine = lds + static_cast<size_t>(path) * 3 * tri;
+  const float kr = at.rate ? rate_kr(m, at.r) : 1.0f;
+  const float xf = across_steps<F, W>(m, at, kr, [&](int s, float x, float my, float md) {
+    if (at.rate && at.r >= s) {
+      float* o = mine + across_tri_row(N, s) + N - 1 - at.r;
+      o[0] = x;
+      o[tri] = my;
+      o[2 * tri] = md;
+    }
+  });
+  const Fixing fx = across_fixing<W>(m, at, xf);
+  // from here the lane has rate r = N - 1 - (its place)
+  const int l = at.r, r = max(N - 1 - l, 0);
+  const bool rate = at.rate;
+  const float x = __shfl(xf, r, W), inv = __shfl(fx.inv, r, W), before = __shfl(fx.before, r, W);
+  const float v = __shfl(fx.v, r, W);
+  const float above = __shfl_up(scan_add<W>(rate ? v : 0.0f), 1, W);
+  float lam = 0.0f, krr = 1.0f;
+  if (rate) krr = rate_kr(m, r);
+  if (at.live) {
+    const float tau = m.taus[r], xs = start_level(m, r) * fast_exp2(x);
+    const float tail = l ? above : 0.0f;
+    lam = (caplet_deriv(xs - m.disp[r], tau, m.strike, inv) * before - tau * inv * tail) * (kLn2 * xs);
+  }
+  __syncthreads();
+  const float w = across_reverse<F, W>(m, rate ? r : -1, rate, krr, lam,
+                                       [&](int s, float& xo, float& my, float& md) {
+    const float* o = mine + min(across_tri_row(N, s) + l, tri - 1);
+    xo = o[0];
+    my = o[tri];
+    md = o[2 * tri];
+  });
+  // the block's sums, FP64
+  __syncthreads();
+  float* sums = lds;  // [path][2][W]
+  sums[(path * 2) * W + l] = lam;
+  sums[(path * 2 + 1) * W + l] = w;
+  __syncthreads();
+  for (int t = threadIdx.x; t < 2 * N; t += kAcrossLanes) {
+    const int which = t >= N, rr = which ? t - N : t;
+    double sum = 0.0;
+    for (int i = 0; i < kAcrossBlock<W>; ++i)
+      sum += static_cast<double>(sums[(i * 2 + which) * W + N - 1 - rr]);
+    part[static_cast<size_t>(t) * gridDim.x + blockIdx.x] =
+        which ? sum / static_cast<double>(vols[rr])
+              : sum * static_cast<double>(kLog2e) / static_cast<double>(start_level(m, rr));
+  }
+}
+
+// Lanes per path of the across form, 0 for a path per lane.  The across form
+// takes time with its wavefronts beyond the first thousand, the path per lane
+// the same up to 2^15 paths; forward and backward together cross at about 10000
+// wavefronts of 64-lane paths (40 rates, 5 factors: 158 us for 336 at 4096
+// paths, 273 at 8192, 479 at 16384), 7500 of 32-lane ones (20 rates, 3 factors:
+// 71 us for 100 at 8192 paths, 107 at 16384) and 5500 of 16-lane ones (16
+// rates, 5 factors: 76 us for 93 at 16384 paths, 116 at 32768).
+int across_lanes(int paths, int N) {
+  if (N < kShortCurve || N > 64) return 0;
+  const int W = N <= 16 ? 16 : (N <= 32 ? 32 : 64);
+  const int most = W == 16 ? 4096 : (W == 32 ? 6144 : 8192);  // wavefronts
+  return paths <= most * (64 / W) ? W : 0;
+}
+size_t across_lds(int N, int W) {
+  const size_t kept = sizeof(float) * (kAcrossLanes / W) * 3 * across_tri(N);
+  return std::max(kept, sizeof(float) * 2 * kAcrossLanes);
+}
+int across_blocks(int paths, int W) { return (paths + kAcrossLanes / W - 1) / (kAcrossLanes / W); }
+
 int fwd_lanes(int paths, int N) {
   return N >= kShortCurve && N <= 2 * kAdjRates && paths >= 32768 ? kAdjLanes : 64;
 }
@@ -197,7 +312,11 @@ int bwd_lanes(int paths, int N) {
 size_t rows_lds(int rows, int lanes) { return sizeof(float) * static_cast<size_t>(rows) * lanes; }
 // Doubles of the partials before the step table of a forward without
 // checkpoints.
-size_t partial_doubles(int paths, int N) { return static_cast<size_t>(wave_count(paths)) * 2 * N; }
+size_t partial_doubles(int paths, int N) {
+  const int W = across_lanes(paths, N);
+  const int columns = W ? std::max(across_blocks(paths, W), wave_count(paths)) : wave_count(paths);
+  return static_cast<size_t>(columns) * 2 * N;
+}
 
 int check_model(const char* who, int paths, int rates, int factors, int k, int product) {
   if (paths < 1 || rates < 1 || rates > kMaxRates || factors < 1 || factors > kMaxFactors || k < 1)
@@ -209,6 +328,19 @@ int check_model(const char* who, int paths, int rates, int factors, int k, int p
     return set_error(KOO_ERR_INVALID, "%s: unknown product %d", who, product);
   return KOO_OK;
 }
+
+// KOO_W(F, W) for the factors and the lanes per path of the call.
+#define KOO_ACROSS_CASE(F)        \
+  case F:                         \
+    if (W == 16) KOO_W(F, 16);    \
+    else if (W == 32) KOO_W(F, 32); \
+    else KOO_W(F, 64);            \
+    break;
+#define KOO_ACROSS_CASES                                                                    \
+  switch (factors) {                                                                        \
+    KOO_ACROSS_CASE(1) KOO_ACROSS_CASE(2) KOO_ACROSS_CASE(3) KOO_ACROSS_CASE(4)             \
+    KOO_ACROSS_CASE(5) KOO_ACROSS_CASE(6) KOO_ACROSS_CASE(7) KOO_ACROSS_CASE(8)             \
+  }
 
 }  // namespace
 }  // namespace koo
@@ -257,6 +389,17 @@ extern "C" int lmm_price_fwd(int paths, int rates, int factors, int checkpoint_e
                                        paths
                    : reinterpret_cast<float*>(partials + partial_doubles(paths, rates));
   hipStream_t st = as_stream(stream);
+  if (const int W = across_lanes(paths, rates)) {
+    const int nb = across_blocks(paths, W);
+#define KOO_W(F, W)                                                                              \
+  hipLaunchKernelGGL((k_price_fwd_across<F, W>), dim3(nb), dim3(kAcrossLanes), 0, st, m.z, m.f0, \
+                     m.taus, m.disp, m.A, m.strike, m.P, m.N, m.S1, m.L, partials)
+    KOO_ACROSS_CASES
+#undef KOO_W
+    hipLaunchKernelGGL(k_finalize_rows, dim3(1), dim3(finalize_lanes(nb)), 0, st, partials, nb,
+                       1.0 / static_cast<double>(paths), price_out);
+    return check_launch("lmm_price_fwd");
+  }
   switch (factors) {
 #define KOO_FWD(F, BD, U)                                                                        \
   hipLaunchKernelGGL((k_price_fwd<F, BD, U>), dim3(blocks), dim3(BD), lds, st, m.z, m.f0,        \
@@ -303,6 +446,18 @@ extern "C" int lmm_price_bwd(int paths, int rates, int factors, int checkpoint_e
   const float* tab =
       checkpoints + static_cast<size_t>(ckpt_rows(rates, factors, checkpoint_every)) * paths;
   hipStream_t st = as_stream(stream);
+  if (const int W = across_lanes(paths, rates)) {
+    const int nb = across_blocks(paths, W);
+    const size_t bytes = across_lds(rates, W);
+#define KOO_W(F, W)                                                                              \
+  hipLaunchKernelGGL((k_price_bwd_across<F, W>), dim3(nb), dim3(kAcrossLanes), bytes, st, m.z,   \
+                     m.f0, m.taus, m.disp, m.A, m.strike, m.P, m.N, m.S1, m.L, vols, partials)
+    KOO_ACROSS_CASES
+#undef KOO_W
+    hipLaunchKernelGGL(k_finalize_rows, dim3(2 * rates), dim3(finalize_lanes(nb)), 0, st, partials,
+                       nb, 1.0 / static_cast<double>(paths), greeks_out);
+    return check_launch("lmm_price_bwd");
+  }
   switch (factors) {
 #define KOO_BWD(F, BD, U, W)                                                                     \
   hipLaunchKernelGGL((k_price_bwd<F, BD, U, W>), dim3(blocks), dim3(BD), lds, st, m.z, m.f0,     \
