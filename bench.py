@@ -40,22 +40,38 @@ def flops_per_rate_update(F):
     """Algorithmic flops of one rate update (one path, step and alive rate),
     an FMA counted as 2 and a hardware exp or reciprocal as 1, counted from
     the arithmetic of the shared step code (lmm_step.h):
-      forward PC step (pc_step): 5F FMA (e, mu, dW, e^, mu^ sums), 3 MUL,
-        4 ADD, 4 transcendental (exp and reciprocal of g and g^) = 10F + 11;
-      reverse step (reverse_step): 9F + 6 FMA (mu, mu^, dW recomputed, the
-        adjoint sums E^, E and their contractions, e and e^ un-accumulated,
-        the lambda, lambda^ and vega terms), 7 MUL, 7 ADD (three of them the
-        DPP fold of the vega term), 4 transcendental = 18F + 30.
-    At F = 5: 61 + 120 = 181 for the backward kernel (segment recompute plus
-    reverse).  The SQ counters of k_price_bwd<5> read 195 executed FP32 flops
-    per update (85.1 FMA, 6.6 MUL, 10.1 ADD, 8.2 transcendental): the
-    difference is per-step work spread over the rates and multiply-adds the
-    compiler forms from a MUL and an ADD."""
-    return 10 * F + 11, 18 * F + 30
+      forward PC step (pc_step): 4F + 3 FMA (the sums y and d and their
+        contractions; G, Gh and the corrector), 2 ADD, 4 transcendental (exp
+        and reciprocal of G and Gh) = 8F + 12;
+      reverse step (reverse_step): 8F + 9 FMA (the contractions of y and d, the
+        adjoint sums D and Y and theirs, y and d un-accumulated; the states
+        before the step, G, Gh and their slopes, the adjoint, the vega term),
+        3 MUL, 6 ADD, 4 transcendental = 16F + 31."""
+    return 8 * F + 12, 16 * F + 31
 
 
 def rate_updates_per_path(N):
     return N * (N + 1) // 2  # sum over steps s of alive rates N - s
+
+
+def recomputed_updates_per_path(N, F, k):
+    """Rate updates that the reverse sweep runs again: those of the steps from
+    S1 on, the first whose sums the checkpoint rows of interval k have no room
+    for (sweep_plan, lmm_step.h)."""
+    if k == 1:
+        return 0
+    room = -(-N // k) * (N + 1)
+    L = min(N, min(k, N) * (N + 1 + 2 * F) // (2 * F))
+    S1 = N
+    while S1 > 0:
+        more = -(-(N - S1) // L)
+        rows = 2 * F * S1 + N + 1
+        if more > 1:
+            rows += (more - 1) * (N - S1 + 1) - L * (more * (more - 1) // 2)
+        if rows <= room:
+            break
+        S1 -= 1
+    return sum(N - s for s in range(S1, N))
 
 
 # Bytes the LS first pass must move per path and exercise date (FP32): the two basis
@@ -760,7 +776,8 @@ def main():
 
     f_fwd, f_bwd = flops_per_rate_update(F)
     upd = rate_updates_per_path(N) * P
-    bwd_flops = (f_fwd + f_bwd) * upd  # segment recompute + reverse step
+    again = recomputed_updates_per_path(N, F, w.checkpoint_every) * P
+    bwd_flops = f_bwd * upd + f_fwd * again  # reverse steps, steps run again
     achieved_tflops = bwd_flops / (bwd_ms * 1e-3) / 1e12
 
     out = {
@@ -790,7 +807,7 @@ def main():
                        "price_bwd": bwd_ms, "price_fwd": fwd_ms},
         "checkpoint_every_1": k1,
         "roofline": with_traffic({
-            "kernel": f"k_price_bwd<{F}> (reverse sweep + segment recompute)",
+            "kernel": f"k_price_bwd<{F}> (reverse sweep, the steps run again included)",
             "bound": "valu",
             "achieved": achieved_tflops,
             "peak": FP32_VECTOR_PEAK_TFLOPS,

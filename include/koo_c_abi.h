@@ -387,7 +387,8 @@ int koo_sum_f64(const double* in, long long n, double* workspace, double* out, v
  * floats).  checkpoint_every sets the room it has: rates + 1 floats per path
  * and checkpoint_every steps (with 1 also 2 factors floats a step, and nothing
  * is recomputed).  Backward: one reverse sweep per path from those checkpoints
- * (recomputing into segment_scratch the steps there was no room for), giving
+ * (recomputing into segment_scratch the steps there was no room for; for few
+ * paths all of them, on chip, with neither buffer touched), giving
  * greeks_out[0..N) = dV/df_i(0) and greeks_out[N..2N) = dV/dsigma_i with
  * A(s,i,f) proportional to sigma_i.  Sizes of all device buffers come from
  * lmm_price_workspace().  rates <= 90, factors <= 8.  product_aux is a HOST

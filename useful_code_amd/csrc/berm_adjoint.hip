@@ -2,19 +2,19 @@
 // strategy: price and pathwise adjoint Greeks, gfx950.
 //
 // Forward (k_berm_fwd): one lane per path evolves the curve (the shared PC
-// step, state in LDS), checkpoints the state every k steps, and at each
-// exercise date applies the frozen Longstaff-Schwartz rule (exercise when the
-// exercise value is positive, if asked, and exceeds the continuation value of
-// the given coefficients).  At exercise it records the step, the deflated
-// value and the payoff's adjoint on the end-of-step log-rates,
-// d(ev/B)/dl_r = g_r (P_N + K Q_r) / B e^{l_r}, g_r = tau_r / (1 + tau_r f_r),
-// Q_r = sum_{m>r} tau_{m-1} P_m (two passes over the alive rates).  A
+// step, state in LDS), keeps what the reverse needs (SweepPlan, lmm_step.h),
+// and at each exercise date applies the frozen Longstaff-Schwartz rule (exercise
+// when the exercise value is positive, if asked, and exceeds the continuation
+// value of the given coefficients).  At exercise it records the step, the
+// deflated value and the payoff's adjoint on the end-of-step states,
+// d(ev/B)/dx_r = ln2 g_r (P_N + K Q_r) / B (f_r + d_r), g_r = tau_r / (1 + tau_r
+// f_r), Q_r = sum_{m>r} tau_{m-1} P_m (two passes over the alive rates).  A
 // wavefront stops once all its paths have exercised.
 //
-// Backward (k_berm_bwd): the caplet backward's segment recompute and reverse
-// step (lmm_step.h), run per wavefront only up to its last exercise step; at a
-// path's exercise step the recorded payoff adjoint seeds lambda, and each
-// earlier fixing f_s(T_s) inside the numeraire adds -V g_s e^{l_s}.
+// Backward (k_berm_bwd): the caplet backward's sweep (lmm_step.h), run per
+// wavefront only from its last exercise step; at a path's exercise step the
+// recorded payoff adjoint seeds lambda, and each earlier fixing f_s(T_s) inside
+// the numeraire adds -V g_s (f_s + d_s) ln2.
 #include <algorithm>
 #include <vector>
 
