@@ -637,6 +637,38 @@ def test_persistent_portfolio_equals_stage_calls(torch_cuda, seed, paths):
         assert abs(pr.price1.item() - p1) <= 1e-12 * abs(p1), j
 
 
+@pytest.mark.parametrize("persistent", [False, True])
+def test_portfolio_longest_curves_equal_single_calls(torch_cuda, persistent):
+    """45 rates and 5 factors, the most that the batched and persistent launches
+    take (the batched backward's 90 rows of lanes are 92 KB of LDS), beside 41
+    rates: bit for bit the single-product frozen calls on the same variates and
+    coefficients, as the shorter curves."""
+    torch = torch_cuda
+    prods = []
+    for N, F in ((45, 5), (41, 2)):
+        rng = np.random.RandomState(N)
+        f0 = 0.05 + rng.uniform(-0.005, 0.005, N)
+        vols = np.full(N, 0.2)
+        times = 0.5 * np.arange(1, N + 2)
+        A = koo.flat_vol_pseudo_roots(times, times[:N], vols, F, 0.0, 0.1)
+        ex = np.arange(3, N - 1, 6, dtype=np.int32)
+        prods.append(configs.LMMWorkload(
+            f"bermudan_{N}x{F}", 600, N, F, 0.5, f0, vols, times, A, 0.05, "bermudan",
+            rng.randint(0, 2**32, N * F, dtype=np.uint64).astype(np.uint32), exercise_steps=ex,
+            basis_shift=np.full((ex.size, 2), 0.05), basis_scale=np.full((ex.size, 2), 100.0)))
+    pf = pipeline.PortfolioPricer(prods, checkpoint_every=8, n_streams=2, persistent=persistent)
+    assert pf.batched and pf.persistent == persistent
+    print(f"portfolio of 45 and 41 rates, persistent={persistent}", flush=True)
+    pf.run(capture=False)
+    torch.cuda.synchronize()
+    got = pf.results()
+    for j, pr in enumerate(pf.pricers):
+        _, p2, g = got[j]
+        fp, fg = pr.greeks(checkpoint_every=8)
+        torch.cuda.synchronize()
+        assert np.isfinite(p2) and fp.item() == p2 and np.array_equal(fg.cpu().numpy(), g), j
+
+
 @pytest.mark.parametrize("paths", [257, 1 << 16, (1 << 16) + 300])
 def test_persistent_teams_of_a_block_per_chunk(torch_cuda, paths):
     """Teams of as many blocks as the product has 256-path chunks, up to 256
