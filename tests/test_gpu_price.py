@@ -296,3 +296,41 @@ def test_rates_across_lanes_and_single_wavefront_blocks(torch_cuda, P, N, F, k):
     assert abs(alone / pp.mean() - 1) <= bound
     assert np.all(err[:N] <= bound * size[0])
     assert np.all(err[N:] <= bound * size[1])
+
+
+@pytest.mark.parametrize("P,N,F,k", [(200, 90, 2, 1), (300, 70, 5, 8), (8200, 50, 8, 5),
+                                     (32805, 40, 1, 40), (300, 40, 5, 8)])
+def test_greeks_past_an_underflowing_discount_factor(torch_cuda, P, N, F, k):
+    """Rates so high that 1/B leaves FP32's range (2^-160 at the last fixing)
+    long after the caplets that make up the value have paid: the reverse starts
+    from there and still has to arrive at their Greeks.  Every step kept, one and
+    two segments run again, both block sizes, and the rates across lanes.  Bound
+    as in the test above."""
+    rng = np.random.RandomState(N + F)
+    f0 = 2.0 * (2.0 ** (160.0 / N) - 1.0) * rng.uniform(1.0, 1.1, size=N)
+    vols = rng.uniform(0.1, 0.15, N)
+    A = vols[None, :, None] * np.sqrt(0.5 / F) * rng.uniform(0.5, 1.0, size=(N, N, F))
+    f0, vols, A = (x.astype(np.float32).astype(np.float64) for x in (f0, vols, A))
+    w = configs.LMMWorkload("high", P, N, F, 0.5, f0, vols, 0.5 * np.arange(1, N + 2), A, 0.05,
+                            "caplets", np.zeros(N * F, np.uint32), checkpoint_every=k)
+    pr = pipeline.LMMPricer(w)
+    z = rng.normal(size=(N, F, P)).astype(np.float32)
+    pr.z.copy_(torch_cuda.from_numpy(z.reshape(-1)))
+
+    def fp64(zz):
+        return O.caplet_adjoint_paths(O.caplet_model(f0, w.taus, w.disp(), A, vols, w.strike,
+                                                     zz.shape[2]), zz.astype(np.float64))
+
+    pp, d, v = fp64(z)
+    few = [fp64(np.ascontiguousarray(z[:, :, p:p + 1])) for p in range(32)]
+    size = [2 * np.mean([np.abs(x[i]) for x in few], axis=0).max() for i in (1, 2)]
+    pr.price_kernel(checkpoints=True)
+    pr.greeks_kernel()
+    price, g = pr.price_out.item(), pr.greeks_out.cpu().numpy()
+    err = np.abs(g - np.concatenate([d, v]) / P)
+    print(f"P={P} N={N} F={F} k={k}: price rel {price / pp.mean() - 1:.2e}, deltas "
+          f"{err[:N].max() / size[0]:.2e}, vegas {err[N:].max() / size[1]:.2e}", flush=True)
+    bound = 4 * N * 2.0**-24
+    assert abs(price / pp.mean() - 1) <= bound
+    assert np.all(err[:N] <= bound * size[0])
+    assert np.all(err[N:] <= bound * size[1])

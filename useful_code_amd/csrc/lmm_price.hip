@@ -76,7 +76,8 @@ __global__ void __launch_bounds__(BD)
   const int N = m.N;
   const c_cfloat ctab = cmem(tab);
   for (int r = 0; r < N; ++r) X.set(r, 0.0f);
-  float invB = 1.0f, v = 0.0f, vc = 0.0f;
+  Deflator B;
+  float v = 0.0f, vc = 0.0f;
   auto row = [&](int r) { return ckpt + static_cast<size_t>(r) * b.P; };
   int seg_step = ckpt ? m.S1 : N + 1, seg = 0;  // the next step whose states are kept
   auto keep_states = [&](int s) {
@@ -84,7 +85,8 @@ __global__ void __launch_bounds__(BD)
                                      : sweep_segment_row(N, F, m.S1, m.L, seg));
     const int lo = seg == 0 ? 0 : s;
     dump_states(b, X, rows, lo, N);
-    b.row(rows, N - lo).store(invB);
+    b.row(rows, N - lo).store(B.m);
+    if (seg > 0 || sweep_exponent_row(N, m.S1)) b.row(rows, N - lo + 1).store(__int_as_float(B.e));
     ++seg;
     seg_step += m.L;
   };
@@ -107,11 +109,11 @@ __global__ void __launch_bounds__(BD)
     const float fs = fmaf(start_level(m, s), fast_exp2(xs), -m.disp[s]);
     const float inv = fast_rcp(1.0f + tau * fs);
     // Kahan-compensated path sum of the deflated caplet values.
-    const float term = caplet_value(fs, tau, m.strike, inv) * invB - vc;
+    const float term = caplet_value(fs, tau, m.strike, inv) * B.value() - vc;
     const float sum = v + term;
     vc = (sum - v) - term;
     v = sum;
-    invB *= inv;
+    B.scale(inv);
   }
   if (ckpt && seg == 0) keep_states(N);  // S1 == N
   const double sum = wave_sum_f64(static_cast<int>(threadIdx.x) < b.n ? static_cast<double>(v) : 0.0);
@@ -140,7 +142,12 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
   for (int r = 0; r < N; ++r) lam.set(r, 0.0f);
 
   auto row = [&](int r) { return ckpt + static_cast<size_t>(r) * b.P; };
-  float tail = 0.0f, invB = 0.0f;  // invB: 1/B after the step being reversed
+  float tail = 0.0f;
+  Deflator B;  // after the step being reversed
+  auto load_deflator = [&](const float* rows, int r, bool exponent) {
+    B.m = b.row(rows, r).load();
+    B.e = exponent ? __float_as_int(b.row(rows, r + 1).load()) : 0;
+  };
   auto fixing = [&](int s, float& lp, float x) {
     // The rate fixing at the end of this step: caplet value and the numeraire
     // it enters for later fixings.  (Lanes past the last path read 1/B = 0,
@@ -149,7 +156,8 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
     const float xs = start_level(m, s) * fast_exp2(x);
     const float fs = xs - m.disp[s];
     const float grow = 1.0f + tau * fs, inv = fast_rcp(grow);
-    invB *= grow;
+    B.scale(grow);
+    const float invB = B.value();
     const float v = caplet_value(fs, tau, m.strike, inv);
     const float dv = caplet_deriv(fs, tau, m.strike, inv);
     lp = fmaf(dv * invB - tau * inv * tail, kLn2 * xs, lp);
@@ -164,7 +172,7 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
                                      : sweep_segment_row(N, F, m.S1, m.L, seg));
     if (seg == 0) rows += static_cast<size_t>(s0) * b.P;  // the rates that have fixed come first
     load_states(b, X, rows, s0, N);
-    invB = b.row(rows, N - s0).load();
+    load_deflator(rows, N - s0, seg > 0 || sweep_exponent_row(N, m.S1));
     auto load = [&](int r) { return X.get(r); };
     float zn[F];
     load_z<F>(m, b, s0, zn);
@@ -180,7 +188,7 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
       if (s + 1 < s1) pc_fetch<F, U>(ahead, m, s + 1, ctab, load);
       store_sums<F>(b, scratch + static_cast<size_t>(2 * F * (s - s0)) * b.P, y, d);
       const float fs = fmaf(start_level(m, s), fast_exp2(xs), -m.disp[s]);
-      invB *= fast_rcp(1.0f + m.taus[s] * fs);
+      B.scale(fast_rcp(1.0f + m.taus[s] * fs));
     }
     reverse_steps<F, U>(m, b, s1, s0, scratch, ctab, X, lam, nothing, fixing, vegas);
   }
@@ -188,7 +196,7 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
   if (m.S1 > 0) {
     const float* rows = row(sweep_state_row(F, m.S1));
     load_states(b, X, rows, 0, N);
-    invB = b.row(rows, N).load();
+    load_deflator(rows, N, sweep_exponent_row(N, m.S1));
     reverse_steps<F, U>(m, b, m.S1, 0, ckpt, ctab, X, lam, nothing, fixing, vegas);
   }
   adjoint_sums<BD>(m, vols, lam, vegas, part, blockIdx.x);

@@ -108,22 +108,28 @@ struct Model {
 // segment scratch holds, from the states at S1, S1 + L, ...
 // Checkpoint rows: the sums; the N states when step S1 begins (those of rates
 // that have fixed as they fixed) and 1/B there; then per further segment the
-// alive states and 1/B when it begins.
+// alive states and 1/B when it begins.  1/B takes two rows (Deflator); where it
+// has not moved out of FP32's range yet, at step 0 and on a single rate, one.
 struct SweepPlan {
   int S1, L;
 };
 __host__ __device__ constexpr int sweep_state_row(int F, int S1) { return 2 * F * S1; }
+__host__ __device__ constexpr bool sweep_exponent_row(int N, int S1) { return S1 > 0 && N > 1; }
+// Rows up to and including segment 0's.
+__host__ __device__ constexpr int sweep_first_rows(int N, int F, int S1) {
+  return 2 * F * S1 + N + 1 + (sweep_exponent_row(N, S1) ? 1 : 0);
+}
 // First row of segment i >= 1, which begins at step S1 + i L.
 __host__ __device__ constexpr int sweep_segment_row(int N, int F, int S1, int L, int i) {
-  return 2 * F * S1 + N + 1 + (i - 1) * (N - S1 + 1) - L * (i * (i - 1) / 2);
+  return sweep_first_rows(N, F, S1) + (i - 1) * (N - S1 + 2) - L * (i * (i - 1) / 2);
 }
 // Rows of the checkpoint buffer and of the segment scratch at interval k.
 inline int ckpt_rows(int N, int F, int k) {
   return k == 1 ? N * (N + 1 + 2 * F) : (N + k - 1) / k * (N + 1);
 }
 inline int scratch_rows(int N, int F, int k) { return k == 1 ? 0 : (k < N ? k : N) * (N + 1 + 2 * F); }
-// (With S1 = 0 the segments are at least k long and fit the checkpoint rows:
-// a plan always exists.)
+// (With S1 = 0 the segments are at least k long, and each takes at most N + 1
+// rows: a plan always exists.)
 inline SweepPlan sweep_plan(int N, int F, int k) {
   if (k == 1) return {N, N};
   const int room = ckpt_rows(N, F, k);
@@ -132,11 +138,26 @@ inline SweepPlan sweep_plan(int N, int F, int k) {
   int S1 = N;
   for (; S1 > 0; --S1) {
     const int more = (N - S1 + L - 1) / L;  // segments
-    const int rows = more > 1 ? sweep_segment_row(N, F, S1, L, more) : 2 * F * S1 + N + 1;
+    const int rows =
+        more > 1 ? sweep_segment_row(N, F, S1, L, more) : sweep_first_rows(N, F, S1);
     if (rows <= room) break;
   }
   return {S1, L};
 }
+
+// 1/B of a path as m 2^e, m in [0.5, 1): on a path whose rates run away it falls
+// below FP32's range while the caplets that paid before still count, and the
+// reverse, which multiplies it back step by step, has to come out at theirs.
+struct Deflator {
+  float m = 1.0f;
+  int e = 0;
+  __device__ __forceinline__ void scale(float by) {
+    m *= by;
+    e += __builtin_amdgcn_frexp_expf(m);
+    m = __builtin_amdgcn_frexp_mantf(m);
+  }
+  __device__ __forceinline__ float value() const { return ldexpf(m, e); }
+};
 
 // The step table: for every step s and alive rate r >= s the pair
 // {fixed drift c = -0.5 log2(e) sum_f A(s,r,f)^2, kr of drift_coeff}, steps one
