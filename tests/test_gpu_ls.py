@@ -542,6 +542,30 @@ def test_bermudan_windows_and_blocks_vs_fp64_oracle(torch_cuda, P, N, F, k):
     _check_frozen(torch, w, pr, z, price.item(), greeks, f"P={P} N={N} F={F} k={k}")
 
 
+@pytest.mark.parametrize("P", [300, 40000])
+def test_bermudan_rate_past_fp32_leaves_the_rates_above_it(torch_cuda, P):
+    """A rate that overflows FP32 on part of the paths before the exercise: the
+    Greeks of the rates up to it are NaN, those above stay numbers."""
+    torch = torch_cuda
+    N, r = 20, 8
+    rng = np.random.RandomState(N)
+    f0 = 0.06 + 0.01 * rng.uniform(size=N)
+    f0[r] = 3e38
+    ex = np.array([12, 16], np.int32)
+    w = configs.LMMWorkload("overflow", P, N, 2, 0.5, f0, np.full(N, 0.2),
+                            0.5 * np.arange(1, N + 2), np.full((N, N, 2), 0.1), 0.03, "bermudan",
+                            np.zeros(N * 2, np.uint32), exercise_steps=ex,
+                            basis_shift=np.full((2, 2), 0.05),
+                            basis_scale=np.full((2, 2), 100.0))
+    pr = pipeline.BermudanPricer(w)
+    pr.z.copy_(torch.from_numpy(rng.normal(size=pr.z.numel()).astype(np.float32)))
+    pr.coeffs.zero_()
+    _, g = pr.greeks(checkpoint_every=4)
+    g = g.cpu().numpy().reshape(2, N)
+    assert np.all(np.isnan(g[:, :r + 1])), np.isnan(g)
+    assert np.all(np.isfinite(g[:, r + 1:])), np.isnan(g)
+
+
 # ---------------------------------------------------------------- batched portfolio
 
 def test_batched_portfolio_equals_per_product_calls(torch_cuda):

@@ -334,3 +334,25 @@ def test_greeks_past_an_underflowing_discount_factor(torch_cuda, P, N, F, k):
     assert abs(price / pp.mean() - 1) <= bound
     assert np.all(err[:N] <= bound * size[0])
     assert np.all(err[N:] <= bound * size[1])
+
+
+@pytest.mark.parametrize("P,N,r", [(300, 70, 60), (40000, 20, 9), (300, 40, 30)])
+def test_rate_past_fp32_leaves_the_rates_above_it(torch_cuda, P, N, r):
+    """A rate that overflows FP32 on part of the paths: the price and its own
+    Greeks and those of the rates below are NaN, those above stay numbers (of
+    the size of 1/B, which the rate has taken below 1e-30 on every path)."""
+    rng = np.random.RandomState(N)
+    f0 = 0.04 + 0.01 * rng.uniform(size=N)
+    f0[r] = 3e38
+    A = np.full((N, N, 2), 0.1)
+    w = configs.LMMWorkload("overflow", P, N, 2, 0.5, f0, np.full(N, 0.2),
+                            0.5 * np.arange(1, N + 2), A, 0.05, "caplets",
+                            np.zeros(N * 2, np.uint32), checkpoint_every=8)
+    pr = pipeline.LMMPricer(w)
+    pr.z.copy_(torch_cuda.from_numpy(rng.normal(size=pr.z.numel()).astype(np.float32)))
+    pr.price_kernel(checkpoints=True)
+    pr.greeks_kernel()
+    g = pr.greeks_out.cpu().numpy().reshape(2, N)
+    assert np.isnan(pr.price_out.item())
+    assert np.all(np.isnan(g[:, :r + 1])), np.isnan(g)
+    assert np.all(np.abs(g[:, r + 1:]) < 1e-30), g[:, r + 1:]

@@ -191,15 +191,21 @@ __device__ __forceinline__ void berm_bwd_block(const Model& m, const float* __re
   // past the last path read 0; a wavefront of such lanes does nothing.)
   const int top = __builtin_amdgcn_readfirstlane(static_cast<int>(bp.row(states, N).load()));
   // Lanes past the last path have no exercise step: their adjoints stay zero.
+  NonFinite bad;
   auto seed = [&](int s) {
     if (s == tau)  // the payoff adjoint recorded at exercise
-      for (int r = s; r < N; ++r) lam.set(r, bp.row(lamt, r).load());
+      for (int r = s; r < N; ++r) {
+        float lp = bp.row(lamt, r).load();
+        bad.take(lp, r);
+        lam.set(r, lp);
+      }
   };
   auto fixing = [&](int s, float& lp, float x) {
     // the fixing inside B_tau
     const float xs = start_level(m, s) * fast_exp2(x);
     const float ti = m.taus[s] * fast_rcp(1.0f + m.taus[s] * (xs - m.disp[s]));
     if (s < tau) lp -= ti * V * xs * kLn2;
+    bad.take(lp, s);
   };
   // The steps from S1 on: each segment run again, its sums to scratch, then
   // reversed.
@@ -232,7 +238,7 @@ __device__ __forceinline__ void berm_bwd_block(const Model& m, const float* __re
   }();
   if (!Agent && top <= m.S1) load_states(bp, X, states, 0, N);
   reverse_steps<F, U>(m, bp, min(top, m.S1), 0, ckpt, ctab, X, lam, seed, fixing, vegas);
-  adjoint_sums<BD, Agent>(m, vols, lam, vegas, part, block);
+  adjoint_sums<BD, Agent>(m, vols, lam, vegas, bad, part, block);
 }
 
 // Lanes per block of the single-product kernels (the batched and persistent

@@ -142,6 +142,7 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
   for (int r = 0; r < N; ++r) lam.set(r, 0.0f);
 
   auto row = [&](int r) { return ckpt + static_cast<size_t>(r) * b.P; };
+  NonFinite bad;
   float tail = 0.0f;
   Deflator B;  // after the step being reversed
   auto load_deflator = [&](const float* rows, int r, bool exponent) {
@@ -161,6 +162,7 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
     const float v = caplet_value(fs, tau, m.strike, inv);
     const float dv = caplet_deriv(fs, tau, m.strike, inv);
     lp = fmaf(dv * invB - tau * inv * tail, kLn2 * xs, lp);
+    bad.take(lp, s);
     tail += v * invB;
   };
   auto nothing = [](int) {};
@@ -199,7 +201,7 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
     load_deflator(rows, N, sweep_exponent_row(N, m.S1));
     reverse_steps<F, U>(m, b, m.S1, 0, ckpt, ctab, X, lam, nothing, fixing, vegas);
   }
-  adjoint_sums<BD>(m, vols, lam, vegas, part, blockIdx.x);
+  adjoint_sums<BD>(m, vols, lam, vegas, bad, part, blockIdx.x);
 }
 
 // Few paths: the rates of a path across W lanes (lmm_across.h).  Once the paths

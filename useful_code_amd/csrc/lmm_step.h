@@ -259,7 +259,8 @@ struct GlobalRows {
 // whose B is one in column j mod 16, so column j of tile j / 16 collects 16
 // partial sums (of four lanes each) over all steps.  Two issue slots a rate
 // (the one-hot column and the product), where folding the 64 lanes by DPP and
-// adding to LDS takes about eight.
+// adding to LDS takes about eight.  The terms have to be finite (zero times
+// infinity would reach the other columns): see NonFinite.
 template <int TILES>
 struct VegaSums {
   typedef float f4 __attribute__((ext_vector_type(4)));
@@ -297,6 +298,22 @@ struct VegaSums {
       v += __shfl_xor(v, 32, 64);
       if (lane < 16 && 16 * t + lane < rates) put(16 * t + lane, v);
     }
+  }
+};
+
+// A path's adjoints that are infinite or NaN.  States and what the reverse forms
+// from them are finite; an adjoint becomes infinite or NaN only where it begins,
+// at a fixing or a payoff whose rate has left FP32's range, and from there
+// reaches the rates below.  There it is set to zero and its rate remembered, and
+// the Greeks of that rate and those below are made NaN in the end: the rates
+// above keep theirs.  (Caught at each term instead, the caplet backward took 5%
+// longer.)
+struct NonFinite {
+  int rate = -1;  // the highest of them
+  __device__ __forceinline__ void take(float& lp, int r) {
+    if (fabsf(lp) < __builtin_inff()) return;
+    lp = 0.0f;
+    rate = max(rate, r);
   }
 };
 
@@ -766,12 +783,17 @@ __device__ __forceinline__ void put_partial(double* part, int waves, int w, int 
 
 // A wavefront's sums of the state adjoints and vega terms, as deltas
 // (d/df0_r = log2(e) lam_r / (f0_r + d_r)) and vegas (over sigma_r): columns
-// 0..N-1 and N..2N-1.  Agent: the stores are agent-coherent.
+// 0..N-1 and N..2N-1, NaN where `bad` says so.  Agent: the stores are
+// agent-coherent.
 template <int BD, bool Agent = false, class Lanes, class Vegas>
 __device__ __forceinline__ void adjoint_sums(const Model& m, const float* __restrict__ vols,
-                                             const Lanes& lam, const Vegas& vegas, double* part,
-                                             int block) {
+                                             const Lanes& lam, const Vegas& vegas,
+                                             const NonFinite& bad, double* part, int block) {
   const int N = m.N, lane = threadIdx.x & 63;
+  int nan_to = bad.rate;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) nan_to = max(nan_to, __shfl_xor(nan_to, o, 64));
+  const auto at = [&](int r, double v) { return r <= nan_to ? __builtin_nan("") : v; };
   const int waves = wave_count(m.P), w = wave_index<BD>(block);
   // four rates at a time, so that their butterflies overlap
   for (int r0 = 0; r0 < N; r0 += 4) {
@@ -786,12 +808,12 @@ __device__ __forceinline__ void adjoint_sums(const Model& m, const float* __rest
     for (int i = 0; i < 4; ++i)
       if (lane == i && r0 + i < N)
         put_partial<Agent>(part, waves, w, r0 + i,
-                           v[i] * static_cast<double>(kLog2e) /
-                               static_cast<double>(start_level(m, r0 + i)));
+                           at(r0 + i, v[i] * static_cast<double>(kLog2e) /
+                                          static_cast<double>(start_level(m, r0 + i))));
   }
   vegas.sums(N, [&](int j, double v) {
     const int r = N - 1 - j;
-    put_partial<Agent>(part, waves, w, N + r, v / static_cast<double>(vols[r]));
+    put_partial<Agent>(part, waves, w, N + r, at(r, v / static_cast<double>(vols[r])));
   });
 }
 
