@@ -566,6 +566,27 @@ def test_bermudan_rate_past_fp32_leaves_the_rates_above_it(torch_cuda, P):
     assert np.all(np.isfinite(g[:, r + 1:])), np.isnan(g)
 
 
+def test_bermudan_negative_displaced_rate_is_nan(torch_cuda):
+    """A rate below minus its displacement makes the swap rates and the numeraires
+    after its fixing NaN."""
+    torch = torch_cuda
+    N, P = 12, 300
+    f0 = np.full(N, 0.05)
+    f0[5] = -0.01
+    ex = np.array([2, 8], np.int32)
+    w = configs.LMMWorkload("negative", P, N, 2, 0.5, f0, np.full(N, 0.2),
+                            0.5 * np.arange(1, N + 2), np.full((N, N, 2), 0.1), 0.03, "bermudan",
+                            np.zeros(N * 2, np.uint32), exercise_steps=ex,
+                            basis_shift=np.full((2, 2), 0.05),
+                            basis_scale=np.full((2, 2), 100.0))
+    pr = pipeline.BermudanPricer(w)
+    rng = np.random.RandomState(3)
+    pr.z.copy_(torch.from_numpy(rng.normal(size=pr.z.numel()).astype(np.float32)))
+    pr.paths_kernel()
+    assert torch.isnan(pr.bv.view(2, 2, P)[:, 0]).all()
+    assert torch.isnan(pr.num.view(2, P)[1]).all()
+
+
 # ---------------------------------------------------------------- batched portfolio
 
 def test_batched_portfolio_equals_per_product_calls(torch_cuda):

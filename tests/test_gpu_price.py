@@ -356,3 +356,24 @@ def test_rate_past_fp32_leaves_the_rates_above_it(torch_cuda, P, N, r):
     assert np.isnan(pr.price_out.item())
     assert np.all(np.isnan(g[:, :r + 1])), np.isnan(g)
     assert np.all(np.abs(g[:, r + 1:]) < 1e-30), g[:, r + 1:]
+
+
+@pytest.mark.parametrize("P,N", [(300, 70), (40000, 20), (300, 40)])
+def test_negative_displaced_rate_is_nan(torch_cuda, P, N):
+    """A rate below minus its displacement has no displaced diffusion: its price
+    is NaN and not a number."""
+    rng = np.random.RandomState(N)
+    f0 = 0.04 + 0.01 * rng.uniform(size=N)
+    f0[N // 2] = -0.01
+    w = configs.LMMWorkload("negative", P, N, 2, 0.5, f0, np.full(N, 0.2),
+                            0.5 * np.arange(1, N + 2), np.full((N, N, 2), 0.1), 0.05, "caplets",
+                            np.zeros(N * 2, np.uint32))
+    pr = pipeline.LMMPricer(w)
+    pr.z.copy_(torch_cuda.from_numpy(rng.normal(size=pr.z.numel()).astype(np.float32)))
+    pr.price_kernel()
+    assert np.isnan(pr.price_out.item())
+    w.displacements = np.full(N, 0.015)
+    pr = pipeline.LMMPricer(w)
+    pr.z.copy_(torch_cuda.from_numpy(rng.normal(size=pr.z.numel()).astype(np.float32)))
+    pr.price_kernel()
+    assert pr.price_out.item() > 0.0

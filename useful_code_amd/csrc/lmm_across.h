@@ -135,10 +135,6 @@ __device__ __forceinline__ float dot(const float (&a)[F], const float (&b)[F]) {
   return s;
 }
 
-__device__ __forceinline__ float rate_kr(const Model& m, int r) {
-  return kLn2 * (1.0f / m.taus[r] - m.disp[r]) / (m.f0[r] + m.disp[r]);
-}
-
 // All N steps of the lanes' paths (pc_step, lmm_step.h, with the sums as
 // scans); returns the rate's state as it fixed.  keep(s, x, my, md): the state
 // before step s and the step's sums sum_f a y, sum_f a d.

@@ -231,7 +231,7 @@ __global__ void __launch_bounds__(kAcrossLanes)
   KOO_MODEL_LOCAL;
   __shared__ double red[kAcrossLanes / 64];
   const AcrossLane<W> at(m, blockIdx.x);
-  const float kr = at.rate ? rate_kr(m, at.r) : 1.0f;
+  const float kr = at.rate ? drift_constant(m, at.r) : 1.0f;
   const float x = across_steps<F, W>(m, at, kr, [](int, float, float, float) {});
   block_sum_to(static_cast<double>(across_fixing<W>(m, at, x).v), red, part + blockIdx.x);
 }
@@ -246,7 +246,7 @@ __global__ void __launch_bounds__(kAcrossLanes)
   const AcrossLane<W> at(m, blockIdx.x);
   const int N = m.N, path = static_cast<int>(threadIdx.x) / W, tri = across_tri(N);
   float* mine = lds + static_cast<size_t>(path) * 3 * tri;
-  const float kr = at.rate ? rate_kr(m, at.r) : 1.0f;
+  const float kr = at.rate ? drift_constant(m, at.r) : 1.0f;
   const float xf = across_steps<F, W>(m, at, kr, [&](int s, float x, float my, float md) {
     if (at.rate && at.r >= s) {
       float* o = mine + across_tri_row(N, s) + N - 1 - at.r;
@@ -263,7 +263,7 @@ __global__ void __launch_bounds__(kAcrossLanes)
   const float v = __shfl(fx.v, r, W);
   const float above = __shfl_up(scan_add<W>(rate ? v : 0.0f), 1, W);
   float lam = 0.0f, krr = 1.0f;
-  if (rate) krr = rate_kr(m, r);
+  if (rate) krr = drift_constant(m, r);
   if (at.live) {
     const float tau = m.taus[r], xs = start_level(m, r) * fast_exp2(x);
     const float tail = l ? above : 0.0f;

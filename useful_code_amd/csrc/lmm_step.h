@@ -168,6 +168,16 @@ __host__ __device__ constexpr size_t step_table_floats(int N) {
 // First float of step s.
 __host__ __device__ constexpr int step_table_row(int N, int s) { return s * (2 * N + 1 - s); }
 
+// A rate's f + d at the start, by which 2^x is scaled.
+__device__ __forceinline__ float start_level(const Model& m, int r) { return m.f0[r] + m.disp[r]; }
+
+// kr of drift_coeff; NaN below zero, where a rate has no logarithm: NaN is then
+// what the rate, those above it and the price come to.
+__device__ __forceinline__ float drift_constant(const Model& m, int r) {
+  const float level = start_level(m, r);
+  return level < 0.0f ? __builtin_nanf("") : kLn2 * (1.0f / m.taus[r] - m.disp[r]) / level;
+}
+
 // Entry q < N * N of the square (s, r) = (q / N, q % N) into the table (nothing
 // below the diagonal).  One function for every copy of the table, so an LDS
 // copy and a global one hold the same bits.
@@ -181,7 +191,7 @@ __device__ __forceinline__ void put_step_entry(const Model& m, int q, float* tab
   for (int f = 0; f < F; ++f) c = fmaf(a[f], a[f], c);
   float* t = tab + step_table_row(m.N, s) + 2 * (r - s);
   t[0] = -0.5f * kLog2e * c;
-  t[1] = kLn2 * (1.0f / m.taus[r] - m.disp[r]) / (m.f0[r] + m.disp[r]);
+  t[1] = drift_constant(m, r);
 }
 
 // Every lane of the block takes part; the caller then synchronises.
@@ -189,9 +199,6 @@ template <int F>
 __device__ __forceinline__ void fill_step_table(const Model& m, float* tab) {
   for (int q = threadIdx.x; q < m.N * m.N; q += blockDim.x) put_step_entry<F>(m, q, tab);
 }
-
-// A rate's f + d at the start, by which 2^x is scaled.
-__device__ __forceinline__ float start_level(const Model& m, int r) { return m.f0[r] + m.disp[r]; }
 
 // One value per lane and rate in LDS: lane-minor rows of BD lanes, so a
 // wavefront's access is free of bank conflicts and, BD being a constant, the
