@@ -102,10 +102,11 @@ def test_fused_sobol_bridge_equals_staged(torch_cuda, S, F, P, off):
                                  (128, 2)])
 @pytest.mark.parametrize("P,off", [(1, 0), (63, 0), (64, 63), (65, 62), (129, 1), (20003, 130)])
 def test_fused_sobol_bridge_chunks_and_rows(torch_cuda, S, F, P, off):
-    """Path counts that end inside either chunk of a pair, first points at
-    every place in a group of 64, and step counts around the groups of four
-    dimensions and the two-register split, against the stages; the word behind
-    the last path keeps its value.
+    """Path counts about a 64-path chunk and its end, first points at every place
+    in a group of 64, and step counts around the groups of four dimensions and
+    the two-register split, against the stages; the words behind the last path
+    keep their value.  (At these counts a wavefront has one chunk; runs of them
+    in the next test.)
 
     Both sides form a bridge point with three roundings from points at most
     log2(S) + 1 levels above it (a convex combination, which does not amplify
@@ -125,6 +126,40 @@ def test_fused_sobol_bridge_chunks_and_rows(torch_cuda, S, F, P, off):
     w = staged.double().reshape(S, F, P).cumsum(0).abs().max().item()
     levels = int(np.ceil(np.log2(S))) + 1
     bound = 2 * 2 * 3 * levels * 2.0**-24 * w  # two sides, two points, three roundings a level
+    assert (fused[:D * P] - staged).abs().max().item() <= bound
+
+
+@pytest.mark.parametrize("S", [3, 8, 64, 65, 80, 128])
+@pytest.mark.parametrize("run", [1.5, 2.5, 4.25])
+def test_fused_sobol_bridge_runs_of_chunks(torch_cuda, S, run):
+    """Wavefronts that walk one to five chunks of 64 paths (up to 64 steps in
+    pairs and a last one alone, beyond in pairs): enough factors that the blocks
+    the GPU holds at once are few for each.  `run` chunks for each wavefront that
+    fits, by threads and LDS, so that runs have at least that many.  Points from
+    shortly before 2^20, where a high bit of the Gray code flips inside a run; a
+    path count that ends inside a chunk.  Bound as above."""
+    torch = torch_cuda
+    F, off = min(100, 10200 // S), (1 << 20) - 777  # 10200: the most dimensions
+    groups = (S + 3) // 4
+    lds = S * 128 + groups * 1024 + 12 * groups * 16 + S * 16
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    waves = 4 * max(1, min(8, (160 << 10) // lds) * cus // F)
+    P = int(64 * waves * run) + 37
+    D = S * F
+    dirs = dev(torch, koo.sobol_directions(D))
+    scr = dev(torch, np.random.RandomState(6).randint(0, 2**32, D, dtype=np.uint64).astype(np.uint32))
+    alloc = dev(torch, O.bridge_allocate_diagonal(F, S))
+    print(f"S={S} F={F} P={P}: {waves} wavefronts a factor, run {run}", flush=True)
+    normals = torch.empty(D * P, dtype=torch.float32, device="cuda")
+    koo.sobol_scramble_normal_gpu(P, D, off, dirs, scr, D, normals)
+    staged = torch.empty(D * P, dtype=torch.float32, device="cuda")
+    koo.brownian_bridge_gpu(S, alloc, normals, staged, P, F)
+    fused = torch.full((D * P + 64,), 7.0, dtype=torch.float32, device="cuda")
+    koo.sobol_bridge_gpu(P, off, S, F, dirs, scr, D, alloc, fused)
+    assert bool((fused[D * P:] == 7.0).all())
+    w = staged.reshape(S, F, P).cumsum(0).abs().max().item()
+    levels = int(np.ceil(np.log2(S))) + 1
+    bound = 2 * 2 * 3 * levels * 2.0**-24 * w
     assert (fused[:D * P] - staged).abs().max().item() <= bound
 
 

@@ -12,6 +12,7 @@
 #include <array>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <unordered_map>
 #include <vector>
@@ -180,21 +181,25 @@ __global__ void __launch_bounds__(kBridgeThreads)
 }
 
 // Fused generator on the register bridge, every step count.  Each wavefront
-// walks a contiguous run of 64-path chunks of one factor, two at a time.  With
-// n = G + l (G a multiple of 64, l < 64) the Gray code splits, gray(n) =
-// gray(G) ^ gray(l), so the scrambled Sobol integer is X(G) ^ T(l) with X(G) =
-// scrambler ^ XOR of the direction numbers over the set bits of gray(G).  A
-// lane's l is the same in every chunk; T(l) sits in LDS.  X(G) is kept one
-// dimension per lane (two registers beyond 64 steps): from G = 64m to 64(m+1)
-// gray flips bits 5 and 6 + ctz(m+1), so advancing costs two XORs.  A chunk
-// (lanes at n = 64c + off1 + lane) spans G and G + 64, two chunks three values:
-// the wavefront writes them to rows of its own in LDS, from which each lane
-// reads those of its group, four dimensions to a read.
+// walks a contiguous run of 64-path chunks of one factor, two at a time and an
+// odd last one alone.  With n = G + l (G a multiple of 64, l < 64) the Gray code
+// splits, gray(n) = gray(G) ^ gray(l), so the scrambled Sobol integer is
+// X(G) ^ T(l) with X(G) = scrambler ^ XOR of the direction numbers over the set
+// bits of gray(G).  A lane's l is the same in every chunk; T(l) sits in LDS.
+// X(G) is kept one dimension per lane (two registers beyond 64 steps): from
+// G = 64m to 64(m+1) gray flips bits 5 and 6 + ctz(m+1), so advancing costs two
+// XORs.  A chunk (lanes at n = 64c + off1 + lane) spans G and G + 64, two chunks
+// three values: the wavefront writes them to rows of its own in LDS, from which
+// each lane reads those of its group, four dimensions to a read.
 // Bound by the vector instructions, 26 a point, most of them the quantile; 43
 // with one chunk at a time, X(G) read out by readlane and 64-bit store
 // addresses.  2^20 paths: 40 steps x 5 factors 232 -> 175 us, 64 x 32 2.59 ->
 // 1.93 ms (4.4 TB/s of stores).  Step counts above 64 kept the points in LDS
 // and walked the bits of the Gray code for each: 2^17 x 80 x 2 238 -> 43 us.
+// Few paths leave a wavefront one chunk: in a pair half of that is for nothing
+// (65536 paths x 32 x 5 24.6 us, 18.4 alone; 4096 x 40 x 8 12.2, 10.4).  Beyond
+// kRegSteps the body for one chunk is left out: those kernels take most of this
+// file's compile time.
 template <int S>
 __global__ void __launch_bounds__(kBridgeThreads)
     k_sobol_bridge_reg(const BridgeTables T, int factors, int paths, uint32_t off1,
@@ -266,47 +271,65 @@ __global__ void __launch_bounds__(kBridgeThreads)
   // the lane's own group of the first chunk; of the second, a row further
   const u32x4* xl = xrows + wave * 3 * Q + (r + static_cast<uint32_t>(lane) >= 64u ? Q : 0);
   // the wavefront's paths as a buffer per step: stores past its last path are
-  // dropped (the second chunk of the last pair, lanes past the last path)
+  // dropped (lanes past the last path; the second chunk of a last pair)
   const int bytes = 4 * min(paths - c0 * 64, (c1 - c0) * 64);
   float* first = out + static_cast<size_t>(f) * paths + static_cast<size_t>(c0) * 64;
-  for (int c = c0; c < c1; c += 2) {
+  // `chunks`: two at a time, or one
+  auto walk = [&](int c, auto chunks) {
+    constexpr bool two = decltype(chunks)::value == 2;
+    using V = typename std::conditional<two, f32x2, float>::type;
     // a wavefront's LDS operations keep their order, and the rows are its own
     put(0);
     advance();
     put(1);
-    advance();
-    put(2);
+    if constexpr (two) {
+      advance();
+      put(2);
+    }
     __builtin_amdgcn_wave_barrier();
     u32x4 t, a, b;
     auto z = [&](int i) {
       if (i % 4 == 0) {
         t = tl[(i >> 2) * 64];
         a = xl[i >> 2];
-        b = xl[Q + (i >> 2)];
+        if constexpr (two) b = xl[Q + (i >> 2)];
       }
-      return f32x2{invnorm_u32(t[i & 3] ^ a[i & 3]), invnorm_u32(t[i & 3] ^ b[i & 3])};
+      const float first = invnorm_u32(t[i & 3] ^ a[i & 3]);
+      if constexpr (two) return f32x2{first, invnorm_u32(t[i & 3] ^ b[i & 3])};
+      else return first;
     };
     // The weights come from LDS at an offset, and the rows of the steps from a
     // stride, made opaque each time (a zero from s_mov), so that their reads
     // and sums stay in the loop.
     int zero;
     asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
-    f32x2 w[S];
+    V w[S];
     const LdsWeights wt{wts, zero};
     bridge_points<S>(w, wt, z, std::make_integer_sequence<int, S>{});
     const size_t stride = (static_cast<size_t>(factors) + zero) * paths;
     float* row = first;
     const int byte = (c - c0) * 256 + lane * 4;
-    f32x2 prev = {0.0f, 0.0f};
+    V prev{};
 #pragma unroll
     for (int i = 0; i < S; ++i, row += stride) {
       const auto rs = __builtin_amdgcn_make_buffer_rsrc(row, 0, bytes, 0x00027000);
-      const f32x2 dz = w[i] - prev;
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz.x), rs, byte, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz.y), rs, byte + 256, 0, 0);
+      const V dz = w[i] - prev;
+      if constexpr (two) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz.x), rs, byte, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz.y), rs, byte + 256, 0, 0);
+      } else {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz), rs, byte, 0, 0);
+      }
       prev = w[i];
     }
     __builtin_amdgcn_wave_barrier();
+  };
+  int c = c0;
+  if constexpr (S <= kRegSteps) {
+    for (; c + 1 < c1; c += 2) walk(c, std::integral_constant<int, 2>{});
+    if (c < c1) walk(c, std::integral_constant<int, 1>{});
+  } else {
+    for (; c < c1; c += 2) walk(c, std::integral_constant<int, 2>{});
   }
 }
 
