@@ -745,9 +745,10 @@ typedef struct koo_berm_product {
   double* greeks_out; /* device */
 } koo_berm_product;
 
-/* Products are grouped by rate count into up to 4 classes (<= 16, 24, 32
- * and more rates), one launch each, so a block reserves LDS for its class's
- * largest curve rather than the portfolio's. */
+/* Products are grouped by rate count into up to 4 classes (<= 16, 24, 40 and
+ * more rates; the LS launches <= 16, 24, 32 and more), one launch each, so a
+ * block reserves LDS for its class's largest curve rather than the
+ * portfolio's. */
 typedef struct koo_portfolio_plan {
   int products, blocks, max_rates; /* the 256-lane kernels */
   int ls_blocks, max_ex;           /* the 1024-lane LS kernels (LS batch only) */

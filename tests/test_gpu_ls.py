@@ -714,6 +714,40 @@ def test_portfolio_longest_curves_equal_single_calls(torch_cuda, persistent):
         assert np.isfinite(p2) and fp.item() == p2 and np.array_equal(fg.cpu().numpy(), g), j
 
 
+@pytest.mark.parametrize("persistent", [False, True])
+@pytest.mark.parametrize("rates,paths", [((16, 17, 24, 25, 40, 41), 4096 + 257)])
+def test_portfolio_classes_equal_single_calls(torch_cuda, persistent, rates, paths):
+    """Curves on both sides of every launch class of the batched kernels (beyond 40
+    rates the backward runs single-wavefront blocks; 257 paths past a multiple
+    leave some of them without a path): bit for bit the single-product frozen calls on the same variates and
+    coefficients."""
+    torch = torch_cuda
+    prods = []
+    for j, N in enumerate(rates):
+        rng = np.random.RandomState(10 * N + j)
+        F = 1 + (2 * j + 1) % min(5, N)
+        f0 = 0.05 + rng.uniform(-0.005, 0.005, N)
+        times = 0.5 * np.arange(1, N + 2)
+        A = koo.flat_vol_pseudo_roots(times, times[:N], np.full(N, 0.2), F, 0.0, 0.1)
+        ex = np.unique(np.linspace(0, max(N - 2, 0), 5).astype(np.int32))
+        prods.append(configs.LMMWorkload(
+            f"bermudan_{N}x{F}", paths, N, F, 0.5, f0, np.full(N, 0.2), times, A, 0.05, "bermudan",
+            rng.randint(0, 2**32, N * F, dtype=np.uint64).astype(np.uint32), exercise_steps=ex,
+            basis_shift=np.full((ex.size, 2), 0.05), basis_scale=np.full((ex.size, 2), 100.0)))
+    pf = pipeline.PortfolioPricer(prods, checkpoint_every=4, n_streams=2, persistent=persistent)
+    assert pf.batched and pf.persistent == persistent
+    print(f"portfolio of {rates} rates, persistent={persistent}", flush=True)
+    pf.run(capture=False)
+    torch.cuda.synchronize()
+    got = pf.results()
+    for j, pr in enumerate(pf.pricers):
+        _, p2, g = got[j]
+        fp, fg = pr.greeks(checkpoint_every=4)
+        torch.cuda.synchronize()
+        assert np.isfinite(p2) and fp.item() == p2, rates[j]
+        assert np.all(np.isfinite(g)) and np.array_equal(fg.cpu().numpy(), g), rates[j]
+
+
 @pytest.mark.parametrize("paths", [257, 1 << 16, (1 << 16) + 300])
 def test_persistent_teams_of_a_block_per_chunk(torch_cuda, paths):
     """Teams of as many blocks as the product has 256-path chunks, up to 256

@@ -123,26 +123,41 @@ __global__ void __launch_bounds__(kAdjLanes)
   }
 }
 
-__global__ void __launch_bounds__(kAdjLanes) __attribute__((amdgpu_waves_per_eu(2, 4)))
+// BD = kAdjLanes, or single-wavefront blocks, four to each of the plan's blocks,
+// for curves whose 2 N rows of kAdjLanes leave one block a CU (kAdjRates < N, 84
+// to 92 KB).  Ten products of 41 to 45 rates, 65536 paths and k = 1: 2337 us in
+// blocks of kAdjLanes, 1781 in wavefronts.
+template <int BD, int W0, int W1>
+__global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W0, W1)))
     k_berm_bwd_batch(const BermItem* __restrict__ items, int n, int block_offset) {
-  const int block = blockIdx.x + block_offset;
+  constexpr int kParts = kAdjLanes / BD;
+  const int block = blockIdx.x / kParts + block_offset;
   const BermItem& it = find_item(items, n, block);
   const Model m = item_model(it);
-  const int blk = block - it.block0;
+  const int blk = (block - it.block0) * kParts + blockIdx.x % kParts;
+  if (blk * BD >= m.P) return;
   switch (it.F) {
-#define KOO_CASE(F)                                                                            \
-  case F:                                                                                      \
-    if (it.N >= kShortCurve)                                                                   \
-      berm_bwd_block<F, kAdjLanes, kWindow<F>>(m, gmem(it.vols), gmem(it.tab), gmem(it.ckpt), gmem(it.lamt),       \
-                                         gmem(it.tau), gmem(it.vout), gmem(it.scratch),        \
-                                         gmem(it.part_bwd), blk);                              \
-    else                                                                                       \
-      berm_bwd_block<F, kAdjLanes, 1>(m, gmem(it.vols), gmem(it.tab), gmem(it.ckpt), gmem(it.lamt), gmem(it.tau),  \
-                                gmem(it.vout), gmem(it.scratch), gmem(it.part_bwd), blk);      \
+#define KOO_CASE(F)                                                                               \
+  case F:                                                                                         \
+    if (BD != kAdjLanes || it.N >= kShortCurve)                                                   \
+      berm_bwd_block<F, BD, kWindow<F>>(m, gmem(it.vols), gmem(it.tab), gmem(it.ckpt),            \
+                                        gmem(it.lamt), gmem(it.tau), gmem(it.vout),               \
+                                        gmem(it.scratch), gmem(it.part_bwd), blk);                \
+    else                                                                                          \
+      berm_bwd_block<F, BD, 1>(m, gmem(it.vols), gmem(it.tab), gmem(it.ckpt), gmem(it.lamt),      \
+                               gmem(it.tau), gmem(it.vout), gmem(it.scratch), gmem(it.part_bwd),  \
+                               blk);                                                              \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
 #undef KOO_CASE
   }
+}
+
+// Launch class of a product: curves up to 16, 24 and kAdjRates rates and longer
+// ones, each with LDS for the longest curve of its class (five, three, two
+// blocks a CU in the backward; the class beyond: single wavefronts).
+int adj_class(int rates) {
+  return rates <= 16 ? 0 : (rates <= 24 ? 1 : (rates <= kAdjRates ? 2 : 3));
 }
 
 // Per product: price (column 0 of the forward partials) and the 2N Greeks.
@@ -355,7 +370,7 @@ extern "C" int bermudan_portfolio_prepare(int n_products, const koo_berm_product
   for (int i = 0; i < n_products; ++i) order[i] = i;
   // rate class first (one launch per class), then most expensive first
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-    const int ca = rate_class(items[a].N), cb = rate_class(items[b].N);
+    const int ca = adj_class(items[a].N), cb = adj_class(items[b].N);
     return ca != cb ? ca < cb : cost[a] > cost[b];
   });
   std::vector<BermItem> sorted(n_products);
@@ -364,8 +379,8 @@ extern "C" int bermudan_portfolio_prepare(int n_products, const koo_berm_product
   for (int i = 0; i < n_products; ++i) {
     sorted[i] = items[order[i]];
     sorted[i].block0 = static_cast<int>(block0);
-    const int c = rate_class(sorted[i].N);
-    if (plan->classes == 0 || rate_class(sorted[i - 1].N) != c) {
+    const int c = adj_class(sorted[i].N);
+    if (plan->classes == 0 || adj_class(sorted[i - 1].N) != c) {
       plan->class_first_block[plan->classes] = static_cast<int>(block0);
       ++plan->classes;
     }
@@ -401,11 +416,14 @@ static int portfolio_launch(const char* who, bool fwd, const koo_portfolio_plan*
     if (nc < 1 || nc > N || nb < 1 || b0 < 0 || b0 + nb > plan->blocks)
       return set_error(KOO_ERR_INVALID, "%s: bad plan class %d", who, c);
     if (fwd)
-      hipLaunchKernelGGL(k_berm_fwd_batch, dim3(nb), dim3(kAdjLanes), rows_lds(nc, nc, kAdjLanes, false), st, items,
-                         plan->products, b0);
+      hipLaunchKernelGGL(k_berm_fwd_batch, dim3(nb), dim3(kAdjLanes),
+                         rows_lds(nc, nc, kAdjLanes, false), st, items, plan->products, b0);
+    else if (nc > kAdjRates)
+      hipLaunchKernelGGL((k_berm_bwd_batch<64, 2, 2>), dim3(kAdjLanes / 64 * nb), dim3(64),
+                         rows_lds(nc, 2 * nc, 64, false), st, items, plan->products, b0);
     else
-      hipLaunchKernelGGL(k_berm_bwd_batch, dim3(nb), dim3(kAdjLanes), rows_lds(nc, 2 * nc, kAdjLanes, false), st, items,
-                         plan->products, b0);
+      hipLaunchKernelGGL((k_berm_bwd_batch<kAdjLanes, 2, 4>), dim3(nb), dim3(kAdjLanes),
+                         rows_lds(nc, 2 * nc, kAdjLanes, false), st, items, plan->products, b0);
   }
   hipLaunchKernelGGL(k_berm_finalize_batch, dim3(fwd ? 1 : 2 * N, plan->products), dim3(256), 0,
                      st, items, fwd ? 1 : 0);

@@ -318,9 +318,9 @@ struct VegaSums {
 struct NonFinite {
   int rate = -1;  // the highest of them
   __device__ __forceinline__ void take(float& lp, int r) {
-    if (fabsf(lp) < __builtin_inff()) return;
-    lp = 0.0f;
-    rate = max(rate, r);
+    const bool finite = fabsf(lp) < __builtin_inff();
+    lp = finite ? lp : 0.0f;
+    rate = finite ? rate : max(rate, r);
   }
 };
 
@@ -869,8 +869,8 @@ __device__ __forceinline__ int find_block_owner(const Item* items, int n, int bl
   return lo;
 }
 
-// Rate-count class of a product in a batched portfolio (launches are per
-// class so LDS is reserved for the class's largest curve).
+// Rate-count class of a product in the batched LS launches (a launch per class,
+// so LDS is reserved for the class's largest curve).
 inline int rate_class(int rates) { return rates <= 16 ? 0 : (rates <= 24 ? 1 : (rates <= 32 ? 2 : 3)); }
 
 // out[col] = (sum_b part[b*ncols + col]) * scale, compensated; called by a
