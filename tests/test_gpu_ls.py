@@ -715,11 +715,13 @@ def test_portfolio_longest_curves_equal_single_calls(torch_cuda, persistent):
 
 
 @pytest.mark.parametrize("persistent", [False, True])
-@pytest.mark.parametrize("rates,paths", [((16, 17, 24, 25, 40, 41), 4096 + 257)])
+@pytest.mark.parametrize("rates,paths", [((2, 3, 4, 3), 1000),
+                                         ((16, 17, 24, 25, 40, 41), 4096 + 257)])
 def test_portfolio_classes_equal_single_calls(torch_cuda, persistent, rates, paths):
-    """Curves on both sides of every launch class of the batched kernels (beyond 40
-    rates the backward runs single-wavefront blocks; 257 paths past a multiple
-    leave some of them without a path): bit for bit the single-product frozen calls on the same variates and
+    """Curves below the step loops' window, and on both sides of every launch
+    class of the batched kernels (beyond 40 rates the backward runs
+    single-wavefront blocks; 257 paths past a multiple leave some of them without
+    a path): bit for bit the single-product frozen calls on the same variates and
     coefficients."""
     torch = torch_cuda
     prods = []

@@ -567,7 +567,7 @@ __device__ __forceinline__ void reverse_fetch(Ahead<F, U>& h, const Model& m, in
 // descending),
 //   D_f += 0.5 lp a_f, q = sum a D;   xhb = lp + q dGh/dx
 //   Y_f += xhb a_f,    p = sum a Y;   lam = xhb + (p - q) dG/dx
-//   w = 0.5 lp sum a d + (Gh - G) q + G p + xhb (sum a y + 2 c).
+//   w = 0.5 lp sum a d + Gh q + G (p - q) + xhb (sum a y + 2 c).
 template <int F, int U, class Tab, class States, class Lanes, class Fixing, class Vegas>
 __device__ __forceinline__ void reverse_step(const Model& m, int s, Tab tab, Ahead<F, U>& h,
                                              const States& X, const Lanes& lam, float (&y)[F],
@@ -614,7 +614,9 @@ __device__ __forceinline__ void reverse_step(const Model& m, int s, Tab tab, Ahe
       y[f] = fmaf(-G, v.a[u][f], y[f]);
       d[f] = fmaf(-g, v.a[u][f], d[f]);
     }
-    return fmaf(xhb, mc + c, fmaf(lh, md, uh + ug));
+    // uh + ug, as one multiply-add written out: left to the compiler, the single,
+    // batched and persistent kernels would not all round it alike
+    return fmaf(xhb, mc + c, fmaf(lh, md, fmaf(G, p - q, uh)));
   };
   Ahead<F, U> g;
   auto fetch = [&](Ahead<F, U>& to, int r) {
