@@ -25,21 +25,22 @@ namespace {
 
 using namespace lmm;
 
-template <int F, int BD, int U>
+template <int F, int BD, int U, bool Own>
 __global__ void __launch_bounds__(BD)
     k_berm_fwd(KOO_MODEL_PARAMS, const BermArgs b, const double* __restrict__ coeffs,
-               const float* __restrict__ tab, float* __restrict__ ckpt, float* __restrict__ lamt, int* __restrict__ tau_out,
-               float* __restrict__ vout, double* __restrict__ part) {
+               float* __restrict__ tab, float* __restrict__ ckpt, float* __restrict__ lamt,
+               int* __restrict__ tau_out, float* __restrict__ vout, double* __restrict__ part) {
   KOO_MODEL_LOCAL;
-  berm_fwd_block<F, BD, U>(m, b, CoefGlobal{coeffs}, tab, ckpt, lamt, tau_out, vout, part, blockIdx.x);
+  berm_fwd_block<F, BD, U, false, Own>(m, b, CoefGlobal{coeffs}, tab, ckpt, lamt, tau_out, vout,
+                                       part, blockIdx.x);
 }
 
 template <int F, int BD, int U, int W>
 __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
     k_berm_bwd(KOO_MODEL_PARAMS, const float* __restrict__ vols, const float* __restrict__ tab,
-               float* __restrict__ ckpt, const float* __restrict__ lamt, const int* __restrict__ tau_in,
-               const float* __restrict__ vin, float* __restrict__ scratch,
-               double* __restrict__ part) {
+               float* __restrict__ ckpt, const float* __restrict__ lamt,
+               const int* __restrict__ tau_in, const float* __restrict__ vin,
+               float* __restrict__ scratch, double* __restrict__ part) {
   KOO_MODEL_LOCAL;
   berm_bwd_block<F, BD, U>(m, vols, tab, ckpt, lamt, tau_in, vin, scratch, part, blockIdx.x);
 }
@@ -110,13 +111,14 @@ __global__ void __launch_bounds__(kAdjLanes)
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
     if (it.N >= kShortCurve)                                                                   \
-      berm_fwd_block<F, kAdjLanes, kWindow<F>>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.tab), gmem(it.ckpt),  \
-                                         gmem(it.lamt), gmem(it.tau), gmem(it.vout),           \
-                                         gmem(it.part_fwd), blk);                              \
+      berm_fwd_block<F, kAdjLanes, kWindow<F>>(m, it.b, CoefGlobal{gmem(it.coeffs)},           \
+                                               gmem(it.tab), gmem(it.ckpt), gmem(it.lamt),     \
+                                               gmem(it.tau), gmem(it.vout),                    \
+                                               gmem(it.part_fwd), blk);                        \
     else                                                                                       \
-      berm_fwd_block<F, kAdjLanes, 1>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.tab), gmem(it.ckpt),           \
-                                gmem(it.lamt), gmem(it.tau), gmem(it.vout), gmem(it.part_fwd), \
-                                blk);                                                          \
+      berm_fwd_block<F, kAdjLanes, 1>(m, it.b, CoefGlobal{gmem(it.coeffs)}, gmem(it.tab),      \
+                                      gmem(it.ckpt), gmem(it.lamt), gmem(it.tau),              \
+                                      gmem(it.vout), gmem(it.part_fwd), blk);                  \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5)
 #undef KOO_CASE
@@ -222,27 +224,31 @@ extern "C" int bermudan_frozen_fwd(int paths, int rates, int factors, int checkp
   float* vout = path_buffers + static_cast<size_t>(rates + 1) * P;
   const int threads = fwd_lanes(paths, rates);
   const int blocks = (paths + threads - 1) / threads;
-  const size_t lds = rows_lds(rates, rates, threads, false);
+  // a short curve's blocks form the step table (no launch before them)
+  const bool own = rates < kShortCurve;
+  const size_t lds = rows_lds(rates, rates, threads, own);
   const SweepPlan plan = sweep_plan(rates, factors, checkpoint_every);
   float* tab =
       checkpoints + static_cast<size_t>(ckpt_rows(rates, factors, checkpoint_every)) * paths;
   hipStream_t st = as_stream(stream);
   switch (factors) {
-#define KOO_FWD(F, BD, U)                                                                      \
-  hipLaunchKernelGGL((k_berm_fwd<F, BD, U>), dim3(blocks), dim3(BD), lds, st, variates,           \
+#define KOO_FWD(F, BD, U, Own)                                                                 \
+  hipLaunchKernelGGL((k_berm_fwd<F, BD, U, Own>), dim3(blocks), dim3(BD), lds, st, variates,   \
                      initial_rates, taus, displacements, pseudo_roots, strike, paths, rates,   \
-                     plan.S1, plan.L, b, coefficients, tab, checkpoints, lamt, tau, vout, partials)
+                     plan.S1, plan.L, b, coefficients, tab, checkpoints, lamt, tau, vout,      \
+                     partials)
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
-    hipLaunchKernelGGL(k_berm_step_table<F>, dim3((rates * rates + 255) / 256), dim3(256), 0,  \
-                       st, variates, initial_rates, taus, displacements, pseudo_roots, strike, \
-                       paths, rates, plan.S1, plan.L, tab);                                    \
-    if (threads == 64)                                                                         \
-      KOO_FWD(F, 64, kWindow<F>);                                                               \
-    else if (rates >= kShortCurve)                                                             \
-      KOO_FWD(F, kAdjLanes, kWindow<F>);                                                         \
+    if (!own)                                                                                  \
+      hipLaunchKernelGGL(k_berm_step_table<F>, dim3((rates * rates + 255) / 256), dim3(256),   \
+                         0, st, variates, initial_rates, taus, displacements, pseudo_roots,    \
+                         strike, paths, rates, plan.S1, plan.L, tab);                          \
+    if (own)                                                                                   \
+      KOO_FWD(F, kAdjLanes, 1, true);                                                          \
+    else if (threads == 64)                                                                    \
+      KOO_FWD(F, 64, kWindow<F>, false);                                                       \
     else                                                                                       \
-      KOO_FWD(F, kAdjLanes, 1);                                                                  \
+      KOO_FWD(F, kAdjLanes, kWindow<F>, false);                                                \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5) KOO_CASE(6) KOO_CASE(7)
     KOO_CASE(8)
@@ -278,10 +284,10 @@ extern "C" int bermudan_frozen_bwd(int paths, int rates, int factors, int checkp
   hipStream_t st = as_stream(stream);
   switch (factors) {
 #define KOO_BWD(F, BD, U, W)                                                                     \
-  hipLaunchKernelGGL((k_berm_bwd<F, BD, U, W>), dim3(blocks), dim3(BD), lds, st, variates,           \
+  hipLaunchKernelGGL((k_berm_bwd<F, BD, U, W>), dim3(blocks), dim3(BD), lds, st, variates,     \
                      initial_rates, taus, displacements, pseudo_roots, strike, paths, rates,   \
-                     plan.S1, plan.L, vols, tab, const_cast<float*>(checkpoints), lamt, tau, vin, segment_scratch,     \
-                     partials)
+                     plan.S1, plan.L, vols, tab, const_cast<float*>(checkpoints), lamt, tau,   \
+                     vin, segment_scratch, partials)
 #define KOO_CASE(F)                                                                            \
   case F:                                                                                      \
     if (rates < kShortCurve)                                                                   \

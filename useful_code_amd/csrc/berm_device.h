@@ -30,13 +30,14 @@ struct CoefTable {
 };
 
 // One block of the forward: paths [block * BD, ...) of product m.  tab: the step
-// table (scalar loads); the persistent kernel (Agent) keeps its own in LDS
-// behind the states and stores the block's price partial agent-coherent.
+// table (scalar loads).  Own: the blocks form one in LDS behind the states, and
+// the first leaves it at `tab` if there is one.  Agent (the persistent kernel):
+// the block's price partial is stored agent-coherent.
 // The checkpoint rows are SweepPlan's, the 1/B row of the states at S1 holding
 // the number of steps the wavefront ran (as float) in its place.
-template <int F, int BD, int U, bool Agent = false, class Coef>
+template <int F, int BD, int U, bool Agent = false, bool Own = Agent, class Coef>
 __device__ __forceinline__ void berm_fwd_block(const Model& m, const BermArgs& b, const Coef& cf,
-                                               const float* __restrict__ tab,
+                                               float* __restrict__ tab,
                                                float* __restrict__ ckpt, float* __restrict__ lamt,
                                                int* __restrict__ tau_out,
                                                float* __restrict__ vout,
@@ -48,11 +49,13 @@ __device__ __forceinline__ void berm_fwd_block(const Model& m, const BermArgs& b
   const size_t p = bp.p0 + threadIdx.x;
   const LaneRows<BD> X{lds + threadIdx.x};
   float* ltab = lds + static_cast<size_t>(N) * BD;
-  if (Agent) fill_step_table<F>(m, ltab);
+  if (Own) fill_step_table<F>(m, ltab);
   for (int r = 0; r < N; ++r) X.set(r, 0.0f);
-  if (Agent) __syncthreads();
+  if (Own) __syncthreads();
+  if (Own && tab && block == 0)
+    for (int i = threadIdx.x; i < static_cast<int>(step_table_floats(N)); i += BD) tab[i] = ltab[i];
   const auto ctab = [&]() {
-    if constexpr (Agent) return static_cast<const float*>(ltab);
+    if constexpr (Own) return static_cast<const float*>(ltab);
     else return cmem(tab);
   }();
   float invB = 1.0f, V = 0.0f;

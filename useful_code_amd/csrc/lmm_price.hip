@@ -64,17 +64,28 @@ __global__ void __launch_bounds__(256) k_step_table(KOO_MODEL_PARAMS, float* __r
 }
 
 // Forward: the state of every rate in LDS, the uniform data of a step through
-// scalar registers (pc_step): 4F + 10 vector instructions a rate update.
-template <int F, int BD, int U>
+// scalar registers (pc_step): 4F + 10 vector instructions a rate update.  Own:
+// the blocks form the step table in LDS and the first leaves it at `tab`.
+template <int F, int BD, int U, bool Own>
 __global__ void __launch_bounds__(BD)
-    k_price_fwd(KOO_MODEL_PARAMS, const float* __restrict__ tab, float* __restrict__ ckpt,
+    k_price_fwd(KOO_MODEL_PARAMS, float* __restrict__ tab, float* __restrict__ ckpt,
                 double* __restrict__ part) {
   KOO_MODEL_LOCAL;
   extern __shared__ float lds[];
   const BlockPaths b(m.P, blockIdx.x, BD);
   const LaneRows<BD> X{lds + threadIdx.x};
   const int N = m.N;
-  const c_cfloat ctab = cmem(tab);
+  const auto ctab = [&]() {
+    if constexpr (Own) return static_cast<const float*>(lds + N * BD);
+    else return cmem(tab);
+  }();
+  if (Own) {
+    fill_step_table<F>(m, lds + N * BD);
+    __syncthreads();
+    if (ckpt && blockIdx.x == 0)
+      for (int i = threadIdx.x; i < static_cast<int>(step_table_floats(N)); i += BD)
+        tab[i] = lds[N * BD + i];
+  }
   for (int r = 0; r < N; ++r) X.set(r, 0.0f);
   Deflator B;
   float v = 0.0f, vc = 0.0f;
@@ -319,6 +330,11 @@ int fwd_lanes(int paths, int N) {
 int bwd_lanes(int paths, int N) {
   return N >= kShortCurve && N <= kAdjRates && paths >= 32768 ? kAdjLanes : 64;
 }
+// Whether the forward's blocks form the step table, and not a launch before it:
+// on short curves the launch is longer than what its scalar loads save (price of
+// 16448 paths, 5 factors x 4 rates 14.1 us for 11.4, 8 factors x 8 rates 14.4 for
+// 12.7; at 12 rates the table has 144 entries a block to form).
+bool own_table(int rates, int lanes) { return rates < kShortCurve || (rates <= 8 && lanes == 64); }
 size_t rows_lds(int rows, int lanes) { return sizeof(float) * static_cast<size_t>(rows) * lanes; }
 // Doubles of the partials before the step table of a forward without
 // checkpoints.
@@ -393,7 +409,9 @@ extern "C" int lmm_price_fwd(int paths, int rates, int factors, int checkpoint_e
           strike, paths, rates, plan.S1, plan.L};
   const int threads = fwd_lanes(paths, rates);
   const int blocks = (paths + threads - 1) / threads;
-  const size_t lds = rows_lds(rates, threads);
+  const bool own = own_table(rates, threads);
+  const size_t lds =
+      rows_lds(rates, threads) + (own ? sizeof(float) * step_table_floats(rates) : 0);
   float* tab = checkpoints
                    ? checkpoints + static_cast<size_t>(ckpt_rows(rates, factors, checkpoint_every)) *
                                        paths
@@ -411,19 +429,23 @@ extern "C" int lmm_price_fwd(int paths, int rates, int factors, int checkpoint_e
     return check_launch("lmm_price_fwd");
   }
   switch (factors) {
-#define KOO_FWD(F, BD, U)                                                                        \
-  hipLaunchKernelGGL((k_price_fwd<F, BD, U>), dim3(blocks), dim3(BD), lds, st, m.z, m.f0,        \
-                     m.taus, m.disp, m.A, m.strike, m.P, m.N, m.S1, m.L, tab, checkpoints, partials)
+#define KOO_FWD(F, BD, U, Own)                                                                   \
+  hipLaunchKernelGGL((k_price_fwd<F, BD, U, Own>), dim3(blocks), dim3(BD), lds, st, m.z, m.f0,   \
+                     m.taus, m.disp, m.A, m.strike, m.P, m.N, m.S1, m.L, tab, checkpoints,       \
+                     partials)
 #define KOO_CASE(F)                                                                              \
   case F:                                                                                        \
-    hipLaunchKernelGGL(k_step_table<F>, dim3((rates * rates + 255) / 256), dim3(256), 0, st,     \
-                       m.z, m.f0, m.taus, m.disp, m.A, m.strike, m.P, m.N, m.S1, m.L, tab);            \
-    if (threads == kAdjLanes)                                                                          \
-      KOO_FWD(F, kAdjLanes, kWindow<F>);                                                               \
-    else if (rates >= kShortCurve)                                                               \
-      KOO_FWD(F, 64, kWindow<F>);                                                                \
+    if (!own)                                                                                    \
+      hipLaunchKernelGGL(k_step_table<F>, dim3((rates * rates + 255) / 256), dim3(256), 0, st,   \
+                         m.z, m.f0, m.taus, m.disp, m.A, m.strike, m.P, m.N, m.S1, m.L, tab);    \
+    if (threads == kAdjLanes)                                                                    \
+      KOO_FWD(F, kAdjLanes, kWindow<F>, false);                                                  \
+    else if (rates < kShortCurve)                                                                \
+      KOO_FWD(F, 64, 1, true);                                                                   \
+    else if (own)                                                                                \
+      KOO_FWD(F, 64, kWindow<F>, true);                                                          \
     else                                                                                         \
-      KOO_FWD(F, 64, 1);                                                                         \
+      KOO_FWD(F, 64, kWindow<F>, false);                                                         \
     break;
     KOO_CASE(1) KOO_CASE(2) KOO_CASE(3) KOO_CASE(4) KOO_CASE(5) KOO_CASE(6) KOO_CASE(7)
     KOO_CASE(8)
