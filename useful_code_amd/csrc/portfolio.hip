@@ -365,18 +365,20 @@ size_t pf_phase_lds(int N) {
   return (m + 15) & ~static_cast<size_t>(15);
 }
 
-// Work of a product in rate updates per path, weighted by the per-update
-// cost of each phase (generation per variate, evolution to the last exercise
-// date in the path-quantity and forward kernels, the reverse sweep with its
-// recompute, the LS rounds): the team sizes are proportional to it.
+// Work of a product, to which the team sizes are proportional: the time of 256
+// paths in us, as measured for products of 8 to 40 rates, 2 to 5 factors and 4 to
+// 16 dates in full teams (fitted to their block times, which it meets to 20%; the
+// checkpoint interval makes no difference): the sweeps per rate update up to the
+// last exercise date, the generation per variate, the LS rounds per date.  Sixty
+// products of 10 to 40 rates x 20000 paths: 4.12 ms; 6.00 with weights that counted
+// the sweeps' operations as they were before and short curves at half their time.
 double pf_cost(const koo_berm_product& q, int last, int gen) {
   double u = 0.0;
   for (int s = 0; s <= last; ++s) u += q.rates - s;
   const double F = q.factors;
-  const double evolve = u * (13.0 * F + 20.0);
-  const double reverse = u * (34.0 * F + 60.0) + (q.checkpoint_every > 1 ? evolve : 0.0);
-  const double g = gen ? 60.0 * q.rates * F : 0.0;
-  return static_cast<double>(q.paths) * (2.0 * evolve + reverse + g + 400.0 * q.n_ex);
+  const double sweeps = u * (0.08 * F + 0.43);
+  const double g = gen ? 1.2 * q.rates * F : 0.0;
+  return static_cast<double>(q.paths) * (sweeps + g + 9.8 * q.n_ex);
 }
 
 }  // namespace
