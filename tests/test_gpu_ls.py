@@ -504,11 +504,13 @@ def test_frozen_bermudan_with_displaced_rates_vs_fp64_oracle(torch_cuda):
 
 @pytest.mark.parametrize("P,N,F,k", [(70, 2, 2, 1), (500, 3, 5, 2), (300, 4, 6, 1), (777, 5, 3, 2),
                                      (300, 9, 8, 4), (400, 45, 2, 8), (400, 46, 4, 8),
-                                     (130, 60, 7, 1)])
+                                     (130, 60, 7, 1), (32805, 4, 1, 2), (32769, 12, 8, 3),
+                                     (32999, 40, 5, 8), (32801, 41, 7, 4), (33000, 46, 8, 6)])
 def test_bermudan_windows_and_blocks_vs_fp64_oracle(torch_cuda, P, N, F, k):
     """Path quantities and the frozen-strategy adjoint on curves about and below
-    the step loops' window of rates, both block sizes, path counts that leave
-    lanes idle.  The strategy exercises on a constant continuation value, so
+    the step loops' window of rates, both block sizes (from 32768 paths four
+    wavefronts: the forward up to 80 rates, the backward up to 40), path counts
+    that leave lanes idle.  The strategy exercises on a constant continuation value, so
     that no regression is involved; tolerances as the tests above."""
     torch = torch_cuda
     rng = np.random.RandomState(100 * N + F)

@@ -209,7 +209,8 @@ def test_repeat_calls_are_deterministic(torch_cuda):
 
 @pytest.mark.parametrize("P,N,F,k", [
     (70, 1, 1, 1), (65, 2, 8, 1), (130, 3, 2, 2), (64, 4, 8, 2), (257, 5, 6, 3), (1000, 7, 7, 1),
-    (300, 8, 5, 8), (65600, 9, 2, 4), (66000, 13, 3, 1), (65537, 45, 1, 8), (300, 46, 5, 8),
+    (300, 8, 5, 8), (65600, 9, 2, 4), (66000, 13, 3, 1), (32771, 21, 7, 3), (65537, 45, 1, 8),
+    (300, 46, 5, 8),
     (200, 90, 3, 30), (100, 90, 8, 1)])
 def test_windows_blocks_and_intervals_vs_fp64_adjoint(torch_cuda, P, N, F, k):
     """Curves about and below the step loops' window of rates, every factor
