@@ -48,7 +48,8 @@ __global__ void __launch_bounds__(BD) __attribute__((amdgpu_waves_per_eu(W, W)))
 // The step table (lmm_step.h) behind the checkpoints, which the forward and
 // the backward read with scalar loads.  One lane per entry of the square.
 template <int F>
-__global__ void __launch_bounds__(256) k_berm_step_table(KOO_MODEL_PARAMS, float* __restrict__ tab) {
+__global__ void __launch_bounds__(256)
+    k_berm_step_table(KOO_MODEL_PARAMS, float* __restrict__ tab) {
   KOO_MODEL_LOCAL;
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q < m.N * m.N) put_step_entry<F>(m, q, tab);
@@ -192,7 +193,8 @@ extern "C" int bermudan_adjoint_workspace(int paths, int rates, int factors, int
   const int k = checkpoint_every;
   // the checkpoints, then the step table
   if (checkpoint_bytes)
-    *checkpoint_bytes = sizeof(float) * (ckpt_rows(rates, factors, k) * P + step_table_floats(rates));
+    *checkpoint_bytes =
+        sizeof(float) * (ckpt_rows(rates, factors, k) * P + step_table_floats(rates));
   if (scratch_bytes)
     *scratch_bytes = sizeof(float) * (k == 1 ? 1 : scratch_rows(rates, factors, k) * P);
   // payoff adjoints (rates x P floats), exercise step (P ints), value (P floats)

@@ -19,16 +19,14 @@ namespace {
 
 constexpr int kAcrossLanes = 256;
 
-// Paths of a wavefront and of a block.
-template <int W>
-constexpr int kAcrossPaths = 64 / W;
+// Paths of a block.
 template <int W>
 constexpr int kAcrossBlock = kAcrossLanes / W;
 
-template <int Ctrl, int Rows, bool Zero>
+template <int Ctrl, int Rows>
 __device__ __forceinline__ float lane_shift(float old, float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), Ctrl,
-                                                    Rows, 0xf, Zero));
+                                                    Rows, 0xf, false));
 }
 // Sums over this lane and those below it in the path's W lanes, of the F values
 // v[0..F): shifts by 1, 2, 4, 8 inside rows of 16, then the row below's last
@@ -85,12 +83,12 @@ __device__ __forceinline__ float scan_add(float x) {
 #undef KOO_DPP
 template <int W>
 __device__ __forceinline__ float scan_mul(float v) {
-  v *= lane_shift<0x111, 0xf, false>(1.0f, v);
-  v *= lane_shift<0x112, 0xf, false>(1.0f, v);
-  v *= lane_shift<0x114, 0xf, false>(1.0f, v);
-  v *= lane_shift<0x118, 0xf, false>(1.0f, v);
-  if constexpr (W >= 32) v *= lane_shift<0x142, 0xa, false>(1.0f, v);
-  if constexpr (W == 64) v *= lane_shift<0x143, 0xc, false>(1.0f, v);
+  v *= lane_shift<0x111, 0xf>(1.0f, v);
+  v *= lane_shift<0x112, 0xf>(1.0f, v);
+  v *= lane_shift<0x114, 0xf>(1.0f, v);
+  v *= lane_shift<0x118, 0xf>(1.0f, v);
+  if constexpr (W >= 32) v *= lane_shift<0x142, 0xa>(1.0f, v);
+  if constexpr (W == 64) v *= lane_shift<0x143, 0xc>(1.0f, v);
   return v;
 }
 
@@ -117,7 +115,8 @@ __device__ __forceinline__ void load_roots(const Model& m, int s, int r, bool ra
   const int at = rate && r >= s ? 4 * F * r : 0x40000000;
 #pragma unroll
   for (int f = 0; f < F; ++f)
-    a[f] = __int_as_float(static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rs, at + 4 * f, 0, 0)));
+    a[f] = __int_as_float(
+        static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rs, at + 4 * f, 0, 0)));
 }
 
 template <int F>
@@ -184,8 +183,8 @@ __device__ __forceinline__ float across_steps(const Model& m, const AcrossLane<W
 
 // What across_steps keeps for the reverse: per path three triangular arrays in
 // LDS (state, sum a y, sum a d), the N - s alive rates of step s from the top
-// rate down.  A rate dead at the step reads the last entry, which its zero
-// pseudo-roots cancel.
+// rate down.  A rate dead at the step reads entries of later steps (at the
+// array's end the last one): finite ones, which its zero pseudo-roots cancel.
 __host__ __device__ constexpr int across_tri(int N) { return N * (N + 1) / 2; }
 __host__ __device__ constexpr int across_tri_row(int N, int s) { return s * N - s * (s - 1) / 2; }
 

@@ -31,10 +31,14 @@
 // sums on the matrix cores, and fewer steps run again (at 40 rates, 5 factors
 // and k = 8 those of 300 of the 820 rate updates; all of them while each step's
 // states were kept in scratch, 14.8 GB of traffic).  At 2^20 paths, 40 rates, 5
-// factors and k = 8: forward with checkpoints 1250 -> 845 us, backward 3655 ->
-// 2440 us; at k = 8 and 4096 paths 188 -> 107 and 535 -> 230 us, 51 and 107 with
-// the rates across the lanes; price of 2^17 paths, 80 rates, 2 factors 1525 -> 365 us (its step table was in LDS and left
-// room for three wavefronts per CU).
+// factors and k = 8: forward with checkpoints 1250 -> 850 us, backward 3655 ->
+// 2500 us (up to 2700 where the card has clocked down); at k = 8 and 4096 paths
+// 188 -> 107 and 535 -> 230 us, 51 and 107 with the rates across the lanes; price
+// of 2^17 paths, 80 rates, 2 factors 1525 -> 365 us (its step table was in LDS
+// and left room for three wavefronts per CU).  Greeks beyond 40 rates run
+// single-wavefront blocks in the backward, three to seven to a CU: 2^17 paths x 5
+// factors, k = 8, forward and backward 46 rates 1117 -> 868 us, 60 rates 2223 ->
+// 1313, 90 rates 9300 -> 3529.
 #include <algorithm>
 
 #include "lmm_across.h"
@@ -127,7 +131,8 @@ __global__ void __launch_bounds__(BD)
     B.scale(inv);
   }
   if (ckpt && seg == 0) keep_states(N);  // S1 == N
-  const double sum = wave_sum_f64(static_cast<int>(threadIdx.x) < b.n ? static_cast<double>(v) : 0.0);
+  const double sum =
+      wave_sum_f64(static_cast<int>(threadIdx.x) < b.n ? static_cast<double>(v) : 0.0);
   if ((threadIdx.x & 63) == 0)
     put_partial<false>(part, wave_count(m.P), wave_index<BD>(blockIdx.x), 0, sum);
 }
@@ -278,7 +283,8 @@ __global__ void __launch_bounds__(kAcrossLanes)
   if (at.live) {
     const float tau = m.taus[r], xs = start_level(m, r) * fast_exp2(x);
     const float tail = l ? above : 0.0f;
-    lam = (caplet_deriv(xs - m.disp[r], tau, m.strike, inv) * before - tau * inv * tail) * (kLn2 * xs);
+    lam = (caplet_deriv(xs - m.disp[r], tau, m.strike, inv) * before - tau * inv * tail) *
+          (kLn2 * xs);
   }
   __syncthreads();
   const float w = across_reverse<F, W>(m, rate ? r : -1, rate, krr, lam,
@@ -311,7 +317,12 @@ __global__ void __launch_bounds__(kAcrossLanes)
 // wavefronts of 64-lane paths (40 rates, 5 factors: 158 us for 336 at 4096
 // paths, 273 at 8192, 479 at 16384), 7500 of 32-lane ones (20 rates, 3 factors:
 // 71 us for 100 at 8192 paths, 107 at 16384) and 5500 of 16-lane ones (16
-// rates, 5 factors: 76 us for 93 at 16384 paths, 116 at 32768).
+// rates, 5 factors: 76 us for 93 at 16384 paths, 116 at 32768).  With more dead
+// lanes the limits still hold: 33 rates, 5 factors 197 for 235 us, 17 rates 81 for
+// 96, 6 rates 29 for 32, 8 rates and 8 factors 44 each.  The price alone crosses
+// near them too (40 rates 75 for 92 us, 17 rates 26 for 28), but for curves of up
+// to 8 rates and 8 factors, where a path per lane takes 12.7 for 15.8 us at the
+// limit: not worth a limit of its own.
 int across_lanes(int paths, int N) {
   if (N < kShortCurve || N > 64) return 0;
   const int W = N <= 16 ? 16 : (N <= 32 ? 32 : 64);
@@ -412,10 +423,9 @@ extern "C" int lmm_price_fwd(int paths, int rates, int factors, int checkpoint_e
   const bool own = own_table(rates, threads);
   const size_t lds =
       rows_lds(rates, threads) + (own ? sizeof(float) * step_table_floats(rates) : 0);
-  float* tab = checkpoints
-                   ? checkpoints + static_cast<size_t>(ckpt_rows(rates, factors, checkpoint_every)) *
-                                       paths
-                   : reinterpret_cast<float*>(partials + partial_doubles(paths, rates));
+  const size_t kept = static_cast<size_t>(ckpt_rows(rates, factors, checkpoint_every)) * paths;
+  float* tab = checkpoints ? checkpoints + kept
+                           : reinterpret_cast<float*>(partials + partial_doubles(paths, rates));
   hipStream_t st = as_stream(stream);
   if (const int W = across_lanes(paths, rates)) {
     const int nb = across_blocks(paths, W);
@@ -493,7 +503,7 @@ extern "C" int lmm_price_bwd(int paths, int rates, int factors, int checkpoint_e
   switch (factors) {
 #define KOO_BWD(F, BD, U, W)                                                                     \
   hipLaunchKernelGGL((k_price_bwd<F, BD, U, W>), dim3(blocks), dim3(BD), lds, st, m.z, m.f0,     \
-                     m.taus, m.disp, m.A, m.strike, m.P, m.N, m.S1, m.L, vols, checkpoints, tab,       \
+                     m.taus, m.disp, m.A, m.strike, m.P, m.N, m.S1, m.L, vols, checkpoints, tab, \
                      segment_scratch, partials)
 #define KOO_CASE(F)                                                                              \
   case F:                                                                                        \

@@ -127,7 +127,9 @@ __host__ __device__ constexpr int sweep_segment_row(int N, int F, int S1, int L,
 inline int ckpt_rows(int N, int F, int k) {
   return k == 1 ? N * (N + 1 + 2 * F) : (N + k - 1) / k * (N + 1);
 }
-inline int scratch_rows(int N, int F, int k) { return k == 1 ? 0 : (k < N ? k : N) * (N + 1 + 2 * F); }
+inline int scratch_rows(int N, int F, int k) {
+  return k == 1 ? 0 : (k < N ? k : N) * (N + 1 + 2 * F);
+}
 // (With S1 = 0 the segments are at least k long, and each takes at most N + 1
 // rows: a plan always exists.)
 inline SweepPlan sweep_plan(int N, int F, int k) {
@@ -233,11 +235,11 @@ struct BlockPaths {
   int n;
   __device__ __forceinline__ BlockPaths(int paths, int block, int lanes)
       : p0(static_cast<size_t>(block) * lanes), P(paths), n(min(lanes, static_cast<int>(P - p0))) {}
-  // `base`: element 0 of the row; on: no lane reads or stores anything if false
-  __device__ __forceinline__ PathRow row(const float* base, bool on = true) const {
-    return PathRow{__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base) + p0, 0,
-                                                     on ? 4 * n : 0, 0x00027000),
-                   static_cast<int>(4 * threadIdx.x)};
+  // `base`: element 0 of the row
+  __device__ __forceinline__ PathRow row(const float* base) const {
+    return PathRow{
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base) + p0, 0, 4 * n, 0x00027000),
+        static_cast<int>(4 * threadIdx.x)};
   }
   // P, out of the compiler's sight: rows addressed with it inside a loop are
   // formed there, where many of them would be hoisted out of it into more
@@ -248,8 +250,8 @@ struct BlockPaths {
     return q;
   }
   // row `r` of an array of rows of P
-  __device__ __forceinline__ PathRow row(const float* base, int r, bool on = true) const {
-    return row(base + static_cast<size_t>(r) * P, on);
+  __device__ __forceinline__ PathRow row(const float* base, int r) const {
+    return row(base + static_cast<size_t>(r) * P);
   }
 };
 
@@ -400,7 +402,11 @@ __device__ __forceinline__ void window_ready() {
 }
 
 // Uniform values carried round a loop, held in scalar registers (the compiler
-// would carry what only vector instructions use in vector registers).
+// would carry what only vector instructions use in vector registers).  `x` has
+// to be what the compiler itself takes for uniform (read with uniform addresses
+// and not spilled to a lane's register on the way): "+s" makes it an error where
+// it is not, "illegal VGPR to SGPR copy", as when the library is compiled with
+// packed FP32.  The remedy is a __builtin_amdgcn_readfirstlane on x.
 __device__ __forceinline__ float keep_scalar(float x) {
   int i = __float_as_int(x);
   asm volatile("" : "+s"(i));
@@ -873,7 +879,9 @@ __device__ __forceinline__ int find_block_owner(const Item* items, int n, int bl
 
 // Rate-count class of a product in the batched LS launches (a launch per class,
 // so LDS is reserved for the class's largest curve).
-inline int rate_class(int rates) { return rates <= 16 ? 0 : (rates <= 24 ? 1 : (rates <= 32 ? 2 : 3)); }
+inline int rate_class(int rates) {
+  return rates <= 16 ? 0 : (rates <= 24 ? 1 : (rates <= 32 ? 2 : 3));
+}
 
 // out[col] = (sum_b part[b*ncols + col]) * scale, compensated; called by a
 // whole block (k_finalize_cols runs one block per column).  Agent: the
