@@ -384,6 +384,7 @@ def test_discounting_matches_reference_gold():
     assert np.allclose(summed, c["summed"], rtol=1e-14)
 
 
+@pytest.mark.skipif(not O.ref_available(), reason="reference gold library not built")
 def test_partial_discounting_matches_reference_gold():
     """Partial discounting (flows generated at a step, discounted log-linearly
     to their payment time and by the numeraire ratio to an earlier target
@@ -488,6 +489,7 @@ def test_caplet_adjoint_matches_central_fd():
         assert abs(fv - v[i]) <= 1e-7 * abs(v[i]) + 1e-10
 
 
+@pytest.mark.skipif(not O.ref_available(), reason="reference gold library not built")
 def test_caplet_adjoint_matches_reference_gold_bumped_prices():
     """The oracle's pathwise adjoint against central differences of the
     caplet price the reference's own gold pipeline computes on the same
