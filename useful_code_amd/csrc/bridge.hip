@@ -1,6 +1,6 @@
 // bridge.hip -- stage (a)+(b): Brownian bridge (Jaeckel construction on the
-// unit grid) with successive differencing, and the fused
-// Sobol -> scramble -> normal -> bridge generator, for gfx950.
+// unit grid) with successive differencing, and the launch of the fused
+// Sobol -> scramble -> normal -> bridge generator (bridge_gen.h), for gfx950.
 //
 // One lane owns one (path, factor) pair and every global load/store is a
 // contiguous 256-byte row of the path-minor layouts ([D][P] in, (S,F,P)
@@ -12,12 +12,11 @@
 #include <array>
 #include <cmath>
 #include <mutex>
-#include <type_traits>
 #include <utility>
 #include <unordered_map>
 #include <vector>
 
-#include "bridge_device.h"
+#include "bridge_gen.h"
 
 namespace koo {
 
@@ -33,107 +32,6 @@ __global__ void __launch_bounds__(kBridgeThreads)
   const int* idx = alloc + blockIdx.y * steps;
   bridge_lane(T, steps, factors, paths, p, blockIdx.y, lds,
               [&](int i) { return in[static_cast<size_t>(idx[i]) * paths + p]; }, out);
-}
-
-// ---------------------------------------------------------------------------
-// Register-resident bridge (stand-alone for S <= kRegSteps, the generator for
-// every S).  The construction order depends on S only, so for a compile-time S
-// every index is a constant and the S bridge points of a lane stay in VGPRs (no
-// LDS path storage, which held occupancy to one or two waves per SIMD).  The
-// stand-alone bridge reads its weights from the kernel arguments (uniform,
-// scalar loads); the fused generator, which loops over chunks, from an LDS copy
-// (LdsWeights).
-// ---------------------------------------------------------------------------
-constexpr int kRegSteps = 64;
-
-// The index walk of make_tables (brownian_bridge.cu:639-700) as a constant
-// expression.
-template <int S>
-struct BridgeOrder {
-  int16_t bridge[S] = {}, left[S] = {}, right[S] = {};
-  constexpr BridgeOrder() {
-    int map[S] = {};
-    map[S - 1] = 1;
-    bridge[0] = S - 1;
-    for (int j = 0, i = 1; i < S; ++i) {
-      while (map[j]) ++j;
-      int k = j;
-      while (!map[k]) ++k;
-      const int l = j + ((k - 1 - j) >> 1);
-      map[l] = i;
-      bridge[i] = static_cast<int16_t>(l);
-      left[i] = static_cast<int16_t>(j);
-      right[i] = static_cast<int16_t>(k);
-      j = k + 1;
-      if (j >= S) j = 0;
-    }
-  }
-};
-
-// The construction weights of step i, {rw, lw, sd}, from a copy of the
-// tables in LDS ({rw, lw, sd, 0} per step) read at an index offset the
-// compiler cannot see through.  A loop over chunks that reads the
-// kernel-argument tables gets all 3 S weights hoisted into scalar registers,
-// more than there are (spilled through vector lanes); the LDS copy is read
-// where each weight is used.
-struct LdsWeights {
-  const f32x4* w;  // LDS
-  int z;           // zero, opaque to the compiler
-  __device__ __forceinline__ void get(int i, float& rw, float& lw, float& sd) const {
-    const f32x4 q = w[i + z];
-    rw = q.x;
-    lw = q.y;
-    sd = q.z;
-  }
-};
-
-// V is float (one path), f32x2 or f32x4 (two, four paths; the scalar weights
-// broadcast).
-template <int S, int I, class V, class Z, class W>
-__device__ __forceinline__ void bridge_point(V (&w)[S], const W& wt, Z& z) {
-  constexpr BridgeOrder<S> M{};
-  float rw, lw, sd;
-  wt.get(I, rw, lw, sd);
-  if constexpr (I == 0) {
-    w[S - 1] = sd * z(0);
-  } else {
-    constexpr int j = M.left[I], k = M.right[I], l = M.bridge[I];
-    V v = rw * w[k];
-    if constexpr (j != 0) v = bridge_fma(lw, w[j - 1], v);
-    w[l] = bridge_fma(sd, z(I), v);
-  }
-}
-
-template <int S, class V, class Z, class W, int... I>
-__device__ __forceinline__ void bridge_points(V (&w)[S], const W& wt, Z& z,
-                                              std::integer_sequence<int, I...>) {
-  (bridge_point<S, I>(w, wt, z), ...);
-}
-
-// In-place form for variates that come from memory: w[bridge(i)] holds
-// variate i on entry (so all S loads can be in flight at once, into the
-// registers the points end in), and point bridge(i) replaces it; the same
-// operations in the same order as bridge_point.
-template <int S, int I, class V>
-__device__ __forceinline__ void bridge_point_inplace(V (&w)[S], const BridgeTables& T) {
-  constexpr BridgeOrder<S> M{};
-  if constexpr (I == 0) {
-    w[S - 1] = T.sd[0] * w[S - 1];
-  } else {
-    constexpr int j = M.left[I], k = M.right[I], l = M.bridge[I];
-    V v = T.rw[I] * w[k];
-    if constexpr (j != 0) v = bridge_fma(T.lw[I], w[j - 1], v);
-    w[l] = bridge_fma(T.sd[I], w[l], v);
-  }
-}
-
-template <int S, class V, class Load, int... I>
-__device__ __forceinline__ void bridge_points_loaded(V (&w)[S], const BridgeTables& T,
-                                                     Load load,
-                                                     std::integer_sequence<int, I...>) {
-  constexpr BridgeOrder<S> M{};
-  ((w[M.bridge[I]] = load(I)), ...);
-  (bridge_point_inplace<S, I>(w, T), ...);
 }
 
 template <int S>
@@ -180,171 +78,12 @@ __global__ void __launch_bounds__(kBridgeThreads)
   }
 }
 
-// Fused generator on the register bridge, every step count.  Each wavefront
-// walks a contiguous run of 64-path chunks of one factor, two at a time and an
-// odd last one alone.  With n = G + l (G a multiple of 64, l < 64) the Gray code
-// splits, gray(n) = gray(G) ^ gray(l), so the scrambled Sobol integer is
-// X(G) ^ T(l) with X(G) = scrambler ^ XOR of the direction numbers over the set
-// bits of gray(G).  A lane's l is the same in every chunk; T(l) sits in LDS.
-// X(G) is kept one dimension per lane (two registers beyond 64 steps): from
-// G = 64m to 64(m+1) gray flips bits 5 and 6 + ctz(m+1), so advancing costs two
-// XORs.  A chunk (lanes at n = 64c + off1 + lane) spans G and G + 64, two chunks
-// three values: the wavefront writes them to rows of its own in LDS, from which
-// each lane reads those of its group, four dimensions to a read.
-// Bound by the vector instructions, 26 a point, most of them the quantile; 43
-// with one chunk at a time, X(G) read out by readlane and 64-bit store
-// addresses.  2^20 paths: 40 steps x 5 factors 232 -> 175 us, 64 x 32 2.59 ->
-// 1.93 ms (4.4 TB/s of stores).  Step counts above 64 kept the points in LDS
-// and walked the bits of the Gray code for each: 2^17 x 80 x 2 238 -> 43 us.
-// Few paths leave a wavefront one chunk: in a pair half of that is for nothing
-// (65536 paths x 32 x 5 24.6 us, 18.4 alone; 4096 x 40 x 8 12.2, 10.4).  Beyond
-// kRegSteps the body for one chunk is left out: those kernels take most of this
-// file's compile time.
-template <int S>
-__global__ void __launch_bounds__(kBridgeThreads)
-    k_sobol_bridge_reg(const BridgeTables T, int factors, int paths, uint32_t off1,
-                       const uint32_t* __restrict__ dirs, const uint32_t* __restrict__ scr,
-                       int number_scrambled, const int* __restrict__ alloc,
-                       float* __restrict__ out) {
-  constexpr int R = (S + 63) / 64;  // dimensions per lane in the X(G) bookkeeping
-  constexpr int Q = (S + 3) / 4;    // groups of four dimensions
-  __shared__ uint32_t vall[S * 32];                      // direction numbers [bridge variate][bit]
-  __shared__ u32x4 tlo[Q * 64];                          // T(l) [group][l]
-  __shared__ u32x4 xrows[(kBridgeThreads / 64) * 3 * Q]; // X(G), X(G+64), X(G+128) per wavefront
-  __shared__ f32x4 wts[S];                               // construction weights {rw, lw, sd, 0}
-  const int f = blockIdx.y;
-  const int* idx = alloc + f * S;
-  for (int q = threadIdx.x; q < S * 32; q += blockDim.x)
-    vall[q] = dirs[static_cast<size_t>(idx[q >> 5]) * 32 + (q & 31)];
-  for (int q = threadIdx.x; q < S; q += blockDim.x) wts[q] = f32x4{T.rw[q], T.lw[q], T.sd[q], 0.0f};
-  __syncthreads();
-  for (int q = threadIdx.x; q < S * 64; q += blockDim.x) {
-    const uint32_t l = static_cast<uint32_t>(q & 63), g = l ^ (l >> 1);
-    const uint32_t* vv = vall + (q >> 6) * 32;
-    uint32_t x = 0;
-#pragma unroll
-    for (int bit = 0; bit < 6; ++bit)
-      if ((g >> bit) & 1u) x ^= vv[bit];
-    reinterpret_cast<uint32_t*>(tlo)[(q >> 8) * 256 + l * 4 + ((q >> 6) & 3)] = x;
-  }
-  __syncthreads();
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t waves = static_cast<int64_t>(gridDim.x) * (blockDim.x >> 6);
-  const int64_t wv = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave;
-  const int64_t chunks = (static_cast<int64_t>(paths) + 63) >> 6;
-  // scalars: the loop below and its addresses are uniform
-  const int c0 = __builtin_amdgcn_readfirstlane(static_cast<int>(wv * chunks / waves));
-  const int c1 = __builtin_amdgcn_readfirstlane(static_cast<int>((wv + 1) * chunks / waves));
-  if (c0 >= c1) return;
-
-  const uint32_t r = off1 & 63u;
-  const uint32_t l = (r + static_cast<uint32_t>(lane)) & 63u;
-  uint32_t m = static_cast<uint32_t>(c0) + (off1 >> 6);  // G = 64 m for chunk c0
-  // this lane's dimensions for the X(G) bookkeeping
-  const uint32_t* vd[R];
-  uint32_t x[R], v5[R];
-  uint32_t* xw = reinterpret_cast<uint32_t*>(xrows + wave * 3 * Q) + lane;
-#pragma unroll
-  for (int k = 0; k < R; ++k) {
-    const int dl = 64 * k + lane < S ? 64 * k + lane : S - 1;
-    vd[k] = vall + dl * 32;
-    const int d = idx[dl];
-    x[k] = d < number_scrambled ? scr[d] : 0u;
-    const uint32_t G = m << 6, g = G ^ (G >> 1);
-    for (int b = 5; b < 32; ++b)
-      if ((g >> b) & 1u) x[k] ^= vd[k][b];
-    v5[k] = vd[k][5];
-  }
-  auto put = [&](int row) {
-#pragma unroll
-    for (int k = 0; k < R; ++k)
-      if (64 * k + lane < S) xw[row * 4 * Q + 64 * k] = x[k];
-  };
-  // bits 5 and t of gray, t = 6 + ctz of the next m
-  auto advance = [&] {
-    const int t = 6 + __builtin_ctz(++m);
-#pragma unroll
-    for (int k = 0; k < R; ++k) x[k] ^= v5[k] ^ (t < 32 ? vd[k][t] : 0u);
-  };
-  const u32x4* tl = tlo + l;
-  // the lane's own group of the first chunk; of the second, a row further
-  const u32x4* xl = xrows + wave * 3 * Q + (r + static_cast<uint32_t>(lane) >= 64u ? Q : 0);
-  // the wavefront's paths as a buffer per step: stores past its last path are
-  // dropped (lanes past the last path; the second chunk of a last pair)
-  const int bytes = 4 * min(paths - c0 * 64, (c1 - c0) * 64);
-  float* first = out + static_cast<size_t>(f) * paths + static_cast<size_t>(c0) * 64;
-  // `chunks`: two at a time, or one
-  auto walk = [&](int c, auto chunks) {
-    constexpr bool two = decltype(chunks)::value == 2;
-    using V = typename std::conditional<two, f32x2, float>::type;
-    // a wavefront's LDS operations keep their order, and the rows are its own
-    put(0);
-    advance();
-    put(1);
-    if constexpr (two) {
-      advance();
-      put(2);
-    }
-    __builtin_amdgcn_wave_barrier();
-    u32x4 t, a, b;
-    auto z = [&](int i) {
-      if (i % 4 == 0) {
-        t = tl[(i >> 2) * 64];
-        a = xl[i >> 2];
-        if constexpr (two) b = xl[Q + (i >> 2)];
-      }
-      const float first = invnorm_u32(t[i & 3] ^ a[i & 3]);
-      if constexpr (two) return f32x2{first, invnorm_u32(t[i & 3] ^ b[i & 3])};
-      else return first;
-    };
-    // The weights come from LDS at an offset, and the rows of the steps from a
-    // stride, made opaque each time (a zero from s_mov), so that their reads
-    // and sums stay in the loop.
-    int zero;
-    asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
-    V w[S];
-    const LdsWeights wt{wts, zero};
-    bridge_points<S>(w, wt, z, std::make_integer_sequence<int, S>{});
-    const size_t stride = (static_cast<size_t>(factors) + zero) * paths;
-    float* row = first;
-    const int byte = (c - c0) * 256 + lane * 4;
-    V prev{};
-#pragma unroll
-    for (int i = 0; i < S; ++i, row += stride) {
-      const auto rs = __builtin_amdgcn_make_buffer_rsrc(row, 0, bytes, 0x00027000);
-      const V dz = w[i] - prev;
-      if constexpr (two) {
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz.x), rs, byte, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz.y), rs, byte + 256, 0, 0);
-      } else {
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dz), rs, byte, 0, 0);
-      }
-      prev = w[i];
-    }
-    __builtin_amdgcn_wave_barrier();
-  };
-  int c = c0;
-  if constexpr (S <= kRegSteps) {
-    for (; c + 1 < c1; c += 2) walk(c, std::integral_constant<int, 2>{});
-    if (c < c1) walk(c, std::integral_constant<int, 1>{});
-  } else {
-    for (; c < c1; c += 2) walk(c, std::integral_constant<int, 2>{});
-  }
-}
-
 // Launch tables for every S in [1, kRegSteps].
 using RegBridgeFn = void (*)(const BridgeTables, int, int, const int*, const float*, float*);
-using RegGenFn = void (*)(const BridgeTables, int, int, uint32_t, const uint32_t*,
-                          const uint32_t*, int, const int*, float*);
 
 template <int... I>
 constexpr auto reg_bridge_table(std::integer_sequence<int, I...>) {
   return std::array<RegBridgeFn, sizeof...(I)>{&k_bridge_reg<I + 1>...};
-}
-template <int... I>
-constexpr auto reg_gen_table(std::integer_sequence<int, I...>) {
-  return std::array<RegGenFn, sizeof...(I)>{&k_sobol_bridge_reg<I + 1>...};
 }
 using RegBridge4Fn = void (*)(const BridgeTables, int, int, const int*, const f32x4*, f32x4*);
 template <int... I>
@@ -353,7 +92,13 @@ constexpr auto reg_bridge4_table(std::integer_sequence<int, I...>) {
 }
 const auto kRegBridge = reg_bridge_table(std::make_integer_sequence<int, kRegSteps>{});
 const auto kRegBridge4 = reg_bridge4_table(std::make_integer_sequence<int, kRegSteps4>{});
-const auto kRegGen = reg_gen_table(std::make_integer_sequence<int, kBridgeMaxSteps>{});
+
+const void* gen_kernel_for(int steps) {
+  if (steps < kBridgeGenFirst[1]) return bridge_gen_kernel_0(steps);
+  if (steps < kBridgeGenFirst[2]) return bridge_gen_kernel_1(steps);
+  if (steps < kBridgeGenFirst[3]) return bridge_gen_kernel_2(steps);
+  return bridge_gen_kernel_3(steps);
+}
 
 // ---------------------------------------------------------------------------
 // Power-of-two bridge (the reference's legacy BrownianBridge<D>,
@@ -604,13 +349,13 @@ extern "C" int sobol_bridge_gpu(int paths, unsigned path_offset, int steps, int 
   // then walks its own run of chunks, so there is no tail of late blocks.
   static std::array<int, kBridgeMaxSteps> resident{};
   static std::mutex mu;
+  const void* kernel = gen_kernel_for(steps);
   int per_cu;
   {
     std::lock_guard<std::mutex> lock(mu);
     if (!resident[steps - 1]) {
       int nb = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-              &nb, reinterpret_cast<const void*>(kRegGen[steps - 1]), kBridgeThreads, 0) !=
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, kBridgeThreads, 0) !=
               hipSuccess ||
           nb < 1)
         nb = 1;
@@ -623,10 +368,12 @@ extern "C" int sobol_bridge_gpu(int paths, unsigned path_offset, int steps, int 
   const int64_t most = (chunks + kBridgeThreads / 64 - 1) / (kBridgeThreads / 64);
   if (per_factor > most) per_factor = most;
   if (per_factor < 1) per_factor = 1;
-  hipLaunchKernelGGL(kRegGen[steps - 1], dim3(static_cast<unsigned>(per_factor), factors),
-                     dim3(kBridgeThreads), 0, as_stream(stream), tables_for(steps), factors, paths,
-                     path_offset + 1u, d_directions, scramblers, number_scrambled,
-                     allocation_indices, out);
+  BridgeTables tables = tables_for(steps);
+  uint32_t off1 = path_offset + 1u;
+  void* args[] = {&tables,     &factors,          &paths,              &off1, &d_directions,
+                  &scramblers, &number_scrambled, &allocation_indices, &out};
+  (void)hipLaunchKernel(kernel, dim3(static_cast<unsigned>(per_factor), factors),
+                        dim3(kBridgeThreads), args, 0, as_stream(stream));
   return check_launch("sobol_bridge_gpu");
 }
 
